@@ -1288,14 +1288,32 @@ struct tfg_faces {
   int device = 0;            // of h, kept so that destroying needs no h
   int n_faces = 0;
   int n_ambient = 0;         // boundary faces of ambient regions
-  int *cf_off = nullptr, *cf_face = nullptr, *ent_face = nullptr, *c1 = nullptr, *c2 = nullptr;
+  // each cell's faces (tfg::CellFaces)
+  int *cf_off = nullptr, *cf_face = nullptr, *cf_nbr = nullptr;
+  void* cf_slot = nullptr;
+  uint8_t* late = nullptr;
+  bool wide = false;         // some row is longer than 256 entries
+  bool unset = false;        // some off-diagonal entry is set by no face
   uint8_t* flags = nullptr;
-  int* c2b = nullptr;        // c2 as given (1-based, boundary cells < 0)
   int max_bnd = 0;           // largest boundary cell number
   bool shared_entry = false; // some matrix entry set by two faces
   bool shared_bnd = false;   // some boundary cell on two faces
-  double *pmin = nullptr, *pmax = nullptr;  // momentum scratch (nt each), on first use
+  tfg::dbl2* mm = nullptr;   // momentum scratch (nt pairs), on first use
 };
+
+static tfg::CellFaces cell_faces(const tfg_faces* f) {
+  tfg::CellFaces t{};
+  t.n = f->h->nt;
+  t.row = f->h->row;
+  t.off = f->cf_off;
+  t.face = f->cf_face;
+  t.nbr = f->cf_nbr;
+  t.slot = f->cf_slot;
+  t.late = f->late;
+  t.wide = f->wide ? 1 : 0;
+  t.unset = f->unset ? 1 : 0;
+  return t;
+}
 
 // hipFree waits for the device, so no stream of the matrix handle (which
 // may be gone already) is needed; errors of the release are dropped here
@@ -1303,8 +1321,7 @@ struct tfg_faces {
 static void faces_free(tfg_faces* f) {
   if (!f) return;
   (void)hipSetDevice(f->device);
-  void* dev[] = {f->cf_off, f->cf_face, f->ent_face, f->c1, f->c2, f->flags, f->c2b, f->pmin,
-                 f->pmax};
+  void* dev[] = {f->cf_off, f->cf_face, f->cf_nbr, f->cf_slot, f->late, f->flags, f->mm};
   for (void* d : dev)
     if (d) (void)hipFree(d);
   (void)hipGetLastError();
@@ -1322,7 +1339,8 @@ int tfg_faces_create(tfg_matrix* h, int n_faces, const int* c1, const int* c2, c
   HIP_TRY(hipSetDevice(h->device));
   HIP_TRY(hipMemcpy(row.data(), h->row, sizeof(int) * (n + 1), hipMemcpyDeviceToHost));
   HIP_TRY(hipMemcpy(col.data(), h->col, sizeof(int) * (size_t)h->nnz, hipMemcpyDeviceToHost));
-  std::vector<int> cnt(n + 1, 0), ent(h->nnz, -1), a(n_faces), b(n_faces);
+  std::vector<int> cnt(n + 1, 0);
+  std::vector<char> set(h->nnz, 0);   // entries some face sets
   std::vector<uint8_t> fl(n_faces);
   bool shared_entry = false;
   int max_bnd = 0;
@@ -1336,8 +1354,6 @@ int tfg_faces_create(tfg_matrix* h, int n_faces, const int* c1, const int* c2, c
     if (p < 0 || p >= n || q >= n) return fail(TFG_EINVAL, "face %d: cells out of range", s + 1);
     if (b_region[s] < TFG_REGION_NONE || b_region[s] > TFG_REGION_AMBIENT)
       return fail(TFG_EINVAL, "face %d: region code %d", s + 1, b_region[s]);
-    a[s] = p;
-    b[s] = q;
     uint8_t code = 0;
     if (q < 0 && c2[s] < 0) {   // a boundary cell: its region's assignment of b(c1)
       code = b_region[s] == TFG_REGION_PRESSURE ? 2 : (b_region[s] == TFG_REGION_AMBIENT ? 4 : 0);
@@ -1351,19 +1367,38 @@ int tfg_faces_create(tfg_matrix* h, int n_faces, const int* c1, const int* c2, c
       if (j1 <= row[p] || j1 >= row[p + 1] || col[j1] != q || j2 <= row[q] || j2 >= row[q + 1] ||
           col[j2] != p)
         return fail(TFG_EINVAL, "face %d: pos does not point at (c1,c2) / (c2,c1)", s + 1);
-      if (ent[j1] >= 0 || ent[j2] >= 0) shared_entry = true;
-      ent[j1] = s;   // the last face that sets the entry wins, as in the loop
-      ent[j2] = s;
+      if (set[j1] || set[j2]) shared_entry = true;
+      set[j1] = 1;
+      set[j2] = 1;
     } else if (c2[s] < 0) {
       if (bnd_seen[-c2[s]]) shared_bnd = true;
       bnd_seen[-c2[s]] = 1;
     }
   }
-  for (int c = 0; c < n; ++c) cnt[c + 1] += cnt[c];
-  std::vector<int> cf(cnt[n]), fill(cnt.begin(), cnt.end() - 1);
-  for (int s = 0; s < n_faces; ++s) {   // increasing face order within each cell
-    cf[fill[a[s]]++] = s << 1;
-    if (b[s] >= 0) cf[fill[b[s]]++] = (s << 1) | 1;
+  bool wide = false, unset = false;
+  for (int c = 0; c < n; ++c) {
+    wide = wide || row[c + 1] - row[c] > 256;
+    cnt[c + 1] += cnt[c];
+    for (int j = row[c] + 1; j < row[c + 1]; ++j) unset = unset || !set[j];
+  }
+  // increasing face order within each cell; a face that shares an entry with
+  // an earlier one overwrites it, as in the loop
+  std::vector<int> cf(cnt[n]), nbr(cnt[n]), fill(cnt.begin(), cnt.end() - 1);
+  std::vector<int> slot32(wide ? cnt[n] : 0);
+  std::vector<uint8_t> slot8(wide ? 0 : cnt[n]), late(n, 0);
+  auto list = [&](int c, int face, int other, int place) {
+    const int t = fill[c]++;
+    cf[t] = face;
+    nbr[t] = other;
+    if (wide) slot32[t] = place;
+    else slot8[t] = (uint8_t)place;
+    if (other < 0 && t > cnt[c] && nbr[t - 1] >= 0) late[c] = 1;
+  };
+  for (int s = 0; s < n_faces; ++s) {
+    const int p = c1[s] - 1, q = c2[s] - 1;
+    const bool inner = c2[s] > 0;
+    list(p, s << 1, c2[s], inner ? pos[2 * s] - 1 - row[p] : 0);
+    if (inner) list(q, (s << 1) | 1, c1[s], pos[2 * s + 1] - 1 - row[q]);
   }
   tfg_faces* f = new tfg_faces();
   f->h = h;
@@ -1376,11 +1411,13 @@ int tfg_faces_create(tfg_matrix* h, int n_faces, const int* c1, const int* c2, c
   };
   up((void**)&f->cf_off, cnt.data(), sizeof(int) * cnt.size());
   up((void**)&f->cf_face, cf.data(), sizeof(int) * cf.size());
-  up((void**)&f->ent_face, ent.data(), sizeof(int) * ent.size());
-  up((void**)&f->c1, a.data(), sizeof(int) * a.size());
-  up((void**)&f->c2, b.data(), sizeof(int) * b.size());
+  up((void**)&f->cf_nbr, nbr.data(), sizeof(int) * nbr.size());
+  if (wide) up(&f->cf_slot, slot32.data(), sizeof(int) * slot32.size());
+  else up(&f->cf_slot, slot8.data(), slot8.size());
+  up((void**)&f->late, late.data(), late.size());
   up((void**)&f->flags, fl.data(), fl.size());
-  up((void**)&f->c2b, c2, sizeof(int) * (size_t)n_faces);
+  f->wide = wide;
+  f->unset = unset;
   f->max_bnd = max_bnd;
   f->n_ambient = n_ambient;
   f->shared_entry = shared_entry;
@@ -1413,19 +1450,10 @@ int tfg_momentum_assemble(tfg_faces* f, const tfg_momentum* m, double* val, doub
     return fail(TFG_ENOTSUP, "a matrix entry or a boundary cell belongs to two faces");
   tfg_matrix* h = f->h;
   HIP_TRY(hipSetDevice(h->device));
-  if (m->adv_scheme != TFG_ADV_CENTRAL && !f->pmin) {
-    HIP_TRY(hipMalloc(&f->pmin, sizeof(double) * (size_t)std::max(1, h->nt)));
-    HIP_TRY(hipMalloc(&f->pmax, sizeof(double) * (size_t)std::max(1, h->nt)));
-  }
+  if (m->adv_scheme != TFG_ADV_CENTRAL && !f->mm)
+    HIP_TRY(hipMalloc(&f->mm, sizeof(tfg::dbl2) * (size_t)std::max(1, h->nt)));
   tfg::MomArgs g{};
-  g.n = h->nt;
-  g.nb = m->n_bnd;
-  g.row = h->row;
-  g.cf_off = f->cf_off;
-  g.cf_face = f->cf_face;
-  g.ent_face = f->ent_face;
-  g.c1 = f->c1;
-  g.c2b = f->c2b;
+  g.t = cell_faces(f);
   g.comp = m->component;
   g.adv = m->adv_scheme;
   g.blend_matrix = m->blend_matrix ? 1 : 0;
@@ -1460,8 +1488,7 @@ int tfg_momentum_assemble(tfg_faces* f, const tfg_momentum* m, double* val, doub
   g.p_i = m->p_i;
   g.cell_f = m->cell_f;
   g.st = m->st;
-  g.pmin = f->pmin;
-  g.pmax = f->pmax;
+  g.mm = f->mm;
   g.val = val;
   g.b = b;
   g.v_m = v_m;
@@ -1494,9 +1521,7 @@ int tfg_rhie_chow_fluxes(tfg_faces* f, const tfg_rhie_chow* r, double* v_flux) {
   }
   HIP_TRY(hipSetDevice(f->device));
   tfg::RcArgs a{};
-  a.n_faces = f->n_faces;
-  a.c1 = f->c1;
-  a.c2 = f->c2;
+  a.t = cell_faces(f);
   a.r = *r;
   a.vof = vof ? 1 : 0;
   a.v_flux = v_flux;
@@ -1524,15 +1549,8 @@ int tfg_pressure_assemble_ex(tfg_faces* f, const double* fc, const double* fw, c
   tfg_matrix* h = f->h;
   HIP_TRY(hipSetDevice(h->device));
   tfg::AsmArgs g{};
-  g.n = h->nt;
-  g.row = h->row;
-  g.cf_off = f->cf_off;
-  g.cf_face = f->cf_face;
-  g.ent_face = f->ent_face;
-  g.c1 = f->c1;
-  g.c2 = f->c2;
+  g.t = cell_faces(f);
   g.flags = f->flags;
-  g.c2b = f->c2b;
   g.pp = pp;
   g.fc = fc;
   g.fw = fw;

@@ -8,6 +8,8 @@
 
 namespace tfg {
 
+typedef double dbl2 __attribute__((ext_vector_type(2)));
+
 constexpr int kBlock = 256;        // threads per workgroup (4 wave64)
 constexpr int kRowsPerBlock = 256; // SpMV rows per staged block (one per thread)
 // Nonzeros per staged block of the stream engines: 2040 (4088) fit 4 (8)
@@ -237,18 +239,25 @@ struct IccArgs {
   const int* toff_host;   // host: tile-level starts in bx.tiles (ntx + nty + ntz - 1 levels)
 };
 
-// Pressure-system assembly from face data (tfg_assembly.hip).
-struct AsmArgs {
+// Each cell's faces in increasing face order (tfg_faces_create).
+struct CellFaces {
   int n;                 // cells (rows) assembled: nt
   const int* row;        // 0-based CSR row starts (diagonal first)
-  const int* cf_off;     // n+1: each cell's faces in cf_face
-  const int* cf_face;    // face index * 2 + (1 if the cell is the face's c2)
-  const int* ent_face;   // nnz: last face setting each off-diagonal entry, -1 none
-  const int* c1;         // n_faces, 0-based
-  const int* c2;         // n_faces, 0-based; -1 for a boundary face
+  const int* off;        // n+1: each cell's faces in the lists below
+  const int* face;       // face index * 2 + (1 if the cell is the face's c2)
+  const int* nbr;        // the other cell, 1-based; c2 as given on the boundary (<= 0)
+  const void* slot;      // place of the entry (cell, nbr) in the cell's row: uint8_t,
+                         // or int when some row is longer than 256 entries (wide)
+  const uint8_t* late;   // n: 1 when a boundary face (c2 < 0) follows another face
+  int wide;
+  int unset;             // 1: some off-diagonal entry is set by no face
+};
+
+// Pressure-system assembly from face data (tfg_assembly.hip).
+struct AsmArgs {
+  CellFaces t;
   const uint8_t* flags;  // n_faces: 1 boundary diagonal term, 2 b(c1) = 0 (pressure
                          // region), 4 b(c1) = fc v_m(c1) pp(c2) (ambient region)
-  const int* c2b;        // n_faces: c2 as given (boundary cells < 0)
   const double* pp;      // pp % n at cell 1 (boundary cell c at pp[c - 1]); ambient only
   const double* fc;
   const double* fw;
@@ -262,30 +271,21 @@ struct AsmArgs {
 // Momentum assembly (tfg_assembly.hip).  Cell arrays point at cell 1 (a
 // 1-based cell C is element C - 1; boundary cells C < 0 below it).
 struct MomArgs {
-  int n, nb;
-  const int* row;
-  const int* cf_off;
-  const int* cf_face;
-  const int* ent_face;
-  const int* c1;         // 0-based
-  const int* c2b;        // 1-based as given (boundary cell < 0)
+  CellFaces t;
   int comp, adv, blend_matrix, td;
   double blend, dt, urf, p_drop;
   const double *f, *fw, *fc, *v_flux, *vis_eff, *f_stress;
   const double *sv[3], *dv[3];
   const int* wall;
   const double *phi, *phi_o, *phi_oo, *g[3], *uj_i, *uk_i, *rho, *vol, *p_i, *cell_f, *st;
-  double* pmin;          // n scratch values: min / max of phi over each cell's faces
-  double* pmax;
+  dbl2* mm;              // n scratch pairs: min and max of phi over each cell's faces
   double *val, *b, *v_m;
 };
 hipError_t launch_momentum(hipStream_t stream, const MomArgs& m);
 
-// Rhie-Chow face fluxes (tfg_assembly.hip); c1 0-based, c2 0-based or -1.
+// Rhie-Chow face fluxes (tfg_assembly.hip).
 struct RcArgs {
-  int n_faces;
-  const int* c1;
-  const int* c2;
+  CellFaces t;
   tfg_rhie_chow r;
   int vof;               // surface tension term active
   double* v_flux;

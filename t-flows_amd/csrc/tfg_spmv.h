@@ -35,7 +35,6 @@
 
 namespace tfg {
 
-typedef double dbl2 __attribute__((ext_vector_type(2)));
 typedef int int4v __attribute__((ext_vector_type(4)));
 
 // Contiguous share [first, end) of `count` items for this workgroup's XCD;
