@@ -210,6 +210,10 @@ struct tfg_matrix {
   int* pslot = nullptr;
   int* sorder = nullptr;  // (start, end) row blocks in processing order
   int nsorder = 0;
+  // window engine (kind 5): columns, counts and places of the row blocks; null
+  // when a block has too many different columns
+  int *ucol = nullptr, *ucnt = nullptr;
+  uint16_t* lidx = nullptr;
   tfg::SymDiag sdg{};     // symmetric engine geometry (offsets, stride, mode)
   int nsym = 0;        // upper diagonals; 0: no symmetric engine
   double* sym = nullptr;
@@ -285,6 +289,18 @@ int grid_vec_of(const tfg_matrix* h) {
   return std::max(1, std::min(gv, std::max(1, h->cu_count) * 3));
 }
 
+// Bytes that one FP64 iteration touches: the matrix as the engine reads it
+// and five vectors (x, r, p, q, the diagonal).  The FP32 forms touch half.
+long long iteration_bytes(const tfg_matrix* h, int kind) {
+  const long long n = h->nt, nnz = h->nnz;
+  const long long matrix = kind == tfg::K_SYM_DIA          ? 8 * (h->nsym + 1) * n
+                           : kind == tfg::K_PIPE_PATTERN   ? 8 * nnz + n
+                           : kind == tfg::K_PIPE2048_CODED ? 9 * nnz + 4 * n
+                           : kind == tfg::K_PIPE2048 && h->ucol ? 10 * nnz + 4 * n
+                                                                : 12 * nnz + 4 * n;
+  return matrix + 40 * n;
+}
+
 tfg::Launch launch_of(const tfg_matrix* h, const void* val, int kind) {
   tfg::Launch L;
   L.stream = h->stream;
@@ -293,6 +309,13 @@ tfg::Launch launch_of(const tfg_matrix* h, const void* val, int kind) {
   L.grid_vec = grid_vec_of(h);
   L.vec_val = ((uintptr_t)val % 16) == 0 && h->nnz >= 4;
   L.sym = false;
+  L.window = h->ucol != nullptr;
+  // Non-temporal loads of the matrix keep it out of the Infinity Cache, which
+  // costs when everything would have stayed there and gains when the vectors
+  // alone do.  Products with plain / non-temporal loads, us: 131x117x97 (107
+  // MB) 14.2 / 18.1, kNN 1M (215 MB) 35.9 / 51.8, upwind 120^3 (165 MB)
+  // 20.1 / 23.9; 160^3 (300 MB) 37.6 / 34.8, upwind 200^3 (766 MB) 112 / 104.
+  L.nt = iteration_bytes(h, kind) > tfg::kInfinityCache;
   return L;
 }
 
@@ -314,6 +337,9 @@ tfg::SpmvShape shape_of(const tfg_matrix* h, int kind) {
   m.sd = h->sym;
   m.sorder = h->sorder;
   m.nsorder = h->nsorder;
+  m.ucol = h->ucol;
+  m.ucnt = h->ucnt;
+  m.lidx = h->lidx;
   m.sdg = h->sdg;
   return m;
 }
@@ -337,6 +363,9 @@ tfg::CgArgs args_of(const tfg_matrix* h, int kind) {
   a.sd = m.sd;
   a.sorder = m.sorder;
   a.nsorder = m.nsorder;
+  a.ucol = m.ucol;
+  a.ucnt = m.ucnt;
+  a.lidx = m.lidx;
   a.sdg = m.sdg;
   return a;
 }
@@ -390,7 +419,7 @@ void free_all(tfg_matrix* h) {
                  h->r32, h->p32, h->q32, h->ad32, h->ns32[0], h->ns32[1], h->ns32[2],
                  h->ns32[3], h->ns32[4], h->valt32, h->rt, h->nv[0], h->nv[1], h->nv[2],
                  h->nv[3], h->valt, h->tpos, h->code, h->tab, h->pat, h->poff, h->plen,
-                 h->pslot, h->sym, h->sym_flag, h->sorder,
+                 h->pslot, h->sym, h->sym_flag, h->sorder, h->ucol, h->ucnt, h->lidx,
                  h->loc, h->vmax, h->vrange, h->icc_r64, h->z32, h->icc_rows[0],
                  h->icc_rows[1], h->icc_d, h->icc_dinv, h->icc_y, h->icc_z,
                  (void*)h->bx.tiles, h->bx.dg, h->bx.lo[0], h->bx.lo[1],
@@ -498,6 +527,45 @@ int tune_all(tfg_matrix* h, const double* val) {
     }
   }
   h->kind = best_k;
+  return TFG_OK;
+}
+
+// The window engine's tables for a handle whose products run kind 5 (made
+// with the handle, so that no product or solve allocates them).  Without the
+// memory for them, or when more than an eighth of the blocks have too many
+// different columns, kind 5 gathers x entry by entry.
+int window_setup(tfg_matrix* h) {
+  const int nb = h->nblk[0];
+  if (h->nnz < 4) return TFG_OK;
+  int* flag = nullptr;
+  int over = 0;
+  hipError_t e = hipMalloc(&h->ucol, sizeof(int) * (size_t)nb * tfg::kWindow);
+  if (e == hipSuccess) e = hipMalloc(&h->ucnt, sizeof(int) * (size_t)nb);
+  if (e == hipSuccess) e = hipMalloc(&h->lidx, sizeof(uint16_t) * ((size_t)h->nnz + 8));
+  if (e == hipSuccess) e = hipMalloc(&flag, sizeof(int));
+  const bool room = e == hipSuccess;
+  if (room) {
+    e = hipMemsetAsync(flag, 0, sizeof(int), h->stream);
+    if (e == hipSuccess)
+      e = hipMemsetAsync(h->lidx, 0, sizeof(uint16_t) * ((size_t)h->nnz + 8), h->stream);
+    if (e == hipSuccess)
+      e = tfg::launch_window_build(h->stream, shape_of(h, tfg::K_PIPE2048), h->ucol, h->ucnt,
+                                   h->lidx, flag);
+    if (e == hipSuccess) e = hipMemcpyAsync(&over, flag, sizeof(int), hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  }
+  if (flag) (void)hipFree(flag);
+  if (!room || e != hipSuccess || over > nb / 8) {
+    for (void* d : {(void*)h->ucol, (void*)h->ucnt, (void*)h->lidx})
+      if (d) (void)hipFree(d);
+    h->ucol = h->ucnt = nullptr;
+    h->lidx = nullptr;
+  }
+  if (!room) {
+    (void)hipGetLastError();
+    return TFG_OK;
+  }
+  HIP_TRY(e);
   return TFG_OK;
 }
 
@@ -793,12 +861,14 @@ int solve_ir(tfg_matrix* h, int prec, const double* val, const double* b, int mi
   if (sym) {
     L32.kind = tfg::K_SYM_DIA;
     L32.grid_spmv = h->grid32;
+    L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
   } else {
     if (L32.kind != tfg::K_STAGE2048 && L32.kind != tfg::K_PIPE2048_CODED &&
         L32.kind != tfg::K_PIPE_PATTERN)
       L32.kind = tfg::K_PIPE2048;
     L32.grid_spmv = h->grid[L32.kind];
     L32.vec_val = h->nnz >= 4;
+    L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
   }
   // one grid for every product-shaped kernel of this solve (their partials
   // are swept with it)
@@ -995,6 +1065,7 @@ int solve_ir_ns(tfg_matrix* h, int method, int prec, const double* val, const do
     L32.kind = tfg::K_PIPE2048;
   L32.grid_spmv = h->grid[L32.kind];
   L32.vec_val = h->nnz >= 4;
+  L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
   tfg::Launch L = launch_of(h, val, h->kind);
   L.grid_spmv = L32.grid_spmv;
   tfg::CgArgs a = args_of(h, h->kind);
@@ -1864,6 +1935,7 @@ int tfg_matrix_create(int ni, int nt, int nnz, const int* row, const int* col, c
           }
       if (cnt > 0 && dist / (double)cnt > nt / 64.0) (void)tfg_matrix_reorder(h, TFG_ORDER_RCM);
     }
+    if (rc == TFG_OK && !h->inner && default_kind(h) == tfg::K_PIPE2048) rc = window_setup(h);
   } while (0);
   if (rc != TFG_OK) {
     free_all(h);
@@ -2631,12 +2703,14 @@ int tfg_spmv_fp32(tfg_matrix* h, const double* d_val, double fn, const float* d_
   if (sym) {
     L32.kind = tfg::K_SYM_DIA;
     L32.grid_spmv = h->grid32;
+    L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
   } else {
     if (L32.kind != tfg::K_STAGE2048 && L32.kind != tfg::K_PIPE2048_CODED &&
         L32.kind != tfg::K_PIPE_PATTERN)
       L32.kind = tfg::K_PIPE2048;
     L32.grid_spmv = h->grid[L32.kind];
     L32.vec_val = h->nnz >= 4;
+    L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
   }
   tfg::Launch L = launch_of(h, d_val, h->kind);
   tfg::CgArgs a = args_of(h, h->kind);

@@ -25,6 +25,11 @@ constexpr int kPatMax = 12;
 // thread with.
 constexpr int kSymMax = 8;
 constexpr int kSymPairMax = 4;
+// Different columns a row block may have for its x entries to be gathered once
+// per block (WindowEngine): 8 KB of LDS in FP64, and four entries per thread; a
+// kNN graph in RCM order has at most about 970.
+constexpr int kWindow = 1024;
+constexpr long long kInfinityCache = 256LL << 20;  // MI355X, memory side
 constexpr int kXcds = 8;           // MI355X: 8 XCDs, workgroups dealt round robin
 constexpr double kHuge = 1.0e+15;  // Const_Mod.f90:84-93 (HUGE, TINY)
 constexpr double kTiny = 1.0e-15;
@@ -120,6 +125,9 @@ struct CgArgs {
   const int* pslot;    // symmetric engine: value slot of each pattern entry
   const int* sorder;   // symmetric engine: (start, end) row blocks in processing order
   int nsorder;
+  const int* ucol;     // window engine: each block's columns, counts, places (or null)
+  const int* ucnt;
+  const uint16_t* lidx;
   const double* sd;    // symmetric engine: diagonal and upper diagonals
   SymDiag sdg;         // symmetric engine: offsets, slot stride, row pairing
   const double* val;   // unscaled values (caller's)
@@ -156,6 +164,11 @@ struct SpmvShape {
   const double* __restrict__ sd;
   const int* __restrict__ sorder;    // symmetric engine: (start, end) row blocks
   int nsorder;                       //   in processing order, and their count
+  // window engine: kWindow slots per row block with its different columns,
+  // ascending; their number; each nonzero's place among its block's (padded)
+  const int* __restrict__ ucol;
+  const int* __restrict__ ucnt;
+  const uint16_t* __restrict__ lidx;
   SymDiag sdg;
 };
 
@@ -292,6 +305,12 @@ struct RcArgs {
 };
 hipError_t launch_rhie_chow(hipStream_t stream, const RcArgs& a);
 
+// Columns, counts and places of the window engine from the structure (m.blk:
+// the kCap blocks); lidx zeroed by the caller; *flag += the blocks
+// with more than kWindow different columns (count 0: gathered entry by entry).
+hipError_t launch_window_build(hipStream_t stream, const SpmvShape& m, int* ucol, int* ucnt,
+                               uint16_t* lidx, int* flag);
+
 // dst[k] = src[map[k]], k < count (permutation of values and vectors)
 hipError_t launch_gather(hipStream_t stream, const double* src, const int* map, double* dst,
                          long long count);
@@ -304,6 +323,9 @@ struct Launch {
   int kind;        // SpmvKind
   bool vec_val;    // val is 16-byte aligned (wide nontemporal loads)
   bool sym;        // products by the symmetric engine (val checked symmetric)
+  bool nt;         // non-temporal loads of what a product reads once: the data that
+                   // one iteration touches exceed the Infinity Cache (launch_of)
+  bool window;     // kind 5 has the columns of its row blocks (WindowEngine)
 };
 
 // Resident SpMV workgroups per CU for an engine (occupancy query).

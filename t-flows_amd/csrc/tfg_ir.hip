@@ -51,27 +51,6 @@ constexpr int kIrRes = 5;
 
 __device__ __forceinline__ bool ir_lead() { return blockIdx.x == 0 && threadIdx.x == 0; }
 
-__device__ __forceinline__ SpmvShape ir_shape(const CgArgs& a) {
-  SpmvShape m;
-  m.n = a.n;
-  m.row = a.row;
-  m.col = a.col;
-  m.blk = a.blk;
-  m.nblk = a.nblk;
-  m.code = a.code;
-  m.tab = a.tab;
-  m.ntab = a.ntab;
-  m.pat = a.pat;
-  m.poff = a.poff;
-  m.plen = a.plen;
-  m.pslot = a.pslot;
-  m.sd = a.sd;
-  m.sorder = a.sorder;
-  m.nsorder = a.nsorder;
-  m.sdg = a.sdg;
-  return m;
-}
-
 __device__ __forceinline__ double ir_measure(const State* st, double nrms, double xmin,
                                              double xmax, double rr) {
   if (st->criterion == TFG_CRIT_RELRES) return sqrt(rr) / st->bnorm;
@@ -229,7 +208,7 @@ __global__ __launch_bounds__(kBlock) void k_ir_spmv(CgArgs a, IrArgs f) {
   if (ir_lead()) a.st->kcur = a.st->kcur + 1;
   double v[1] = {0.0};
   E::template run<false, true>(
-      sm, ir_shape(a), f.val32, 1.0f, f.p32, s_tmp, s_out, [](int) { return 0.0f; },
+      sm, cg_shape(a), f.val32, 1.0f, f.p32, s_tmp, s_out, [](int) { return 0.0f; },
       [&](int i, float qi, float pi, float) {
         f.q32[i] = qi;
         v[0] = v[0] + (double)pi * (double)qi;
@@ -240,14 +219,14 @@ __global__ __launch_bounds__(kBlock) void k_ir_spmv(CgArgs a, IrArgs f) {
 
 // The same with the symmetric FP32 storage (K upper diagonals, MODE as in
 // SymEngine32).
-template <int K, int MODE>
+template <int K, int MODE, bool NT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 6)))
 void k_ir_spmv_sym(CgArgs a, IrArgs f) {
   __shared__ double s_tmp[4], s_out[1];
   if (a.st->done) return;
   if (ir_lead()) a.st->kcur = a.st->kcur + 1;
   double v[1] = {0.0};
-  SymEngine32::run<K, MODE>(
+  SymEngine32::run<K, MODE, NT>(
       a.sdg, f.sd32, f.stride32, a.n, f.sorder32, f.nsorder32, f.p32,
       [&](int i, float qi, float pi, bool own) {
         f.q32[i] = qi;
@@ -419,7 +398,7 @@ __global__ __launch_bounds__(kBlock) void k_ir_resid(CgArgs a, const double* __r
   const double fn = st->fn;
   double v[kIrRes] = {0.0, kHuge, -kHuge, 0.0, 0.0};
   E::template run<true>(
-      sm, ir_shape(a), a.val, fn, a.x, s_tmp, s_out, [&](int i) { return a.b[i] * fn; },
+      sm, cg_shape(a), a.val, fn, a.x, s_tmp, s_out, [&](int i) { return a.b[i] * fn; },
       [&](int i, double ri, double xi, double di) {
         a.r[i] = ri;
         v[0] = v[0] + (ri * ri) / (di * di);
@@ -524,11 +503,11 @@ __global__ __launch_bounds__(kBlock) void k_spmv_lap32(SpmvShape m, const float*
                                [&](int i, float yi, float, float) { y[i] = yi; });
 }
 
-template <int K, int MODE>
+template <int K, int MODE, bool NT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 6)))
 void k_spmv_lap32_sym(SymDiag g, int n, IrArgs f, const float* __restrict__ x,
                       float* __restrict__ y) {
-  SymEngine32::run<K, MODE>(
+  SymEngine32::run<K, MODE, NT>(
       g, f.sd32, f.stride32, n, f.sorder32, f.nsorder32, x,
       [&](int i, float yi, float, bool) { y[i] = yi; },
       [&](int i, const float (&q)[4], flt4, bool) {
@@ -550,23 +529,35 @@ void k_spmv_lap32_sym(SymDiag g, int n, IrArgs f, const float* __restrict__ x,
       case K_STAGE2048:                                                          \
         { using E = StreamEngine<kCap, false, float>; CALL; } break;             \
       case K_PIPE2048_CODED:                                                     \
-        { using E = StreamEngine<kCap, true, float, true>; CALL; } break;        \
+        if ((L).nt) { using E = StreamEngine<kCap, true, float, true, true>; CALL; } \
+        else { using E = StreamEngine<kCap, true, float, true, false>; CALL; }   \
+        break;                                                                   \
       case K_PIPE_PATTERN:                                                       \
-        { using E = PatternEngine<kCap, true, float>; CALL; } break;             \
+        if ((L).nt) { using E = PatternEngine<kCap, true, float, true>; CALL; }  \
+        else { using E = PatternEngine<kCap, true, float, false>; CALL; }        \
+        break;                                                                   \
       default:                                                                   \
-        if ((L).vec_val) { using E = StreamEngine<kCap, true, float>; CALL; }    \
+        if ((L).vec_val && (L).window && (L).nt) {                               \
+          using E = WindowEngine<kCap, float, true>; CALL;                       \
+        } else if ((L).vec_val && (L).window) {                                  \
+          using E = WindowEngine<kCap, float, false>; CALL;                      \
+        }                                                                        \
+        else if ((L).vec_val) { using E = GatherEngine<kCap, float>; CALL; }     \
         else { using E = ScalarStage<kCap, float>; CALL; }                       \
         break;                                                                   \
     }                                                                            \
   } while (0)
 
 template <typename F>
-static hipError_t sym32_dispatch(int K, int mode, F f) {
+static hipError_t sym32_dispatch(int K, int mode, bool nt, F f) {
   auto go = [&](auto kc) {
-    constexpr int KK = decltype(kc)::value;
-    if (mode == 1) f(kc, std::integral_constant<int, 1>{});
-    else f(kc, std::integral_constant<int, 0>{});
-    (void)KK;
+    if (mode == 1) {
+      if (nt) f(kc, std::integral_constant<int, 1>{}, std::true_type{});
+      else f(kc, std::integral_constant<int, 1>{}, std::false_type{});
+    } else {
+      if (nt) f(kc, std::integral_constant<int, 0>{}, std::true_type{});
+      else f(kc, std::integral_constant<int, 0>{}, std::false_type{});
+    }
   };
   switch (K) {
     case 1: go(std::integral_constant<int, 1>{}); break;
@@ -616,10 +607,11 @@ hipError_t launch_ir_pupdate(const Launch& L, const CgArgs& a, const IrArgs& f) 
 
 hipError_t launch_ir_spmv(const Launch& L32, const CgArgs& a, const IrArgs& f) {
   if (L32.kind == K_SYM_DIA) {
-    return sym32_dispatch(a.sdg.k, f.quad, [&](auto kc, auto mc) {
+    return sym32_dispatch(a.sdg.k, f.quad, L32.nt, [&](auto kc, auto mc, auto nc) {
       constexpr int K = decltype(kc)::value, MODE = decltype(mc)::value;
+      constexpr bool NT = decltype(nc)::value;
       if constexpr (MODE == 1 && K > kSymPairMax) return;
-      else k_ir_spmv_sym<K, MODE><<<L32.grid_spmv, kBlock, 0, L32.stream>>>(a, f);
+      else k_ir_spmv_sym<K, MODE, NT><<<L32.grid_spmv, kBlock, 0, L32.stream>>>(a, f);
     });
   }
   TFG_IR_ENGINE_SWITCH(L32, (k_ir_spmv<E><<<L32.grid_spmv, kBlock, 0, L32.stream>>>(a, f)));
@@ -675,10 +667,11 @@ hipError_t launch_ir_fold(const Launch& L, const CgArgs& a, const IrArgs& f) {
 hipError_t launch_spmv_lap32(const Launch& L32, const SpmvShape& m, const IrArgs& f,
                              const float* x, float* y) {
   if (L32.kind == K_SYM_DIA) {
-    return sym32_dispatch(m.sdg.k, f.quad, [&](auto kc, auto mc) {
+    return sym32_dispatch(m.sdg.k, f.quad, L32.nt, [&](auto kc, auto mc, auto nc) {
       constexpr int K = decltype(kc)::value, MODE = decltype(mc)::value;
+      constexpr bool NT = decltype(nc)::value;
       if constexpr (MODE == 1 && K > kSymPairMax) return;
-      else k_spmv_lap32_sym<K, MODE><<<L32.grid_spmv, kBlock, 0, L32.stream>>>(m.sdg, m.n, f, x, y);
+      else k_spmv_lap32_sym<K, MODE, NT><<<L32.grid_spmv, kBlock, 0, L32.stream>>>(m.sdg, m.n, f, x, y);
     });
   }
   TFG_IR_ENGINE_SWITCH(L32, (k_spmv_lap32<E><<<L32.grid_spmv, kBlock, 0, L32.stream>>>(m, f.val32, x, y)));

@@ -23,22 +23,6 @@ typedef float f32;
 
 __device__ __forceinline__ bool lead2() { return blockIdx.x == 0 && threadIdx.x == 0; }
 
-__device__ __forceinline__ SpmvShape shape2(const CgArgs& a) {
-  SpmvShape m;
-  m.n = a.n;
-  m.row = a.row;
-  m.col = a.col;
-  m.blk = a.blk;
-  m.nblk = a.nblk;
-  m.code = a.code;
-  m.tab = a.tab;
-  m.ntab = a.ntab;
-  m.pat = a.pat;
-  m.poff = a.poff;
-  m.plen = a.plen;
-  return m;
-}
-
 __device__ __forceinline__ void stop2(State* st, int k, double res, int status) {
   if (lead2()) {
     st->res = res;
@@ -154,13 +138,13 @@ __global__ __launch_bounds__(kBlock) void k_bicg32_spmv(CgArgs a, IrArgs f, NsAr
   if (in->done) return;
   double v[1] = {0.0};
   E::template run<false, true>(
-      sm, shape2(a), f.val32, 1.0f, f.p32, s_tmp, s_out, [](int) { return 0.0f; },
+      sm, cg_shape(a), f.val32, 1.0f, f.p32, s_tmp, s_out, [](int) { return 0.0f; },
       [&](int i, f32 qi, f32, f32) {
         f.q32[i] = qi;
         v[0] = v[0] + (double)s.v1[i] * (double)qi;
       });
   E::template run<false, true>(
-      sm, shape2(a), s.valt, 1.0f, s.v1, s_tmp, s_out, [](int) { return 0.0f; },
+      sm, cg_shape(a), s.valt, 1.0f, s.v1, s_tmp, s_out, [](int) { return 0.0f; },
       [&](int i, f32 qi, f32, f32) { s.v2[i] = qi; });
   const int ops[1] = {OP_SUM};
   publish<1>(v, ops, a.pt.spmv, a.pt.pstride, s_tmp, s_out);
@@ -231,7 +215,7 @@ __global__ __launch_bounds__(kBlock) void k_ns32_spmv_rv(CgArgs a, IrArgs f, Sta
   if (in->done) return;
   double v[1] = {0.0};
   E::template run<false, true>(
-      sm, shape2(a), f.val32, 1.0f, w, s_tmp, s_out, [](int) { return 0.0f; },
+      sm, cg_shape(a), f.val32, 1.0f, w, s_tmp, s_out, [](int) { return 0.0f; },
       [&](int i, f32 qi, f32, f32) {
         out[i] = qi;
         v[0] = v[0] + (double)rt[i] * (double)qi;
@@ -274,7 +258,7 @@ __global__ __launch_bounds__(kBlock) void k_cgs32_spmv_update(CgArgs a, IrArgs f
   const f32 alpha = (f32)in->alpha;
   double v[3] = {0.0, 0.0, 0.0};
   E::template run<false, true>(
-      sm, shape2(a), f.val32, 1.0f, s.v4, s_tmp, s_out, [](int) { return 0.0f; },
+      sm, cg_shape(a), f.val32, 1.0f, s.v4, s_tmp, s_out, [](int) { return 0.0f; },
       [&](int i, f32 qh, f32, f32) {
         const f32 rv = f.r32[i] - alpha * qh;
         f.r32[i] = rv;
@@ -348,7 +332,7 @@ __global__ __launch_bounds__(kBlock) void k_bcgs32_spmv_t(CgArgs a, IrArgs f, Ns
   __syncthreads();
   double v[2] = {0.0, 0.0};
   E::template run<false, true>(
-      sm, shape2(a), f.val32, 1.0f, s.v3, s_tmp, s_out, [](int) { return 0.0f; },
+      sm, cg_shape(a), f.val32, 1.0f, s.v3, s_tmp, s_out, [](int) { return 0.0f; },
       [&](int i, f32 ti, f32, f32) {
         s.v4[i] = ti;
         v[0] = v[0] + (double)ti * (double)s.v1[i];
@@ -471,11 +455,20 @@ __global__ __launch_bounds__(kBlock) void k_ns32_valt(CgArgs a, const int* __res
       case K_STAGE2048:                                                          \
         { using E = StreamEngine<kCap, false, float>; CALL; } break;             \
       case K_PIPE2048_CODED:                                                     \
-        { using E = StreamEngine<kCap, true, float, true>; CALL; } break;        \
+        if ((L).nt) { using E = StreamEngine<kCap, true, float, true, true>; CALL; } \
+        else { using E = StreamEngine<kCap, true, float, true, false>; CALL; }   \
+        break;                                                                   \
       case K_PIPE_PATTERN:                                                       \
-        { using E = PatternEngine<kCap, true, float>; CALL; } break;             \
+        if ((L).nt) { using E = PatternEngine<kCap, true, float, true>; CALL; }  \
+        else { using E = PatternEngine<kCap, true, float, false>; CALL; }        \
+        break;                                                                   \
       default:                                                                   \
-        if ((L).vec_val) { using E = StreamEngine<kCap, true, float>; CALL; }    \
+        if ((L).vec_val && (L).window && (L).nt) {                               \
+          using E = WindowEngine<kCap, float, true>; CALL;                       \
+        } else if ((L).vec_val && (L).window) {                                  \
+          using E = WindowEngine<kCap, float, false>; CALL;                      \
+        }                                                                        \
+        else if ((L).vec_val) { using E = GatherEngine<kCap, float>; CALL; }     \
         else { using E = ScalarStage<kCap, float>; CALL; }                       \
         break;                                                                   \
     }                                                                            \

@@ -42,27 +42,6 @@ __device__ __forceinline__ double measure(const State* st, double nrms, double x
 
 __device__ __forceinline__ bool lead() { return blockIdx.x == 0 && threadIdx.x == 0; }
 
-__device__ __forceinline__ SpmvShape shape_of(const CgArgs& a) {
-  SpmvShape m;
-  m.n = a.n;
-  m.row = a.row;
-  m.col = a.col;
-  m.blk = a.blk;
-  m.nblk = a.nblk;
-  m.code = a.code;
-  m.tab = a.tab;
-  m.ntab = a.ntab;
-  m.pat = a.pat;
-  m.poff = a.poff;
-  m.plen = a.plen;
-  m.pslot = a.pslot;
-  m.sd = a.sd;
-  m.sorder = a.sorder;
-  m.nsorder = a.nsorder;
-  m.sdg = a.sdg;
-  return m;
-}
-
 // ---------------------------------------------------------------------------
 // Phase kernels
 // ---------------------------------------------------------------------------
@@ -98,7 +77,7 @@ __global__ __launch_bounds__(kBlock) void k_prologue(CgArgs a) {
   }
   double v[7] = {0.0, 0.0, kHuge, -kHuge, 0.0, 0.0, 0.0};
   E::template run<true>(
-      sm, shape_of(a), a.val, fn, a.x, s_tmp, s_out, [&](int i) { return a.b[i] * fn; },
+      sm, cg_shape(a), a.val, fn, a.x, s_tmp, s_out, [&](int i) { return a.b[i] * fn; },
       [&](int i, double ri, double xi, double di) {
         const double bi = a.b[i] * fn;
         const double z = PREC == PREC_JACOBI ? ri * (1.0 / di) : ri;
@@ -261,7 +240,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_pq(CgArgs a, int k) {
   const double fn = a.st->fn;
   double v[1] = {0.0};
   E::template run<false>(
-      sm, shape_of(a), a.val, fn, a.p, s_tmp, s_out, [](int) { return 0.0; },
+      sm, cg_shape(a), a.val, fn, a.p, s_tmp, s_out, [](int) { return 0.0; },
       [&](int i, double qi, double pi, double) {
         a.q[i] = qi;
         v[0] = v[0] + pi * qi;
@@ -427,7 +406,7 @@ __global__ __launch_bounds__(kBlock) void k_true_residual(CgArgs a) {
   __shared__ double s_tmp[2 * 4], s_out[2];
   double v[2] = {0.0, 0.0};
   E::template run<true>(
-      sm, shape_of(a), a.val, 1.0, a.x, s_tmp, s_out, [&](int i) { return a.b[i]; },
+      sm, cg_shape(a), a.val, 1.0, a.x, s_tmp, s_out, [&](int i) { return a.b[i]; },
       [&](int i, double ri, double, double) {
         const double bi = a.b[i];
         v[0] = v[0] + ri * ri;
@@ -463,7 +442,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_plain(SpmvShape m, const double
 // upper diagonals, mode as in SymEngine): the same products as k_spmv_pq.
 // Six waves per SIMD leave the pair mode the registers to have all its
 // loads in flight at once (at eight it waits for the first ones midway).
-template <int K, int MODE>
+template <int K, int MODE, bool NT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 6)))
 void k_spmv_pq_sym(CgArgs a, int k) {
   __shared__ double s_tmp[4], s_out[1];
@@ -471,8 +450,8 @@ void k_spmv_pq_sym(CgArgs a, int k) {
   if (k == 0 && lead()) a.st->kcur = a.st->kcur + 1;  // as in k_spmv_pq
   const double fn = a.st->fn;
   double v[1] = {0.0};
-  SymEngine::run<false, K, MODE>(
-      shape_of(a), fn, a.p, [](int) { return 0.0; },
+  SymEngine::run<false, K, MODE, NT>(
+      cg_shape(a), fn, a.p, [](int) { return 0.0; },
       [&](int i, double qi, double pi, double, bool own) {
         a.q[i] = qi;
         v[0] = v[0] + (own ? pi * qi : 0.0);
@@ -489,10 +468,10 @@ void k_spmv_pq_sym(CgArgs a, int k) {
   publish<1>(v, ops, a.pt.spmv, a.pt.pstride, s_tmp, s_out);
 }
 
-template <int K, int MODE>
+template <int K, int MODE, bool NT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 6)))
 void k_spmv_plain_sym(SpmvShape m, const double* __restrict__ x, double* __restrict__ y) {
-  SymEngine::run<false, K, MODE>(
+  SymEngine::run<false, K, MODE, NT>(
       m, 1.0, x, [](int) { return 0.0; },
       [&](int i, double yi, double, double, bool) { y[i] = yi; },
       [&](int i, double y0, double y1, double, double, bool) {
@@ -541,18 +520,23 @@ __global__ __launch_bounds__(kBlock) void k_sym_pack(SpmvShape m, const double* 
   if (bad) atomicOr(flag, 1);
 }
 
-// Symmetric-engine instantiation for the runtime K: f(integral_constant<K>).
+// Symmetric-engine instantiation for the runtime K and NT:
+// f(integral_constant<K>, bool_constant<NT>).
 template <typename F>
-hipError_t sym_dispatch(int K, F f) {
+hipError_t sym_dispatch(int K, bool nt, F f) {
+  auto go = [&](auto kc) {
+    if (nt) f(kc, std::true_type{});
+    else f(kc, std::false_type{});
+  };
   switch (K) {
-    case 1: f(std::integral_constant<int, 1>{}); break;
-    case 2: f(std::integral_constant<int, 2>{}); break;
-    case 3: f(std::integral_constant<int, 3>{}); break;
-    case 4: f(std::integral_constant<int, 4>{}); break;
-    case 5: f(std::integral_constant<int, 5>{}); break;
-    case 6: f(std::integral_constant<int, 6>{}); break;
-    case 7: f(std::integral_constant<int, 7>{}); break;
-    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 5: go(std::integral_constant<int, 5>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}); break;
+    case 7: go(std::integral_constant<int, 7>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -577,14 +561,16 @@ int spmv_blocks_per_cu(int kind) {
     case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<StreamEngine<kCap2, false, double>>, kBlock, 0); break;
     case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<WaveEngine<4, double>>, kBlock, 0); break;
     case 3: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<WaveEngine<8, double>>, kBlock, 0); break;
-    case 5: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<StreamEngine<kCap, true, double>>, kBlock, 0); break;
-    case 6: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<StreamEngine<kCap, true, double, true>>, kBlock, 0); break;
-    case 7: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<PatternEngine<kCap, true, double>>, kBlock, 0); break;
-    case 8: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq_sym<3, 1>, kBlock, 0); break;
+    case 5: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<GatherEngine<kCap, double>>, kBlock, 0); break;
+    case 6: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<StreamEngine<kCap, true, double, true, true>>, kBlock, 0); break;
+    case 7: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<PatternEngine<kCap, true, double, true>>, kBlock, 0); break;
+    case 8: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq_sym<3, 1, true>, kBlock, 0); break;
     default: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<WaveEngine<16, double>>, kBlock, 0); break;
   }
   if (e != hipSuccess || nb < 1) return 1;
-  return nb;
+  // kind 5: five, as its row-per-thread form had.  The grid fixes the tree of
+  // the dot products, so a solve keeps its bits.
+  return kind == 5 ? std::min(nb, 5) : nb;
 }
 
 hipError_t launch_diag_sum(const Launch& L, const CgArgs& a) {
@@ -624,15 +610,16 @@ hipError_t launch_fold_x(const Launch& L, const CgArgs& a) {
 hipError_t launch_spmv_pq(const Launch& L, const CgArgs& a, int k) {
   if (L.sym) {
     const int mode = sym_mode(a.sdg, a.p, a.q);
-    return sym_dispatch(a.sdg.k, [&](auto kc) {
+    return sym_dispatch(a.sdg.k, L.nt, [&](auto kc, auto nc) {
       constexpr int K = decltype(kc)::value;
+      constexpr bool NT = decltype(nc)::value;
       if constexpr (K <= kSymPairMax)
         if (mode == 1) {
-          k_spmv_pq_sym<K, 1><<<L.grid_spmv, kBlock, 0, L.stream>>>(a, k);
+          k_spmv_pq_sym<K, 1, NT><<<L.grid_spmv, kBlock, 0, L.stream>>>(a, k);
           return;
         }
-      if (mode == 2) k_spmv_pq_sym<K, 2><<<L.grid_spmv, kBlock, 0, L.stream>>>(a, k);
-      else k_spmv_pq_sym<K, 0><<<L.grid_spmv, kBlock, 0, L.stream>>>(a, k);
+      if (mode == 2) k_spmv_pq_sym<K, 2, NT><<<L.grid_spmv, kBlock, 0, L.stream>>>(a, k);
+      else k_spmv_pq_sym<K, 0, NT><<<L.grid_spmv, kBlock, 0, L.stream>>>(a, k);
     });
   }
   TFG_ENGINE_SWITCH(L, (k_spmv_pq<E><<<L.grid_spmv, kBlock, 0, L.stream>>>(a, k)));
@@ -759,15 +746,16 @@ hipError_t launch_spmv_plain(const Launch& L, const SpmvShape& m, const double* 
                              const double* p, double* q) {
   if (L.sym) {
     const int mode = sym_mode(m.sdg, p, q);
-    return sym_dispatch(m.sdg.k, [&](auto kc) {
+    return sym_dispatch(m.sdg.k, L.nt, [&](auto kc, auto nc) {
       constexpr int K = decltype(kc)::value;
+      constexpr bool NT = decltype(nc)::value;
       if constexpr (K <= kSymPairMax)
         if (mode == 1) {
-          k_spmv_plain_sym<K, 1><<<L.grid_spmv, kBlock, 0, L.stream>>>(m, p, q);
+          k_spmv_plain_sym<K, 1, NT><<<L.grid_spmv, kBlock, 0, L.stream>>>(m, p, q);
           return;
         }
-      if (mode == 2) k_spmv_plain_sym<K, 2><<<L.grid_spmv, kBlock, 0, L.stream>>>(m, p, q);
-      else k_spmv_plain_sym<K, 0><<<L.grid_spmv, kBlock, 0, L.stream>>>(m, p, q);
+      if (mode == 2) k_spmv_plain_sym<K, 2, NT><<<L.grid_spmv, kBlock, 0, L.stream>>>(m, p, q);
+      else k_spmv_plain_sym<K, 0, NT><<<L.grid_spmv, kBlock, 0, L.stream>>>(m, p, q);
     });
   }
   TFG_ENGINE_SWITCH(L, (k_spmv_plain<E, false><<<L.grid_spmv, kBlock, 0, L.stream>>>(m, val, nullptr, p, q)));
@@ -787,6 +775,67 @@ hipError_t launch_gather(hipStream_t stream, const double* src, const int* map, 
   if (count <= 0) return hipSuccess;
   const long long blocks = (count + kBlock - 1) / kBlock;
   k_gather<<<(int)std::min<long long>(blocks, 4096), kBlock, 0, stream>>>(src, map, dst, count);
+  return hipGetLastError();
+}
+
+// One row block per workgroup, once per structure: its (column, entry) pairs
+// sorted in LDS (bitonic), then the different columns numbered.
+__global__ __launch_bounds__(kBlock) void k_window_build(SpmvShape m, int* __restrict__ ucol,
+                                                         int* __restrict__ ucnt,
+                                                         uint16_t* __restrict__ lidx, int* flag) {
+  constexpr int N = 2048, PER = N / kBlock;
+  static_assert(kCap <= N, "a block's entries fit the sort");
+  __shared__ unsigned long long key[N];
+  __shared__ int s_wave[kBlock / 64];
+  const int lb = blockIdx.x, tid = threadIdx.x;
+  const int s = m.row[m.blk[lb]], e = m.row[m.blk[lb + 1]], n = e - s;
+  if (n > kCap) {  // one long row: summed from global memory
+    if (tid == 0) {
+      ucnt[lb] = 0;
+      ucol[(size_t)lb * kWindow] = 0;  // read ahead, never used
+    }
+    return;
+  }
+  for (int t = tid; t < N; t += kBlock)
+    key[t] = t < n ? ((unsigned long long)(unsigned)m.col[s + t] << 32) | (unsigned)t : ~0ull;
+  for (int k = 2; k <= N; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      __syncthreads();
+      for (int t = tid; t < N / 2; t += kBlock) {
+        const int lo = 2 * j * (t / j) + (t % j), hi = lo + j;
+        const unsigned long long a = key[lo], b = key[hi];
+        const bool up = (lo & k) == 0;
+        if ((a > b) == up) {
+          key[lo] = b;
+          key[hi] = a;
+        }
+      }
+    }
+  __syncthreads();
+  int heads = 0;
+  for (int u = 0; u < PER; ++u) {
+    const int t = tid * PER + u;
+    heads += t < n && (t == 0 || (key[t] >> 32) != (key[t - 1] >> 32));
+  }
+  int rank = block_exclusive_scan(heads, s_wave) - 1;
+  for (int u = 0; u < PER; ++u) {
+    const int t = tid * PER + u;
+    if (t >= n) break;
+    if (t == 0 || (key[t] >> 32) != (key[t - 1] >> 32)) {
+      ++rank;
+      if (rank < kWindow) ucol[(size_t)lb * kWindow + rank] = (int)(key[t] >> 32);
+    }
+    lidx[s + (int)(key[t] & 0xffffffffu)] = (uint16_t)min(rank, kWindow - 1);
+    if (t == n - 1) {
+      ucnt[lb] = rank < kWindow ? rank + 1 : 0;
+      if (rank >= kWindow) atomicAdd(flag, 1);
+    }
+  }
+}
+
+hipError_t launch_window_build(hipStream_t stream, const SpmvShape& m, int* ucol, int* ucnt,
+                               uint16_t* lidx, int* flag) {
+  k_window_build<<<m.nblk, kBlock, 0, stream>>>(m, ucol, ucnt, lidx, flag);
   return hipGetLastError();
 }
 

@@ -32,22 +32,6 @@ __device__ __forceinline__ double measure1(const State* st, double nrms, double 
   return sqrt(nrms) / range;
 }
 
-__device__ __forceinline__ SpmvShape shape1(const CgArgs& a) {
-  SpmvShape m;
-  m.n = a.n;
-  m.row = a.row;
-  m.col = a.col;
-  m.blk = a.blk;
-  m.nblk = a.nblk;
-  m.code = a.code;
-  m.tab = a.tab;
-  m.ntab = a.ntab;
-  m.pat = a.pat;
-  m.poff = a.poff;
-  m.plen = a.plen;
-  return m;
-}
-
 __device__ __forceinline__ void stop_at(State* st, int k, double res, int status) {
   if (lead1()) {
     st->res = res;
@@ -157,13 +141,13 @@ __global__ __launch_bounds__(kBlock) void k_bicg_spmv(CgArgs a, NsArgs s) {
   const double fn = a.st->fn;
   double v[1] = {0.0};
   E::template run<false>(
-      sm, shape1(a), a.val, fn, a.p, s_tmp, s_out, [](int) { return 0.0; },
+      sm, cg_shape(a), a.val, fn, a.p, s_tmp, s_out, [](int) { return 0.0; },
       [&](int i, double qi, double, double) {
         a.q[i] = qi;
         v[0] = v[0] + s.v1[i] * qi;
       });
   E::template run<false>(
-      sm, shape1(a), s.valt, fn, s.v1, s_tmp, s_out, [](int) { return 0.0; },
+      sm, cg_shape(a), s.valt, fn, s.v1, s_tmp, s_out, [](int) { return 0.0; },
       [&](int i, double qi, double, double) { s.v2[i] = qi; });
   const int ops[1] = {OP_SUM};
   publish<1>(v, ops, a.pt.spmv, a.pt.pstride, s_tmp, s_out);
@@ -237,7 +221,7 @@ __global__ __launch_bounds__(kBlock) void k_ns_spmv_rv(CgArgs a, const double* w
   const double fn = a.st->fn;
   double v[1] = {0.0};
   E::template run<false>(
-      sm, shape1(a), a.val, fn, w, s_tmp, s_out, [](int) { return 0.0; },
+      sm, cg_shape(a), a.val, fn, w, s_tmp, s_out, [](int) { return 0.0; },
       [&](int i, double qi, double, double) {
         out[i] = qi;
         v[0] = v[0] + rt[i] * qi;
@@ -279,7 +263,7 @@ __global__ __launch_bounds__(kBlock) void k_cgs_spmv_update(CgArgs a, NsArgs s) 
   const double fn = st->fn, alpha = st->alpha;
   double v[5] = {0.0, kHuge, -kHuge, 0.0, 0.0};
   E::template run<false>(
-      sm, shape1(a), a.val, fn, s.v4, s_tmp, s_out, [](int) { return 0.0; },
+      sm, cg_shape(a), a.val, fn, s.v4, s_tmp, s_out, [](int) { return 0.0; },
       [&](int i, double qh, double, double d) {
         const double rv = a.r[i] - alpha * qh;
         const double xv = a.x[i];
@@ -361,7 +345,7 @@ __global__ __launch_bounds__(kBlock) void k_bcgs_spmv_t(CgArgs a, NsArgs s) {
   const double fn = st->fn;
   double v[2] = {0.0, 0.0};
   E::template run<false>(
-      sm, shape1(a), a.val, fn, s.v3, s_tmp, s_out, [](int) { return 0.0; },
+      sm, cg_shape(a), a.val, fn, s.v3, s_tmp, s_out, [](int) { return 0.0; },
       [&](int i, double ti, double, double) {
         s.v4[i] = ti;
         v[0] = v[0] + ti * s.v1[i];

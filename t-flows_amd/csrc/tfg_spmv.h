@@ -9,10 +9,12 @@
 // T is the value type of the matrix and of x (double, or float for the
 // inner solves of iterative refinement).
 //
+//  GatherEngine, WindowEngine  entries dealt four at a time, x gathered entry by
+//                         entry or once per row block (see there).
 //  StreamEngine<CAP, PIPE, T>  one row per thread; the workgroup first
 //                         streams the CSR values/columns of up to 256
 //                         consecutive rows (<= CAP nonzeros) into LDS with
-//                         coalesced 16-byte nontemporal loads, then each thread
+//                         coalesced 16-byte loads, then each thread
 //                         sums its row from LDS.  With PIPE, while a workgroup
 //                         sums block b the CSR streams of its next block are
 //                         already in flight into registers (issued after block
@@ -37,6 +39,31 @@ namespace tfg {
 
 typedef int int4v __attribute__((ext_vector_type(4)));
 
+// The structure that a CG kernel's arguments carry.
+__device__ __forceinline__ SpmvShape cg_shape(const CgArgs& a) {
+  SpmvShape m;
+  m.n = a.n;
+  m.row = a.row;
+  m.col = a.col;
+  m.blk = a.blk;
+  m.nblk = a.nblk;
+  m.code = a.code;
+  m.tab = a.tab;
+  m.ntab = a.ntab;
+  m.pat = a.pat;
+  m.poff = a.poff;
+  m.plen = a.plen;
+  m.ucol = a.ucol;
+  m.ucnt = a.ucnt;
+  m.lidx = a.lidx;
+  m.pslot = a.pslot;
+  m.sd = a.sd;
+  m.sorder = a.sorder;
+  m.nsorder = a.nsorder;
+  m.sdg = a.sdg;
+  return m;
+}
+
 // Contiguous share [first, end) of `count` items for this workgroup's XCD;
 // the XCD's workgroups take every `step`-th item starting at `first`.
 struct XcdWalk {
@@ -56,6 +83,15 @@ struct XcdWalk {
   }
 };
 
+// A load of data that one sweep reads once: non-temporal (NT) when a solve's
+// data exceed the Infinity Cache, so that it does not push out what the next
+// kernel reads again, a plain load when they fit it (launch_of).
+template <bool NT, typename V>
+__device__ __forceinline__ V stream_load(const V* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+
 // ---------------------------------------------------------------------------
 // A 16-byte-chunk stream of one CSR array (val or col) for one row block
 // [s, e): chunk t of the workgroup covers elements o + EPC*t .. + EPC-1 with
@@ -73,6 +109,7 @@ struct ChunkStream {
   V v[NCH];
   V tail;
 
+  template <bool NT>
   __device__ __forceinline__ void fetch(const E* __restrict__ arr, int nnz, int s, int e) {
     typedef __attribute__((address_space(4))) const E cE;
     const int tid = threadIdx.x;
@@ -84,7 +121,7 @@ struct ChunkStream {
 #pragma unroll
     for (int u = 0; u < NCH; ++u) {
       const int j = o + EPC * (tid + u * kBlock);
-      v[u] = __builtin_nontemporal_load(reinterpret_cast<const V*>(arr + min(j, lim)));
+      v[u] = stream_load<NT>(reinterpret_cast<const V*>(arr + min(j, lim)));
     }
   }
 
@@ -143,7 +180,7 @@ __device__ __forceinline__ T row_term(T a, T xj, T xi, bool first) {
 // CODED: the column stream is the 1-byte code of each nonzero's offset
 // col - row in a per-matrix table of at most 256 distinct offsets (a
 // structured grid has 7), a quarter of the int32 column traffic.
-template <int CAP, bool PIPE, typename T, bool CODED = false>
+template <int CAP, bool PIPE, typename T, bool CODED = false, bool NT = true>
 struct StreamEngine {
   typedef typename std::conditional<CODED, uint8_t, int>::type C;
   static constexpr int EPV = 16 / (int)sizeof(T);
@@ -179,11 +216,11 @@ struct StreamEngine {
     // A block that is one long row (e - s > CAP) is summed from global memory
     // and never staged; its loads here still stay inside the arrays.  No use
     // of the loaded values here: they stay in flight until put().
-    g.v.fetch(val, nnz, s, e);
+    g.v.template fetch<NT>(val, nnz, s, e);
     if constexpr (CODED)
-      g.c.fetch(m.code, nnz, s, e);
+      g.c.template fetch<NT>(m.code, nnz, s, e);
     else
-      g.c.fetch(m.col, nnz, s, e);
+      g.c.template fetch<NT>(m.col, nnz, s, e);
   }
 
   // column of staged entry j of row i
@@ -271,6 +308,311 @@ struct StreamEngine {
   }
 };
 
+// Kind 5, rows without a structure of their own (unstructured grids).  The
+// entries of a row block are dealt to the threads four at a time, whatever
+// rows they belong to, so every lane has its gathers of x in flight at once;
+// a_ij * x_j goes to LDS, and each row then adds its products in CSR order.
+// (With a row per thread, a block of 17-entry rows kept 120 of 256 threads
+// busy and each gathered its entries past the eighth one after another.)  The
+// row-excess form (LAP) needs the row's own x, so LDS holds a_ij and x_j.
+// While a block is summed the next block's values and columns are in flight
+// into registers.  One line of the L1 per gathered entry is what it takes most
+// time for: 1M rows, 16.8M entries 58 us (63 us with a row per thread); a
+// matrix whose blocks share columns runs WindowEngine instead.
+template <int CAP, typename T>
+struct GatherEngine {
+  static constexpr int NCH = (CAP / 4 + 1 + kBlock - 1) / kBlock;  // 4-entry chunks per thread
+  typedef T V __attribute__((ext_vector_type(4)));
+  struct Smem {
+    __attribute__((aligned(16))) T a[CAP + 8];
+    __attribute__((aligned(16))) T x[sizeof(T) == 4 ? CAP + 8 : 4];
+  };
+  struct Regs {
+    V v[NCH], vt;
+    int4v c[NCH], ct;
+    int r0, nr, s, e, rs, re;
+  };
+
+  template <bool NT>
+  __device__ __forceinline__ static V load4(const T* __restrict__ p) {
+    if constexpr (sizeof(T) == 4) {
+      return stream_load<NT>(reinterpret_cast<const V*>(p));
+    } else {
+      const dbl2 lo = stream_load<NT>(reinterpret_cast<const dbl2*>(p));
+      const dbl2 hi = stream_load<NT>(reinterpret_cast<const dbl2*>(p) + 1);
+      return V{lo.x, lo.y, hi.x, hi.y};
+    }
+  }
+
+  // Row i's terms (LDS, from o) added in CSR order, eight LDS reads at a time.
+  template <bool SUB, bool LAP, typename Epi>
+  __device__ __forceinline__ static void row_sum(const T* a, const T* xs, int o, int rs, int re,
+                                                 int i, T first, T xi,
+                                                 const T* __restrict__ val, T fn, Epi& epi) {
+    T acc = first;
+    for (int j0 = rs; j0 < re; j0 += 8) {
+      T q[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int j = min(j0 + u, re - 1) - o;
+        q[u] = LAP ? row_term<true>(a[j], xs[j], xi, j0 + u == rs) : a[j];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (j0 + u < re) acc = SUB ? acc - q[u] : acc + q[u];
+    }
+    epi(i, acc, xi, val[rs] * fn);
+  }
+
+  // Loads without branches, clamped into the block and the arrays (as in
+  // ChunkStream); the last 1..3 entries of the arrays, which no whole chunk
+  // holds, come from uniform loads (vt, ct).
+  __device__ __forceinline__ static void fetch(const SpmvShape& m, const T* __restrict__ val,
+                                               int nnz, int lb, Regs& g) {
+    typedef __attribute__((address_space(4))) const int cint;
+    typedef __attribute__((address_space(4))) const T cT;
+    const int tid = threadIdx.x;
+    const int r0 = ((cint*)m.blk)[lb], r1 = ((cint*)m.blk)[lb + 1];
+    const int s = ((cint*)m.row)[r0], e = ((cint*)m.row)[r1];
+    g.r0 = r0;
+    g.nr = r1 - r0;
+    g.s = s;
+    g.e = e;
+    g.rs = m.row[r0 + min(tid, r1 - r0)];
+    g.re = m.row[r0 + min(tid + 1, r1 - r0)];
+    const int o = s & ~3, jmax = (nnz - 4) & ~3, lim = min((e - 1) & ~3, jmax);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int j = min(jmax + 4 + k, nnz - 1);
+      g.vt[k] = ((cT*)val)[j];
+      g.ct[k] = ((cint*)m.col)[j];
+    }
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) {
+      const int j = min(o + 4 * (tid + u * kBlock), lim);
+      g.c[u] = *reinterpret_cast<const int4v*>(m.col + j);
+      g.v[u] = load4<false>(val + j);
+    }
+  }
+
+  template <bool SUB, bool LAP = false, typename Init, typename Epi>
+  __device__ __forceinline__ static void run(Smem& sm, const SpmvShape& m,
+                                             const T* __restrict__ val, T fn, const T* x,
+                                             double* s_tmp, double* s_out, Init init, Epi epi) {
+    static_assert(!LAP || sizeof(T) == 4, "LDS holds a and x for float");
+    const int tid = threadIdx.x;
+    const int nnz = m.row[m.n];
+    // laundered as in StreamEngine, so the gathers stay ahead of the prefetch
+    typedef __attribute__((address_space(1))) const T gT;
+    gT* xg = (gT*)x;
+    asm volatile("" : "+s"(xg));
+    const XcdWalk w(m.nblk);
+    Regs g;
+    int lb = w.first;
+    if (lb < w.end) fetch(m, val, nnz, lb, g);
+    while (lb < w.end) {
+      const int nxt = lb + w.step;
+      const int r0 = g.r0, nr = g.nr, s = g.s, e = g.e, rs = g.rs, re = g.re;
+      if (e - s > CAP) {
+        long_row<SUB, LAP>(m, val, fn, x, r0, s, e, s_tmp, s_out, init, epi);
+        fetch(m, val, nnz, min(nxt, w.end - 1), g);
+        lb = nxt;
+        continue;
+      }
+      const int o = s & ~3, jmax = (nnz - 4) & ~3, n = (e - o + 3) / 4;
+      const int i = r0 + min(tid, nr - 1);
+      V v[NCH], xv[NCH];
+#pragma unroll
+      for (int u = 0; u < NCH; ++u) {
+        const bool last = o + 4 * (tid + u * kBlock) > jmax;
+        v[u] = last ? g.vt : g.v[u];
+        const int4v c = last ? g.ct : g.c[u];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xv[u][k] = xg[c[k]];
+      }
+      const T xi = xg[i];
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(m, val, nnz, min(nxt, w.end - 1), g);
+      __builtin_amdgcn_sched_barrier(0);
+      const T first = init(i);
+#pragma unroll
+      for (int u = 0; u < NCH; ++u) {
+        const int t = tid + u * kBlock;
+        const V a = v[u] * fn;
+        if (t < n) {
+          if constexpr (LAP) {
+            *reinterpret_cast<V*>(&sm.a[4 * t]) = a;
+            *reinterpret_cast<V*>(&sm.x[4 * t]) = xv[u];
+          } else {
+            const V q = a * xv[u];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) sm.a[4 * t + k] = q[k];
+          }
+        }
+      }
+      __syncthreads();
+      if (tid < nr)
+        row_sum<SUB, LAP>(sm.a, sm.x, o, rs, re, i, first, xi, val, fn, epi);
+      __syncthreads();
+      lb = nxt;
+    }
+  }
+};
+
+// Kind 5 on a numbering with locality: the x entries a row block reads are
+// gathered once per block.  Of a block's 2040 entries only about 680 columns
+// are different ones on a kNN graph in RCM order, and sorted they lie in about
+// 105 lines of 128 bytes, against 2040 lines the entry-wise gathers ask the
+// L1 for.  The block's different columns in ascending order (ucol, at most
+// kWindow) and each entry's place among them (lidx, 16 bits in the place of
+// the 32-bit column) are made once per structure; x[ucol] goes to LDS, the
+// entries take their x from there and leave a_ij * x_j (LAP: a_ij and x_j) in
+// LDS, and each row adds its terms in CSR order.  In flight while a block is
+// summed: the next block's values, places and x entries, and the columns of
+// the one after.  1M rows, 16.8M entries (215 MB, from the Infinity Cache): 36 us,
+// GatherEngine 58 us; 4M rows 181 and 200 us.
+template <int CAP, typename T, bool NT>
+struct WindowEngine {
+  static constexpr int NCH = (CAP / 4 + 1 + kBlock - 1) / kBlock;  // 4-entry chunks per thread
+  static constexpr int NW = kWindow / kBlock;                      // window entries per thread
+  typedef T V __attribute__((ext_vector_type(4)));
+  typedef unsigned short us4 __attribute__((ext_vector_type(4)));
+  struct Smem {
+    __attribute__((aligned(16))) T a[CAP + 8];
+    __attribute__((aligned(16))) T x[sizeof(T) == 4 ? CAP + 8 : 4];
+    T win[kWindow];
+  };
+  struct Regs {
+    V v[NCH], vt;
+    us4 l[NCH];
+    int r0, nr, s, e, rs, re, cols;
+  };
+  struct Cols {
+    int c[NW];
+  };
+
+  // the columns of block lb (the last one repeated past their number)
+  __device__ __forceinline__ static void fetch_cols(const SpmvShape& m, int lb, Cols& q) {
+    typedef __attribute__((address_space(4))) const int cint;
+    const int last = max(((cint*)m.ucnt)[lb], 1) - 1;
+#pragma unroll
+    for (int u = 0; u < NW; ++u)
+      q.c[u] = m.ucol[(size_t)lb * kWindow + min((int)threadIdx.x + u * kBlock, last)];
+  }
+  __device__ __forceinline__ static void fetch(const SpmvShape& m, const T* __restrict__ val,
+                                               int nnz, int lb, Regs& g) {
+    typedef __attribute__((address_space(4))) const int cint;
+    typedef __attribute__((address_space(4))) const T cT;
+    const int tid = threadIdx.x;
+    const int r0 = ((cint*)m.blk)[lb], r1 = ((cint*)m.blk)[lb + 1];
+    const int s = ((cint*)m.row)[r0], e = ((cint*)m.row)[r1];
+    g.r0 = r0;
+    g.nr = r1 - r0;
+    g.s = s;
+    g.e = e;
+    g.cols = ((cint*)m.ucnt)[lb];
+    g.rs = m.row[r0 + min(tid, r1 - r0)];
+    g.re = m.row[r0 + min(tid + 1, r1 - r0)];
+    const int o = s & ~3, jmax = (nnz - 4) & ~3, lim = min((e - 1) & ~3, jmax);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) g.vt[k] = ((cT*)val)[min(jmax + 4 + k, nnz - 1)];
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) {
+      const int t = tid + u * kBlock, j = o + 4 * t;
+      // lidx is padded past its last entry; val is not
+      g.l[u] = stream_load<NT>(reinterpret_cast<const us4*>(m.lidx + min(j, (e - 1) & ~3)));
+      g.v[u] = GatherEngine<CAP, T>::template load4<NT>(val + min(j, lim));
+    }
+  }
+
+  template <bool SUB, bool LAP = false, typename Init, typename Epi>
+  __device__ __forceinline__ static void run(Smem& sm, const SpmvShape& m,
+                                             const T* __restrict__ val, T fn, const T* x,
+                                             double* s_tmp, double* s_out, Init init, Epi epi) {
+    static_assert(!LAP || sizeof(T) == 4, "LDS holds a and x for float");
+    const int tid = threadIdx.x;
+    const int nnz = m.row[m.n];
+    typedef __attribute__((address_space(1))) const T gT;
+    gT* xg = (gT*)x;
+    asm volatile("" : "+s"(xg));
+    const XcdWalk w(m.nblk);
+    Regs g;
+    Cols q;
+    T xw[NW];
+    int lb = w.first;
+    if (lb < w.end) {
+      fetch_cols(m, lb, q);
+      fetch(m, val, nnz, lb, g);
+#pragma unroll
+      for (int u = 0; u < NW; ++u) xw[u] = xg[q.c[u]];
+      fetch_cols(m, min(lb + w.step, w.end - 1), q);
+    }
+    while (lb < w.end) {
+      const int nxt = lb + w.step;
+      const int r0 = g.r0, nr = g.nr, s = g.s, e = g.e, rs = g.rs, re = g.re;
+      const int o = s & ~3, jmax = (nnz - 4) & ~3, n = (e - o + 3) / 4, cols = g.cols;
+      const int i = r0 + min(tid, nr - 1);
+      V v[NCH];
+      us4 l[NCH];
+#pragma unroll
+      for (int u = 0; u < NW; ++u) sm.win[tid + u * kBlock] = xw[u];
+#pragma unroll
+      for (int u = 0; u < NCH; ++u) {
+        v[u] = (o + 4 * (tid + u * kBlock) > jmax) ? g.vt : g.v[u];
+        l[u] = g.l[u];
+      }
+      const T xi = xg[i];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < NW; ++u) xw[u] = xg[q.c[u]];
+      fetch(m, val, nnz, min(nxt, w.end - 1), g);
+      fetch_cols(m, min(nxt + w.step, w.end - 1), q);
+      __builtin_amdgcn_sched_barrier(0);
+      if (e - s > CAP) {
+        __syncthreads();
+        long_row<SUB, LAP>(m, val, fn, x, r0, s, e, s_tmp, s_out, init, epi);
+        lb = nxt;
+        continue;
+      }
+      const T first = init(i);
+      __syncthreads();
+      if (cols > 0) {
+#pragma unroll
+        for (int u = 0; u < NCH; ++u) {
+          const int t = tid + u * kBlock;
+          V xv;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) xv[k] = sm.win[l[u][k]];
+          const V a = v[u] * fn;
+          if (t < n) {
+            if constexpr (LAP) {
+              *reinterpret_cast<V*>(&sm.a[4 * t]) = a;
+              *reinterpret_cast<V*>(&sm.x[4 * t]) = xv;
+            } else {
+              const V p = a * xv;
+#pragma unroll
+              for (int k = 0; k < 4; ++k) sm.a[4 * t + k] = p[k];
+            }
+          }
+        }
+      } else {  // more columns than the window holds: entry by entry
+#pragma unroll 1
+        for (int j = s + tid; j < e; j += kBlock) {
+          const T a = val[j] * fn, xj = x[m.col[j]];
+          sm.a[j - o] = LAP ? a : a * xj;
+          if constexpr (LAP) sm.x[j - o] = xj;
+        }
+      }
+      __syncthreads();
+      if (tid < nr)
+        GatherEngine<CAP, T>::template row_sum<SUB, LAP>(sm.a, sm.x, o, rs, re, i, first, xi,
+                                                         val, fn, epi);
+      lb = nxt;
+    }
+    __syncthreads();
+  }
+};
+
 // Exclusive prefix sum of v over the workgroup (thread order); s_wave needs
 // kBlock/64 ints.  Contains barriers: every thread must call it.
 __device__ __forceinline__ int block_exclusive_scan(int v, int* s_wave) {
@@ -296,7 +638,7 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* s_wave) {
 // pointers are read, only the values and one byte per row; a row's first
 // nonzero is the block's first plus the prefix sum of the pattern lengths
 // before it (one scan per block).  Otherwise the pipelined stream engine.
-template <int CAP, bool PIPE, typename T>
+template <int CAP, bool PIPE, typename T, bool NT = true>
 struct PatternEngine {
   static constexpr int EPV = 16 / (int)sizeof(T);
   static constexpr int NV = (CAP / EPV + 2 + kBlock - 1) / kBlock;
@@ -321,7 +663,7 @@ struct PatternEngine {
     g.s = s;
     g.e = e;
     g.pat = m.pat[r0 + min((int)threadIdx.x, r1 - r0 - 1)];
-    g.v.fetch(val, nnz, s, e);
+    g.v.template fetch<NT>(val, nnz, s, e);
   }
 
   template <bool SUB, bool LAP = false, typename Init, typename Epi>
@@ -431,13 +773,15 @@ struct SymEngine {
   __device__ __forceinline__ static T at(gB* base, unsigned byte) {
     return *(__attribute__((address_space(1))) const T*)(base + byte);
   }
-  template <typename T>  // non-temporal: no other row reads it
-  __device__ __forceinline__ static T at_nt(gB* base, unsigned byte) {
-    return __builtin_nontemporal_load((__attribute__((address_space(1))) const T*)(base + byte));
+  template <bool NT, typename T>  // what no other row reads
+  __device__ __forceinline__ static T at_own(gB* base, unsigned byte) {
+    const auto p = (__attribute__((address_space(1))) const T*)(base + byte);
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
   }
 
   // rows r0 + h * kBlock + tid, h < H, of block [r0, r1)
-  template <bool SUB, int K, int H, typename Init, typename Epi>
+  template <bool SUB, int K, int H, bool NT, typename Init, typename Epi>
   __device__ __forceinline__ static void rows(const SpmvShape& m, double fn, const double* x,
                                               int r0, int r1, Init& init, Epi& epi) {
     gB* xb = (gB*)x;
@@ -450,7 +794,7 @@ struct SymEngine {
       const int i = min(t, r1 - 1);
       const unsigned ib = 8u * (unsigned)i;
       double lo[K], up[K], xl[K], xu[K];
-      const double d = at_nt<double>(sb, ib);
+      const double d = at_own<NT, double>(sb, ib);
       const double x0 = at<double>(xb, ib);
 #pragma unroll
       for (int k = 0; k < K; ++k) {
@@ -473,7 +817,7 @@ struct SymEngine {
 
   // rows i, i + 1 (i = r0 + 2 tid, even) of block [r0, r1), r1 - r0 even;
   // epi2(i, y_i, y_{i+1}, x_i, x_{i+1}, own)
-  template <bool SUB, int K, typename Init, typename Epi2>
+  template <bool SUB, int K, bool NT, typename Init, typename Epi2>
   __device__ __forceinline__ static void pairs(const SpmvShape& m, double fn, const double* x,
                                                int r0, int r1, Init& init, Epi2& epi2) {
     gB* xb = (gB*)x;
@@ -497,7 +841,7 @@ struct SymEngine {
     }
     __builtin_amdgcn_sched_barrier(0);
     dbl2 lo[K], up[K], xl[K], xu[K];
-    const dbl2 d = at_nt<dbl2>(sb, ib);
+    const dbl2 d = at_own<NT, dbl2>(sb, ib);
     const dbl2 x0 = at<dbl2>(xb, ib);
     up[0] = at<dbl2>(sb + S8, ib);        // a(i, i+1), a(i+1, i+2)
     lo[0] = at<dbl2>(sb + S8 - 16, ib);   // .y = a(i-1, i)
@@ -532,7 +876,7 @@ struct SymEngine {
     epi2(i, a0, a1, x0.x, x0.y, t < r1);
   }
 
-  template <bool SUB, int K, int MODE, typename Init, typename Epi, typename Epi2>
+  template <bool SUB, int K, int MODE, bool NT, typename Init, typename Epi, typename Epi2>
   __device__ __forceinline__ static void run(const SpmvShape& m, double fn, const double* x,
                                              Init init, Epi epi, Epi2 epi2) {
     const XcdWalk w(m.nsorder);
@@ -540,8 +884,8 @@ struct SymEngine {
     int2 b = ids(m, w.first);
     for (int lb = w.first; lb < w.end; lb += w.step) {
       const int2 nb = ids(m, min(lb + w.step, w.end - 1));  // in flight during this block
-      if constexpr (MODE == 1) pairs<SUB, K>(m, fn, x, b.x, b.y, init, epi2);
-      else rows<SUB, K, MODE == 2 ? 2 : 1>(m, fn, x, b.x, b.y, init, epi);
+      if constexpr (MODE == 1) pairs<SUB, K, NT>(m, fn, x, b.x, b.y, init, epi2);
+      else rows<SUB, K, MODE == 2 ? 2 : 1, NT>(m, fn, x, b.x, b.y, init, epi);
       b = nb;
     }
   }
@@ -570,15 +914,17 @@ struct SymEngine32 {
   __device__ __forceinline__ static V at(gB* base, unsigned byte) {
     return *(__attribute__((address_space(1))) const V*)(base + byte);
   }
-  template <typename V>  // non-temporal: no other row reads it
-  __device__ __forceinline__ static V at_nt(gB* base, unsigned byte) {
-    return __builtin_nontemporal_load((__attribute__((address_space(1))) const V*)(base + byte));
+  template <bool NT, typename V>  // what no other row reads
+  __device__ __forceinline__ static V at_own(gB* base, unsigned byte) {
+    const auto p = (__attribute__((address_space(1))) const V*)(base + byte);
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
   }
   __device__ __forceinline__ static float term(float acc, float a, float xj, float xi) {
     return acc + a * (xj - xi);
   }
 
-  template <int K, typename Epi>
+  template <int K, bool NT, typename Epi>
   __device__ __forceinline__ static void rows(const SymDiag& g, const float* sd, long long S, int n,
                                               const float* x, int r0, int r1, Epi& epi) {
     gB* xb = (gB*)x;
@@ -589,7 +935,7 @@ struct SymEngine32 {
     const int i = min(t, r1 - 1);
     const unsigned ib = 4u * (unsigned)i;
     float lo[K], up[K], xl[K], xu[K];
-    const float s = at_nt<float>(sb, ib);
+    const float s = at_own<NT, float>(sb, ib);
     const float x0 = at<float>(xb, ib);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -608,7 +954,7 @@ struct SymEngine32 {
     epi(i, acc, x0, t < r1);
   }
 
-  template <int K, typename Epi4>
+  template <int K, bool NT, typename Epi4>
   __device__ __forceinline__ static void quads(const SymDiag& g, const float* sd, long long S,
                                                int n, const float* x, int r0, int r1, Epi4& epi4) {
     gB* xb = (gB*)x;
@@ -630,7 +976,7 @@ struct SymEngine32 {
     }
     __builtin_amdgcn_sched_barrier(0);
     flt4 lo[K], up[K], xl[K], xu[K];
-    const flt4 s = at_nt<flt4>(sb, ib);
+    const flt4 s = at_own<NT, flt4>(sb, ib);
     const flt4 x0 = at<flt4>(xb, ib);
     up[0] = at<flt4>(sb + S4, ib);        // a(i, i+1) .. a(i+3, i+4)
     lo[0] = at<flt4>(sb + S4 - 16, ib);   // .w = a(i-1, i)
@@ -664,7 +1010,7 @@ struct SymEngine32 {
     epi4(i, y, x0, t < r1);
   }
 
-  template <int K, int MODE, typename Epi, typename Epi4>
+  template <int K, int MODE, bool NT, typename Epi, typename Epi4>
   __device__ __forceinline__ static void run(const SymDiag& g, const float* sd, long long S, int n,
                                              const int* sorder, int nsorder, const float* x,
                                              Epi epi, Epi4 epi4) {
@@ -672,8 +1018,8 @@ struct SymEngine32 {
     const XcdWalk w(nsorder);
     for (int lb = w.first; lb < w.end; lb += w.step) {
       const int r0 = ((cint*)sorder)[2 * lb], r1 = ((cint*)sorder)[2 * lb + 1];
-      if constexpr (MODE == 1) quads<K>(g, sd, S, n, x, r0, r1, epi4);
-      else rows<K>(g, sd, S, n, x, r0, r1, epi);
+      if constexpr (MODE == 1) quads<K, NT>(g, sd, S, n, x, r0, r1, epi4);
+      else rows<K, NT>(g, sd, S, n, x, r0, r1, epi);
     }
   }
 };
@@ -849,8 +1195,9 @@ struct WaveEngine {
 };
 
 // kind: 0 stage/kCap, 1 stage/kCap2, 2 wave/4, 3 wave/8, 4 wave/16,
-// 5 pipelined stage/kCap, 6 the same with offset-coded columns, 7 the same
-// with row patterns (also kind 8: the symmetric engine serves only the CG
+// 5 entries dealt to the threads (GatherEngine, or WindowEngine where the handle
+// holds the blocks' columns), 6 pipelined stage/kCap with offset-coded columns,
+// 7 the same with row patterns (also kind 8: the symmetric engine serves only the CG
 // product and the plain product, when Launch::sym is set; every other
 // kernel uses the row-pattern engine).  The stage engines fall back to scalar staging
 // (ScalarStage) when val is not 16-byte aligned or nnz < 4.
@@ -866,16 +1213,29 @@ struct WaveEngine {
         else { using E = ScalarStage<kCap2, T>; CALL; }                             \
         break;                                                                     \
       case 5:                                                                      \
-        if ((L).vec_val) { using E = StreamEngine<kCap, true, T>; CALL; }          \
+        if ((L).vec_val && (L).window && (L).nt) {                                 \
+          using E = WindowEngine<kCap, T, true>; CALL;                             \
+        } else if ((L).vec_val && (L).window) {                                    \
+          using E = WindowEngine<kCap, T, false>; CALL;                            \
+        }                                                                          \
+        else if ((L).vec_val) { using E = GatherEngine<kCap, T>; CALL; }           \
         else { using E = ScalarStage<kCap, T>; CALL; }                             \
         break;                                                                     \
       case 6:                                                                      \
-        if ((L).vec_val) { using E = StreamEngine<kCap, true, T, true>; CALL; }    \
+        if ((L).vec_val && (L).nt) {                                               \
+          using E = StreamEngine<kCap, true, T, true, true>; CALL;                 \
+        } else if ((L).vec_val) {                                                  \
+          using E = StreamEngine<kCap, true, T, true, false>; CALL;                \
+        }                                                                          \
         else { using E = ScalarStage<kCap, T>; CALL; }                             \
         break;                                                                     \
       case 7:                                                                      \
       case 8:                                                                      \
-        if ((L).vec_val) { using E = PatternEngine<kCap, true, T>; CALL; }         \
+        if ((L).vec_val && (L).nt) {                                               \
+          using E = PatternEngine<kCap, true, T, true>; CALL;                      \
+        } else if ((L).vec_val) {                                                  \
+          using E = PatternEngine<kCap, true, T, false>; CALL;                     \
+        }                                                                          \
         else { using E = ScalarStage<kCap, T>; CALL; }                             \
         break;                                                                     \
       case 2: { using E = WaveEngine<4, T>; CALL; } break;                         \
