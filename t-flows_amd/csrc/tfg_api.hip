@@ -113,10 +113,10 @@ unsigned char* scratch_of(int device) {
 struct GraphKey {
   const void* val;
   const void* b;
-  int prec, dx, chunk, kind, sym;
+  int prec, dx, rel, chunk, kind, sym;
   bool operator==(const GraphKey& o) const {
-    return val == o.val && b == o.b && prec == o.prec && dx == o.dx && chunk == o.chunk &&
-           kind == o.kind && sym == o.sym;
+    return val == o.val && b == o.b && prec == o.prec && dx == o.dx && rel == o.rel &&
+           chunk == o.chunk && kind == o.kind && sym == o.sym;
   }
 };
 
@@ -2307,6 +2307,7 @@ int tfg_solve_native_ex(tfg_matrix* h, const char* solver, int solver_len, const
     a.pt = partials_of(h, L);
     a.st = h->st;
     if (method == tfg::NS_CGS) a.pt.g_upd = L.grid_spmv;
+    a.rel = method == tfg::NS_NONE && o.criterion == TFG_CRIT_RELRES ? 1 : 0;
     tfg::NsArgs ns{};
     if (method != tfg::NS_NONE) {
       const int rn = ensure_nonsym(h, method, dval, L);
@@ -2379,7 +2380,7 @@ int tfg_solve_native_ex(tfg_matrix* h, const char* solver, int solver_len, const
       return TFG_OK;
     };
     if (graph) {
-      const GraphKey key{dval, db, pr, dx ? 1 : 0, chunk, h->kind, L.sym ? 1 : 0};
+      const GraphKey key{dval, db, pr, dx ? 1 : 0, a.rel, chunk, h->kind, L.sym ? 1 : 0};
       if (!h->cg_graph || !(h->cg_key == key)) {
         if (h->cg_graph) {
           HIP_TRY(hipGraphExecDestroy(h->cg_graph));
@@ -2579,6 +2580,7 @@ int tfg_solve_native_noalloc(tfg_matrix* h, const char* solver, int solver_len, 
   a.ad = ad;
   a.pt = partials_of(h, L, part);
   a.st = st;
+  a.rel = o.criterion == TFG_CRIT_RELRES ? 1 : 0;
   if (symk) {
     // the diagonals' absent entries and slot gaps must read zero
     HIP_TRY(tfg::launch_zero16(S, sd, (long long)(sdb / 16)));

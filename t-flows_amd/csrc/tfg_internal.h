@@ -136,7 +136,9 @@ struct CgArgs {
   double* r;
   double* p;
   double* q;
-  double* ad;          // scaled diagonal a_ii * fn
+  double* ad;          // scaled diagonal a_ii * fn, or its reciprocal (rel)
+  int rel;             // FP64 CG stopped on the relative residual: ad holds
+                       // 1 / (a_ii fn), and the sums only NRMS needs are not formed
   Partials pt;
   State* st;
 };

@@ -128,33 +128,42 @@ __global__ __launch_bounds__(kBlock) void k_ir_symcheck(const double* __restrict
 // mu = (s, z) / E (deflation; 0 without), p = z + beta p - mu with
 // z = r / a_ii (Jacobi) or r, and the deferred e += alpha_{k-1} p_{k-1} on
 // the p read anyway.
+// Loads in the order of k_pupdate (tfg_kernels.hip): the partials, then
+// kIrItems quadruples, then the wait for the partials, the next quadruples in
+// flight while some are processed.  160^3: 17.3 us without that, 16.0 us now
+// (98 MB; 200^3 29.7 and 28.6); two or four quadruples at a time are slower
+// there (200^3 30.6).
+constexpr int kIrItems = 1;
 template <int PREC>
-__global__ __launch_bounds__(kBlock) void k_ir_pupdate(CgArgs a, IrArgs f) {
-  __shared__ double s_tmp[kIrUpd * 4], s_out[kIrUpd];
+__global__ __launch_bounds__(kBlock, 3) void k_ir_pupdate(CgArgs a, IrArgs f) {
+  __shared__ double s_tmp[3 * 4], s_out[3];
   State* st = a.st;
-  if (st->done) return;
-  const int k = st->kcur;
+  const int done = st->done, k = st->kcur;
   const bool fresh = k == st->kref + 1;
-  const int stride = gridDim.x * kBlock;
   const int n4 = a.n >> 2;
   flt4* p4 = reinterpret_cast<flt4*>(f.p32);
   flt4* e4 = reinterpret_cast<flt4*>(f.e32);
   const flt4* r4 = reinterpret_cast<const flt4*>(f.r32);
   const flt4* d4 = reinterpret_cast<const flt4*>(f.rd32);
-  // this thread's first quadruple, loaded before the sweep of the partials
-  const int t0 = blockIdx.x * kBlock + threadIdx.x;
-  const int tq = n4 > 0 ? min(t0, n4 - 1) : 0;
-  flt4 rv0 = {0.f, 0.f, 0.f, 0.f}, dv0 = {1.f, 1.f, 1.f, 1.f}, pv0 = rv0, ev0 = rv0;
-  if (n4 > 0) {
-    rv0 = r4[tq];
-    if (PREC == PREC_JACOBI) dv0 = d4[tq];
-    if (!fresh) {
-      pv0 = p4[tq];
-      ev0 = e4[tq];
-    }
-  }
-  const int ops[kIrUpd] = {OP_SUM, OP_SUM, OP_SUM, OP_SUM};
-  gather<kIrUpd>(a.pt.upd, a.pt.pstride, a.pt.g_vec, ops, s_tmp, s_out);
+  Sweep<3, 3> sums;  // (z, r), (s, z), (r, r)
+#pragma unroll
+  for (int c = 0; c < 3; ++c) sums.row[c] = a.pt.upd + c * a.pt.pstride;
+  sums.issue(a.pt.g_vec);
+  struct Item {
+    flt4 r, d, p, e;
+  };
+  auto load = [&](Item& w, int t) {
+    w.r = r4[t];
+    if (PREC == PREC_JACOBI) w.d = d4[t];
+    w.p = p4[t];
+    w.e = e4[t];
+  };
+  Item first[kIrItems];
+  if (n4 > 0) first_items<kIrItems>(n4, first, load);
+  __builtin_amdgcn_sched_barrier(0);
+  const int ops[3] = {OP_SUM, OP_SUM, OP_SUM};
+  sums.finish(a.pt.g_vec, ops, s_tmp, s_out);
+  if (done) return;
   const double rho = s_out[0];
   if (!isfinite(rho)) {
     if (ir_lead()) {
@@ -171,21 +180,16 @@ __global__ __launch_bounds__(kBlock) void k_ir_pupdate(CgArgs a, IrArgs f) {
     st->rho[k & 1] = rho;
     if (fresh) st->rref = s_out[2];
   }
-  auto quad = [&](int t, flt4 rv, flt4 dv, flt4 pv, flt4 ev) {
-    const flt4 z = PREC == PREC_JACOBI ? rv * dv : rv;
+  auto quad = [&](int t, const Item& w) {
+    const flt4 z = PREC == PREC_JACOBI ? w.r * w.d : w.r;
     if (fresh) {
       p4[t] = z - mu;
     } else {
-      e4[t] = ev + ap * pv;
-      p4[t] = (z + beta * pv) - mu;
+      e4[t] = w.e + ap * w.p;
+      p4[t] = (z + beta * w.p) - mu;
     }
   };
-  if (t0 < n4) quad(t0, rv0, dv0, pv0, ev0);
-  for (int t = t0 + stride; t < n4; t += stride) {
-    const flt4 dv = PREC == PREC_JACOBI ? d4[t] : flt4{1.f, 1.f, 1.f, 1.f};
-    quad(t, r4[t], dv, fresh ? flt4{0.f, 0.f, 0.f, 0.f} : p4[t],
-         fresh ? flt4{0.f, 0.f, 0.f, 0.f} : e4[t]);
-  }
+  if (n4 > 0) stream_items<kIrItems>(n4, first, load, quad);
   if (blockIdx.x == 0 && (int)threadIdx.x < (a.n & 3)) {
     const int i = 4 * n4 + threadIdx.x;
     const float z = PREC == PREC_JACOBI ? f.r32[i] * f.rd32[i] : f.r32[i];
@@ -248,31 +252,40 @@ void k_ir_spmv_sym(CgArgs a, IrArgs f) {
 
 // alpha = rho_k / (p, q) (FP64); r -= alpha q; partials of the next (z, r),
 // (s, z) (deflation), (r, r) and the NRMS sum of the FP32 residual.
+// Only the sums that are read again are formed.  160^3: 16.5 us before, 15.6 us
+// now (loads ordered as in k_ir_pupdate; 200^3 25.8 and 24.9).
 template <int PREC, bool DEFL, bool NRMS>
-__global__ __launch_bounds__(kBlock) void k_ir_update(CgArgs a, IrArgs f) {
+__global__ __launch_bounds__(kBlock, 3) void k_ir_update(CgArgs a, IrArgs f) {
   __shared__ double s_tmp[kIrUpd * 4], s_out[kIrUpd];
   State* st = a.st;
-  if (st->done) return;
+  const int done = st->done;
   const int k = st->kcur - 1;  // the product of this iteration advanced it
-  const int stride = gridDim.x * kBlock;
   const int n4 = a.n >> 2;
   flt4* r4 = reinterpret_cast<flt4*>(f.r32);
   const flt4* q4 = reinterpret_cast<const flt4*>(f.q32);
   const flt4* d4 = reinterpret_cast<const flt4*>(f.rd32);
   const flt4* s4 = reinterpret_cast<const flt4*>(f.s32);
-  const int t0 = blockIdx.x * kBlock + threadIdx.x;
-  const int tq = n4 > 0 ? min(t0, n4 - 1) : 0;
-  flt4 rv0 = {0.f, 0.f, 0.f, 0.f}, qv0 = rv0, dv0 = rv0, sv0 = rv0;
-  if (n4 > 0) {
-    rv0 = r4[tq];
-    qv0 = q4[tq];
-    dv0 = d4[tq];
-    if (DEFL) sv0 = s4[tq];
-  }
+  constexpr bool kDiag = PREC == PREC_JACOBI || NRMS;
+  Sweep<1, 6> sum;
+  sum.row[0] = a.pt.spmv;
+  sum.issue(a.pt.g_spmv);
+  struct Item {
+    flt4 r, q, d, s;
+  };
+  auto load = [&](Item& w, int t) {
+    w.r = r4[t];
+    w.q = q4[t];
+    if (kDiag) w.d = d4[t];
+    if (DEFL) w.s = s4[t];
+  };
+  Item first[kIrItems];
+  if (n4 > 0) first_items<kIrItems>(n4, first, load);
+  __builtin_amdgcn_sched_barrier(0);
   {
     const int ops1[1] = {OP_SUM};
-    gather<1>(a.pt.spmv, a.pt.pstride, a.pt.g_spmv, ops1, s_tmp, s_out);
+    sum.finish(a.pt.g_spmv, ops1, s_tmp, s_out);
   }
+  if (done) return;
   const double pq = s_out[0];
   if (pq == 0.0 || !isfinite(pq)) {
     if (ir_lead()) {
@@ -297,12 +310,12 @@ __global__ __launch_bounds__(kBlock) void k_ir_update(CgArgs a, IrArgs f) {
       v[3] = v[3] + t * t;
     }
   };
-  auto quad = [&](int t, flt4 rv, flt4 qv, flt4 dv, flt4 sv) {
-    float r0 = rv.x, r1 = rv.y, r2 = rv.z, r3 = rv.w;
-    one(r0, qv.x, dv.x, sv.x);
-    one(r1, qv.y, dv.y, sv.y);
-    one(r2, qv.z, dv.z, sv.z);
-    one(r3, qv.w, dv.w, sv.w);
+  auto quad = [&](int t, const Item& w) {
+    float r0 = w.r.x, r1 = w.r.y, r2 = w.r.z, r3 = w.r.w;
+    one(r0, w.q.x, w.d.x, w.s.x);
+    one(r1, w.q.y, w.d.y, w.s.y);
+    one(r2, w.q.z, w.d.z, w.s.z);
+    one(r3, w.q.w, w.d.w, w.s.w);
     flt4 o;
     o.x = r0;
     o.y = r1;
@@ -310,17 +323,29 @@ __global__ __launch_bounds__(kBlock) void k_ir_update(CgArgs a, IrArgs f) {
     o.w = r3;
     r4[t] = o;
   };
-  if (t0 < n4) quad(t0, rv0, qv0, dv0, sv0);
-  for (int t = t0 + stride; t < n4; t += stride)
-    quad(t, r4[t], q4[t], d4[t], DEFL ? s4[t] : flt4{0.f, 0.f, 0.f, 0.f});
+  if (n4 > 0) stream_items<kIrItems>(n4, first, load, quad);
   if (blockIdx.x == 0 && (int)threadIdx.x < (a.n & 3)) {
     const int i = 4 * n4 + threadIdx.x;
     float r = f.r32[i];
-    one(r, f.q32[i], f.rd32[i], DEFL ? f.s32[i] : 0.0f);
+    one(r, f.q32[i], kDiag ? f.rd32[i] : 0.0f, DEFL ? f.s32[i] : 0.0f);
     f.r32[i] = r;
   }
-  const int ops[kIrUpd] = {OP_SUM, OP_SUM, OP_SUM, OP_SUM};
-  publish<kIrUpd>(v, ops, a.pt.upd, a.pt.pstride, s_tmp, s_out);
+  if (DEFL && NRMS) {
+    const int ops[4] = {OP_SUM, OP_SUM, OP_SUM, OP_SUM};
+    publish<4>(v, ops, a.pt.upd, a.pt.pstride, s_tmp, s_out);
+  } else if (DEFL) {
+    double w[3] = {v[0], v[1], v[2]};
+    const int ops[3] = {OP_SUM, OP_SUM, OP_SUM};
+    publish<3>(w, ops, a.pt.upd, a.pt.pstride, s_tmp, s_out);
+  } else if (NRMS) {
+    double w[3] = {v[0], v[2], v[3]};
+    const int ops[3] = {OP_SUM, OP_SUM, OP_SUM}, rows[3] = {0, 2, 3};
+    publish_rows<3>(w, ops, rows, a.pt.upd, a.pt.pstride, s_tmp, s_out);
+  } else {
+    double w[2] = {v[0], v[2]};
+    const int ops[2] = {OP_SUM, OP_SUM}, rows[2] = {0, 2};
+    publish_rows<2>(w, ops, rows, a.pt.upd, a.pt.pstride, s_tmp, s_out);
+  }
 }
 
 // ---------------------------------------------------------------------------

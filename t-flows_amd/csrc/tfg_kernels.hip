@@ -80,9 +80,10 @@ __global__ __launch_bounds__(kBlock) void k_prologue(CgArgs a) {
       sm, cg_shape(a), a.val, fn, a.x, s_tmp, s_out, [&](int i) { return a.b[i] * fn; },
       [&](int i, double ri, double xi, double di) {
         const double bi = a.b[i] * fn;
-        const double z = PREC == PREC_JACOBI ? ri * (1.0 / di) : ri;
+        const double inv = 1.0 / di;
+        const double z = PREC == PREC_JACOBI ? ri * inv : ri;
         a.r[i] = ri;
-        a.ad[i] = di;
+        a.ad[i] = a.rel ? inv : di;
         v[0] = v[0] + (bi * bi) / (di * di);
         v[1] = v[1] + (ri * ri) / (di * di);
         v[2] = fmin(v[2], xi);
@@ -139,35 +140,55 @@ __global__ __launch_bounds__(kBlock) void k_start(CgArgs a, int rho_slot) {
 // operation on the same operands, one iteration later, 8n bytes fewer per
 // iteration.  The last iteration's term is folded by k_fold_x.
 // k = 0: the iteration number is State::kcur (graph-replayed chunks).
-template <int PREC, bool DX>
-__global__ __launch_bounds__(kBlock) void k_pupdate(CgArgs a, int k) {
-  __shared__ double s_tmp[5 * 4], s_out[5];
+// REL: the stopping test is the relative residual and a.ad holds 1 / a_ii
+// (the same rounding as dividing here), so no row costs a division.
+// What bounds it: the bytes (48 n with DX) from 1M rows on, below that the
+// chain launch -> state -> partials -> reduction.  So the partials' loads go
+// out first, then kPupItems pairs per thread, then the wait for the partials:
+// 131x117x97 14.0 us with one pair in flight and the state read before any
+// load, 10.6 us now (100^3 10.1 and 8.1, 160^3 32.4 and 29.6).  Two pairs: three
+// and four gain 0.3 us at 100^3 and lose as much or more at 131x117x97.
+constexpr int kPupItems = 2;
+template <int PREC, bool DX, bool REL>
+__global__ __launch_bounds__(kBlock, 3) void k_pupdate(CgArgs a, int k) {
+  constexpr int NV = DX ? 2 : 4;
+  __shared__ double s_tmp[NV * 4], s_out[NV];
   State* st = a.st;
-  if (st->done) return;
+  const int done = st->done;
   if (k == 0) k = st->kcur;
-  const int stride = gridDim.x * kBlock;
   const int npair = a.n >> 1;
   dbl2* p2 = reinterpret_cast<dbl2*>(a.p);
   dbl2* x2 = reinterpret_cast<dbl2*>(a.x);
   const dbl2* r2 = reinterpret_cast<const dbl2*>(a.r);
   const dbl2* d2 = reinterpret_cast<const dbl2*>(a.ad);
-  // this thread's first pair, loaded before the sweep of the partials so
-  // that the two memory round trips overlap (small systems are bound by
-  // them)
-  const int t0 = blockIdx.x * kBlock + threadIdx.x;
-  const int tp = npair > 0 ? min(t0, npair - 1) : 0;
-  dbl2 rv0 = {0.0, 0.0}, dv0 = {1.0, 1.0}, pv0 = {0.0, 0.0}, xv0 = {0.0, 0.0};
-  if (npair > 0) {
-    rv0 = r2[tp];
-    if (PREC == PREC_JACOBI) dv0 = d2[tp];
-    pv0 = p2[tp];
-    if (DX) xv0 = x2[tp];
+  // rows of the update's partials: with DX only the measure's sum and (z, r)
+  Sweep<NV, 3> sums;
+  int ops[NV];
+#pragma unroll
+  for (int c = 0; c < NV; ++c) {
+    const int row = DX ? (c == 0 ? (REL ? 4 : 0) : 3) : c;
+    sums.row[c] = a.pt.upd + row * a.pt.pstride;
+    ops[c] = DX || c == 0 || c == 3 ? OP_SUM : (c == 1 ? OP_MIN : OP_MAX);
   }
+  sums.issue(a.pt.g_upd);
+  struct Item {
+    dbl2 r, d, p, x;
+  };
+  auto load = [&](Item& w, int t) {
+    w.r = r2[t];
+    if (PREC == PREC_JACOBI) w.d = d2[t];
+    w.p = p2[t];
+    if (DX) w.x = x2[t];
+  };
+  Item first[kPupItems];
+  if (npair > 0) first_items<kPupItems>(npair, first, load);
+  __builtin_amdgcn_sched_barrier(0);
+  sums.finish(a.pt.g_upd, ops, s_tmp, s_out);
+  if (done) return;
   double beta = 0.0;
   if (k > 1) {
-    const int ops[5] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
-    gather<5>(a.pt.upd, a.pt.pstride, a.pt.g_upd, ops, s_tmp, s_out);
-    const double res = measure(st, s_out[0], s_out[1], s_out[2], s_out[4]);
+    const double res = DX ? measure(st, s_out[0], 0.0, 0.0, s_out[0])
+                          : measure(st, s_out[0], s_out[1], s_out[2], 0.0);
     const bool bad = !isfinite(res);
     if (bad || res < st->tol) {
       if (lead()) {
@@ -179,7 +200,7 @@ __global__ __launch_bounds__(kBlock) void k_pupdate(CgArgs a, int k) {
       }
       return;
     }
-    const double rho = s_out[3];
+    const double rho = s_out[NV - 1];
     beta = rho / st->rho[(k - 1) & 1];
     if (lead()) {
       st->rho[k & 1] = rho;
@@ -189,40 +210,34 @@ __global__ __launch_bounds__(kBlock) void k_pupdate(CgArgs a, int k) {
     }
   }
   const double alpha = DX && k > 1 ? st->alpha : 0.0;
-  auto pair = [&](int t, dbl2 rv, dbl2 dv, dbl2 pv, dbl2 xv) {
+  auto inverse = [](double d) { return REL ? d : 1.0 / d; };
+  auto pair = [&](int t, const Item& w) {
     dbl2 z;
     if (PREC == PREC_JACOBI) {
-      z.x = rv.x * (1.0 / dv.x);
-      z.y = rv.y * (1.0 / dv.y);
+      z.x = w.r.x * inverse(w.d.x);
+      z.y = w.r.y * inverse(w.d.y);
     } else {
-      z = rv;
+      z = w.r;
     }
     if (k == 1) {
       p2[t] = z;
     } else {
       if (DX) {
         dbl2 xo;
-        xo.x = xv.x + alpha * pv.x;
-        xo.y = xv.y + alpha * pv.y;
+        xo.x = w.x.x + alpha * w.p.x;
+        xo.y = w.x.y + alpha * w.p.y;
         x2[t] = xo;
       }
       dbl2 o;
-      o.x = z.x + beta * pv.x;
-      o.y = z.y + beta * pv.y;
+      o.x = z.x + beta * w.p.x;
+      o.y = z.y + beta * w.p.y;
       p2[t] = o;
     }
   };
-  if (t0 < npair) pair(t0, rv0, dv0, pv0, xv0);
-  for (int t = t0 + stride; t < npair; t += stride) {
-    const dbl2 rv = r2[t];
-    const dbl2 dv = PREC == PREC_JACOBI ? d2[t] : dbl2{1.0, 1.0};
-    const dbl2 pv = k == 1 ? dbl2{0.0, 0.0} : p2[t];
-    const dbl2 xv = DX && k > 1 ? x2[t] : dbl2{0.0, 0.0};
-    pair(t, rv, dv, pv, xv);
-  }
+  if (npair > 0) stream_items<kPupItems>(npair, first, load, pair);
   if ((a.n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
     const int i = a.n - 1;
-    const double z = PREC == PREC_JACOBI ? a.r[i] * (1.0 / a.ad[i]) : a.r[i];
+    const double z = PREC == PREC_JACOBI ? a.r[i] * inverse(a.ad[i]) : a.r[i];
     if (DX && k > 1) a.x[i] = a.x[i] + alpha * a.p[i];
     a.p[i] = (k == 1) ? z : z + beta * a.p[i];
   }
@@ -251,38 +266,47 @@ __global__ __launch_bounds__(kBlock) void k_spmv_pq(CgArgs a, int k) {
 
 // alpha = rho / (p,q) (Cg.f90:190-198); x += alpha p, r -= alpha q
 // (Cg.f90:204-209); partials of the NRMS sum, the x range, the next (z, r)
-// and ||r||^2 on the new r and x.
-template <int PREC, bool DX>
-__global__ __launch_bounds__(kBlock) void k_update(CgArgs a, int k) {
+// and ||r||^2 on the new r and x.  REL (as in k_pupdate): of these only (z, r)
+// and ||r||^2, and no division; the others are what NRMS measures.  Loads
+// ordered as in k_pupdate: 131x117x97 12.5 us before, 10.2 us now (100^3 10.7 and
+// 8.5, 160^3 23.6 and 20.9).
+template <int PREC, bool DX, bool REL>
+__global__ __launch_bounds__(kBlock, 3) void k_update(CgArgs a, int k) {
+  constexpr int kItems = 2;
   __shared__ double s_tmp[5 * 4], s_out[5];
   State* st = a.st;
-  if (st->done) return;
+  const int done = st->done;
   if (k == 0) k = st->kcur - 1;  // the SpMV of this iteration advanced it
-  const int stride = gridDim.x * kBlock;
   const int npair = a.n >> 1;
   dbl2* x2 = reinterpret_cast<dbl2*>(a.x);
   dbl2* r2 = reinterpret_cast<dbl2*>(a.r);
   const dbl2* p2 = reinterpret_cast<const dbl2*>(a.p);
   const dbl2* q2 = reinterpret_cast<const dbl2*>(a.q);
   const dbl2* d2 = reinterpret_cast<const dbl2*>(a.ad);
-  // this thread's first pair, loaded before the sweep of the (p, q)
-  // partials so that the two memory round trips overlap
-  const int t0 = blockIdx.x * kBlock + threadIdx.x;
-  const int tp = npair > 0 ? min(t0, npair - 1) : 0;
-  dbl2 rv0 = {0.0, 0.0}, qv0 = {0.0, 0.0}, dv0 = {1.0, 1.0}, xv0 = {0.0, 0.0}, pv0 = {0.0, 0.0};
-  if (npair > 0) {
-    rv0 = r2[tp];
-    qv0 = q2[tp];
-    dv0 = d2[tp];
+  constexpr bool kDiag = !REL || PREC == PREC_JACOBI;
+  Sweep<1, 6> sum;
+  sum.row[0] = a.pt.spmv;
+  sum.issue(a.pt.g_spmv);
+  struct Item {
+    dbl2 r, q, d, x, p;
+  };
+  auto load = [&](Item& w, int t) {
+    w.r = r2[t];
+    w.q = q2[t];
+    if (kDiag) w.d = d2[t];
     if (!DX) {
-      xv0 = x2[tp];
-      pv0 = p2[tp];
+      w.x = x2[t];
+      w.p = p2[t];
     }
-  }
+  };
+  Item first[kItems];
+  if (npair > 0) first_items<kItems>(npair, first, load);
+  __builtin_amdgcn_sched_barrier(0);
   {
     const int ops1[1] = {OP_SUM};
-    gather<1>(a.pt.spmv, a.pt.pstride, a.pt.g_spmv, ops1, s_tmp, s_out);
+    sum.finish(a.pt.g_spmv, ops1, s_tmp, s_out);
   }
+  if (done) return;
   const double pq = s_out[0];
   if (pq == 0.0 || !isfinite(pq)) {
     if (lead()) {
@@ -298,68 +322,54 @@ __global__ __launch_bounds__(kBlock) void k_update(CgArgs a, int k) {
     st->fold = 1;
   }
   double v[5] = {0.0, kHuge, -kHuge, 0.0, 0.0};
-  if (DX) {
-    // r -= alpha q and the sums that need no x (x is folded in k_pupdate),
-    // two rows per thread with 16-byte accesses
-    auto sums = [&](double rv, double dv) {
-      const double z = PREC == PREC_JACOBI ? rv * (1.0 / dv) : rv;
-      v[0] = v[0] + (rv * rv) / (dv * dv);
-      v[3] = v[3] + z * rv;
-      v[4] = v[4] + rv * rv;
-    };
-    auto pair = [&](int t, dbl2 rv, dbl2 qv, dbl2 dv) {
-      dbl2 ro;
-      ro.x = rv.x - alpha * qv.x;
-      ro.y = rv.y - alpha * qv.y;
-      r2[t] = ro;
-      sums(ro.x, dv.x);
-      sums(ro.y, dv.y);
-    };
-    if (t0 < npair) pair(t0, rv0, qv0, dv0);
-    for (int t = t0 + stride; t < npair; t += stride) pair(t, r2[t], q2[t], d2[t]);
-    if ((a.n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
-      const int i = a.n - 1;
-      const double rv = a.r[i] - alpha * a.q[i];
-      a.r[i] = rv;
-      sums(rv, a.ad[i]);
-    }
-    const int ops[5] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
-    publish<5>(v, ops, a.pt.upd, a.pt.pstride, s_tmp, s_out);
-    return;
-  }
   auto one = [&](double& xv, double& rv, double pv, double qv, double dv) {
-    xv = xv + alpha * pv;
+    if (!DX) xv = xv + alpha * pv;
     rv = rv - alpha * qv;
-    const double z = PREC == PREC_JACOBI ? rv * (1.0 / dv) : rv;
-    v[0] = v[0] + (rv * rv) / (dv * dv);
-    v[1] = fmin(v[1], xv);
-    v[2] = fmax(v[2], xv);
+    const double z = PREC == PREC_JACOBI ? rv * (REL ? dv : 1.0 / dv) : rv;
+    if (!REL) {
+      v[0] = v[0] + (rv * rv) / (dv * dv);
+      if (!DX) {
+        v[1] = fmin(v[1], xv);
+        v[2] = fmax(v[2], xv);
+      }
+    }
     v[3] = v[3] + z * rv;
     v[4] = v[4] + rv * rv;
   };
-  auto pair = [&](int t, dbl2 xv, dbl2 rv, dbl2 pv, dbl2 qv, dbl2 dv) {
-    double x0 = xv.x, x1 = xv.y, r0 = rv.x, r1 = rv.y;
-    one(x0, r0, pv.x, qv.x, dv.x);
-    one(x1, r1, pv.y, qv.y, dv.y);
+  auto pair = [&](int t, const Item& w) {
+    double x0 = w.x.x, x1 = w.x.y, r0 = w.r.x, r1 = w.r.y;
+    one(x0, r0, w.p.x, w.q.x, w.d.x);
+    one(x1, r1, w.p.y, w.q.y, w.d.y);
     dbl2 xo, ro;
-    xo.x = x0;
-    xo.y = x1;
     ro.x = r0;
     ro.y = r1;
-    x2[t] = xo;
     r2[t] = ro;
+    if (!DX) {
+      xo.x = x0;
+      xo.y = x1;
+      x2[t] = xo;
+    }
   };
-  if (t0 < npair) pair(t0, xv0, rv0, pv0, qv0, dv0);
-  for (int t = t0 + stride; t < npair; t += stride) pair(t, x2[t], r2[t], p2[t], q2[t], d2[t]);
+  if (npair > 0) stream_items<kItems>(npair, first, load, pair);
   if ((a.n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
     const int i = a.n - 1;
-    double xv = a.x[i], rv = a.r[i];
-    one(xv, rv, a.p[i], a.q[i], a.ad[i]);
-    a.x[i] = xv;
+    double xv = DX ? 0.0 : a.x[i], rv = a.r[i];
+    one(xv, rv, DX ? 0.0 : a.p[i], a.q[i], kDiag ? a.ad[i] : 0.0);
+    if (!DX) a.x[i] = xv;
     a.r[i] = rv;
   }
-  const int ops[5] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
-  publish<5>(v, ops, a.pt.upd, a.pt.pstride, s_tmp, s_out);
+  if (REL) {
+    double w[2] = {v[3], v[4]};
+    const int ops[2] = {OP_SUM, OP_SUM}, rows[2] = {3, 4};
+    publish_rows<2>(w, ops, rows, a.pt.upd, a.pt.pstride, s_tmp, s_out);
+  } else if (DX) {
+    double w[2] = {v[0], v[3]};
+    const int ops[2] = {OP_SUM, OP_SUM}, rows[2] = {0, 3};
+    publish_rows<2>(w, ops, rows, a.pt.upd, a.pt.pstride, s_tmp, s_out);
+  } else {
+    const int ops[5] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
+    publish<5>(v, ops, a.pt.upd, a.pt.pstride, s_tmp, s_out);
+  }
 }
 
 // One workgroup: stopping test of iteration k (Cg.f90:214-220) so that the
@@ -591,14 +601,27 @@ hipError_t launch_start(const Launch& L, const CgArgs& a, int rho_slot) {
   return hipGetLastError();
 }
 
+// f(prec, dx, rel) as constants; the relative residual needs no x range, so
+// the p update runs with dx whenever rel holds.
+template <typename F>
+static void update_dispatch(int prec, bool dx, bool rel, F f) {
+  auto go = [&](auto pc) {
+    if (dx && rel) f(pc, std::true_type{}, std::true_type{});
+    else if (dx) f(pc, std::true_type{}, std::false_type{});
+    else if (rel) f(pc, std::false_type{}, std::true_type{});
+    else f(pc, std::false_type{}, std::false_type{});
+  };
+  if (prec == PREC_JACOBI) go(std::integral_constant<int, PREC_JACOBI>{});
+  else go(std::integral_constant<int, PREC_NONE>{});
+}
+
 hipError_t launch_pupdate(const Launch& L, const CgArgs& a, int prec, int k, bool dx) {
-  if (prec == PREC_JACOBI) {
-    if (dx) k_pupdate<PREC_JACOBI, true><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
-    else k_pupdate<PREC_JACOBI, false><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
-  } else {
-    if (dx) k_pupdate<PREC_NONE, true><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
-    else k_pupdate<PREC_NONE, false><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
-  }
+  if (a.rel && !dx) return hipErrorInvalidValue;
+  update_dispatch(prec, dx, a.rel, [&](auto pc, auto dc, auto rc) {
+    constexpr int P = decltype(pc)::value;
+    constexpr bool D = decltype(dc)::value, R = decltype(rc)::value;
+    if constexpr (D || !R) k_pupdate<P, D, R><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
+  });
   return hipGetLastError();
 }
 
@@ -627,13 +650,11 @@ hipError_t launch_spmv_pq(const Launch& L, const CgArgs& a, int k) {
 }
 
 hipError_t launch_update(const Launch& L, const CgArgs& a, int prec, int k, bool dx) {
-  if (prec == PREC_JACOBI) {
-    if (dx) k_update<PREC_JACOBI, true><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
-    else k_update<PREC_JACOBI, false><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
-  } else {
-    if (dx) k_update<PREC_NONE, true><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
-    else k_update<PREC_NONE, false><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
-  }
+  update_dispatch(prec, dx, a.rel, [&](auto pc, auto dc, auto rc) {
+    constexpr int P = decltype(pc)::value;
+    constexpr bool D = decltype(dc)::value, R = decltype(rc)::value;
+    k_update<P, D, R><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
+  });
   return hipGetLastError();
 }
 

@@ -114,6 +114,17 @@ __device__ __forceinline__ void publish(double (&v)[NV], const int (&ops)[NV], d
   if (threadIdx.x < NV) part[threadIdx.x * pstride + blockIdx.x] = s_out[threadIdx.x];
 }
 
+// The same for the rows rows[k] of part.
+template <int NV>
+__device__ __forceinline__ void publish_rows(double (&v)[NV], const int (&ops)[NV],
+                                             const int (&rows)[NV], double* part, int pstride,
+                                             double* s_tmp, double* s_out) {
+  block_reduce<NV>(v, ops, s_tmp, s_out);
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    if (threadIdx.x == k) part[rows[k] * pstride + blockIdx.x] = s_out[k];
+}
+
 // Consumer side: combine the G partials of a previous kernel in a fixed order.
 // Result in s_out[k] for all threads.
 template <int NV>
@@ -127,6 +138,76 @@ __device__ __forceinline__ void gather(const double* __restrict__ part, int pstr
     for (int k = 0; k < NV; ++k) acc[k] = red_apply(ops[k], acc[k], part[k * pstride + g]);
   }
   block_reduce<NV>(acc, ops, s_tmp, s_out);
+}
+
+// The consumer side in two parts, so that a kernel's own loads can be issued
+// in between: issue() starts the loads of this thread's first U partials of
+// each row, finish() combines them (and what lies past them) as gather() does,
+// bit for bit.  Vector loads complete in issue order, so finish() waits for
+// these but not for what was issued after them.
+template <int NV, int U>
+struct Sweep {
+  const double* row[NV];
+  double w[NV][U];
+  __device__ __forceinline__ void issue(int G) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < NV; ++k) w[k][u] = row[k][min((int)threadIdx.x + u * kBlock, G - 1)];
+  }
+  __device__ __forceinline__ void finish(int G, const int (&ops)[NV], double* s_tmp,
+                                         double* s_out) {
+    double acc[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      acc[k] = red_identity(ops[k]);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const double t = red_apply(ops[k], acc[k], w[k][u]);
+        acc[k] = (int)threadIdx.x + u * kBlock < G ? t : acc[k];
+      }
+    }
+    for (int g = threadIdx.x + U * kBlock; g < G; g += kBlock) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) acc[k] = red_apply(ops[k], acc[k], row[k][g]);
+    }
+    block_reduce<NV>(acc, ops, s_tmp, s_out);
+  }
+};
+
+// Grid-stride sweep over `count` items, B of them per thread and step, the
+// next step's loads in flight while a step is processed (two register sets;
+// `a` holds the first step's items already).  load(item, t), process(t, item).
+template <int B, class Item, class Load, class Process>
+__device__ __forceinline__ void stream_items(int count, Item (&a)[B], Load load, Process process) {
+  const int stride = gridDim.x * kBlock, step = B * stride, tid = threadIdx.x;
+  Item b[B];
+  int at = blockIdx.x * kBlock;
+  auto fetch = [&](Item (&w)[B], int from) {
+#pragma unroll
+    for (int u = 0; u < B; ++u) load(w[u], min(from + tid + u * stride, count - 1));
+  };
+  auto run = [&](const Item (&w)[B]) {
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (at + tid + u * stride < count) process(at + tid + u * stride, w[u]);
+  };
+  while (at < count) {
+    if (at + step < count) fetch(b, at + step);
+    run(a);
+    at += step;
+    if (at >= count) break;
+    if (at + step < count) fetch(a, at + step);
+    run(b);
+    at += step;
+  }
+}
+// The first step's loads (count > 0).
+template <int B, class Item, class Load>
+__device__ __forceinline__ void first_items(int count, Item (&a)[B], Load load) {
+  const int stride = gridDim.x * kBlock, t0 = blockIdx.x * kBlock + threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < B; ++u) load(a[u], min(t0 + u * stride, count - 1));
 }
 
 // Compensated (Neumaier) addition: the running sum and the rounding errors
