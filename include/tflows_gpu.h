@@ -41,7 +41,9 @@ extern "C" {
 #define TFG_DEFLATE_OFF 1
 #define TFG_DEFLATE_ON 2
 
-#define TFG_PATH_AUTO 0        /* graph below 2M nonzeros, kernels above       */
+#define TFG_PATH_AUTO 0        /* small FP64 cg in one launch (up to 65536     */
+                               /* rows, rows from few patterns), else graph    */
+                               /* below 2M nonzeros, kernels above             */
 #define TFG_PATH_KERNELS 1     /* one launch per phase, device-side stop flag  */
 #define TFG_PATH_GRAPH 2       /* chunks of iterations replayed as a hipGraph  */
                                /* (FP64 cg/bicg, jacobi/none; batches too)     */

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <utility>
 #include <cmath>
@@ -187,6 +188,14 @@ struct tfg_matrix {
   // graph path: executable chunk of CG iterations and the operands it holds
   hipGraphExec_t cg_graph = nullptr;
   GraphKey cg_key{};
+  // one-launch CG of a small system: slots, the next tag, the plan (state 0 not
+  // asked yet, 1 made, -1 the system does not fit, or a launch gave up), longest
+  // row
+  unsigned long long* small = nullptr;
+  unsigned small_tag = 1;
+  int small_state = 0;
+  tfg::SmallPlan small_plan{};
+  int pat_len = 0;
   // multi-rank hooks
   tfg_allreduce_fn allreduce = nullptr;
   tfg_exchange_fn exchange = nullptr;
@@ -420,6 +429,7 @@ void free_all(tfg_matrix* h) {
                  h->ns32[3], h->ns32[4], h->valt32, h->rt, h->nv[0], h->nv[1], h->nv[2],
                  h->nv[3], h->valt, h->tpos, h->code, h->tab, h->pat, h->poff, h->plen,
                  h->pslot, h->sym, h->sym_flag, h->sorder, h->ucol, h->ucnt, h->lidx,
+                 h->small,
                  h->loc, h->vmax, h->vrange, h->icc_r64, h->z32, h->icc_rows[0],
                  h->icc_rows[1], h->icc_d, h->icc_dinv, h->icc_y, h->icc_z,
                  (void*)h->bx.tiles, h->bx.dg, h->bx.lo[0], h->bx.lo[1],
@@ -566,6 +576,103 @@ int window_setup(tfg_matrix* h) {
     return TFG_OK;
   }
   HIP_TRY(e);
+  return TFG_OK;
+}
+
+// Whether the one-launch CG (tfg_small.hip) takes a solve with these launches:
+// row patterns of at most 8 entries and no more rows than one XCD holds (65536).
+// Up to there the one launch is the faster form (us per iteration against the
+// replayed graph's: 960 rows 2.8 and 14.0, 6120 rows 6.1 and 12.5, 32768 rows
+// 7.5 and 12.3, 64000 rows 9.6 and 13.7); above, one XCD has no room for it.
+bool small_fits(tfg_matrix* h, const tfg::Launch& L) {
+  if (h->small_state < 0 || L.kind != tfg::K_PIPE_PATTERN || L.sym || h->pat_len > 8) return false;
+  if (h->ni != h->nt || (long long)L.grid_vec * tfg::kBlock < h->nt / 2 || h->cu_count % tfg::kXcds)
+    return false;
+  if (h->small_state == 0) {
+    h->small_plan = tfg::small_plan(h->nblk[0], L.grid_spmv, L.grid_vec,
+                                    h->cu_count / tfg::kXcds);
+    const size_t bytes = sizeof(unsigned long long) * tfg::kSmallWords;
+    const bool ok = h->small_plan.workgroups > 0 && hipMalloc(&h->small, bytes) == hipSuccess &&
+                    hipMemsetAsync(h->small, 0, bytes, h->stream) == hipSuccess;
+    h->small_state = ok ? 1 : -1;
+    (void)hipGetLastError();
+  }
+  return h->small_state > 0;
+}
+
+// One launch at a time of several workgroups that wait for each other, per
+// device: two would share the XCD's room and could wait for each other's
+// workgroups.  A solve that finds the lease taken runs the three-kernel form,
+// with the same bits.
+class XcdLease {
+ public:
+  bool take(int device, const tfg::SmallPlan& p) {
+    if (p.workgroups == 1) return true;
+    std::atomic<bool>* slot = &taken_[device % kDevices];
+    if (slot->exchange(true, std::memory_order_acquire)) return false;
+    mine_ = slot;
+    return true;
+  }
+  ~XcdLease() {
+    if (mine_) mine_->store(false, std::memory_order_release);
+  }
+
+ private:
+  static constexpr int kDevices = 64;
+  static std::atomic<bool> taken_[kDevices];
+  std::atomic<bool>* mine_ = nullptr;
+};
+std::atomic<bool> XcdLease::taken_[XcdLease::kDevices];
+
+// Runs the one-launch CG to its end (some thousand iterations per launch).
+// *given_up: the kernel could not hand over in time; the solve has to start
+// again with the three-kernel form.
+int small_solve(tfg_matrix* h, const tfg::CgArgs& a, int prec, int mode, int miter,
+                bool* given_up) {
+  constexpr int kLaunch = 1 << 14;
+  *given_up = false;
+  tfg::SmallArgs q{};
+  q.n = a.n;
+  q.nblk = a.nblk;
+  q.row = a.row;
+  q.blk = a.blk;
+  q.poff = a.poff;
+  q.plen = a.plen;
+  q.pat = a.pat;
+  q.val = a.val;
+  q.x = a.x;
+  q.r = a.r;
+  q.p = a.p;
+  q.q = a.q;
+  q.ad = a.ad;
+  q.st = a.st;
+  q.g_spmv = a.pt.g_spmv;
+  q.g_vec = a.pt.g_vec;
+  q.flag = h->small;
+  q.xcd = q.flag + 16 * 64;
+  q.out = q.xcd + 128;
+  q.pq = q.out + 16 * tfg::kSmallCopies;
+  q.upd = q.pq + 2 * tfg::kBlock;
+  for (int k = 1; k <= miter; k += kLaunch) {
+    if (h->small_tag > 0xf0000000u) {  // the tags start again on cleared slots
+      HIP_TRY(hipMemsetAsync(h->small, 0, sizeof(unsigned long long) * tfg::kSmallWords, h->stream));
+      h->small_tag = 1;
+    }
+    q.kend = std::min(miter, k + kLaunch - 1);
+    q.tag = h->small_tag;
+    h->small_tag += (unsigned)(q.kend - k) + 3u;
+    HIP_TRY(tfg::launch_small_cg(h->stream, q, h->small_plan, prec, mode));
+    State* s = &h->hst[1];
+    HIP_TRY(hipMemcpyAsync(s, h->st, sizeof(State), hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    if (s->refine) {
+      h->small_state = -1;
+      *given_up = true;
+      return TFG_OK;
+    }
+    if (s->done) break;
+    if (k > INT_MAX - kLaunch) break;
+  }
   return TFG_OK;
 }
 
@@ -1773,6 +1880,7 @@ int tfg_matrix_create(int ni, int nt, int nnz, const int* row, const int* col, c
         std::vector<int> poff(tfg::kPatCount * tfg::kPatMax, 0), plen(tfg::kPatCount, 1);
         for (size_t t = 0; t < seqs.size(); ++t) {
           plen[t] = (int)seqs[t].size();
+          h->pat_len = std::max(h->pat_len, plen[t]);
           for (size_t j = 0; j < seqs[t].size(); ++j) poff[t * tfg::kPatMax + j] = seqs[t][j];
         }
         e = hipMalloc(&h->pat, pat.size());
@@ -2368,7 +2476,28 @@ int tfg_solve_native_ex(tfg_matrix* h, const char* solver, int solver_len, const
     // kernels take the iteration number from State::kcur (k = 0), which the
     // SpMV advances: three launches per iteration.  The executable graph is
     // kept per handle for the same operands.
-    const bool graph = method == tfg::NS_NONE && !icc && !timing &&
+    XcdLease lease;
+    const bool small = method == tfg::NS_NONE && !icc && !timing && o.path == TFG_PATH_AUTO &&
+                       small_fits(h, L) && lease.take(h->device, h->small_plan);
+    bool solved = false;
+    if (small) {
+      bool given_up = false;
+      const int mode = o.criterion == TFG_CRIT_RELRES ? 0 : norm ? 1 : 2;
+      const int rs = small_solve(h, a, pr, mode, miter, &given_up);
+      if (rs != TFG_OK) return rs;
+      solved = !given_up;
+      if (given_up) {
+        if (device_ptrs)
+          HIP_TRY(hipMemcpyAsync(h->x, x, sizeof(double) * n, hipMemcpyDeviceToDevice, h->stream));
+        else
+          HIP_TRY(hipMemcpyAsync(h->x, x, sizeof(double) * n, hipMemcpyHostToDevice, h->stream));
+        HIP_TRY(hipMemcpyAsync(h->st, s0, sizeof(State), hipMemcpyHostToDevice, h->stream));
+        HIP_TRY(tfg::launch_diag_sum(L, a));
+        HIP_TRY(tfg::launch_prologue(L, a, pk));
+        HIP_TRY(tfg::launch_start(L, a));
+      }
+    }
+    const bool graph = method == tfg::NS_NONE && !icc && !timing && !solved &&
                        (o.path == TFG_PATH_GRAPH || (o.path == TFG_PATH_AUTO && h->nnz < (1 << 21)));
     auto enqueue_dev_iterations = [&](int count, bool finish) -> int {
       for (int c = 0; c < count; ++c) {
@@ -2402,7 +2531,7 @@ int tfg_solve_native_ex(tfg_matrix* h, const char* solver, int solver_len, const
     }
     int k = 1, slot = 0, prev = -1;
     bool stop = false;
-    while (k <= miter && !stop) {
+    while (k <= miter && !stop && !solved) {
       const int kend = std::min(miter, k + chunk - 1);
       if (graph) {
         if (kend - k + 1 == chunk) {
@@ -2447,7 +2576,7 @@ int tfg_solve_native_ex(tfg_matrix* h, const char* solver, int solver_len, const
       prev = slot;
       slot ^= 1;
     }
-    if (dx) HIP_TRY(tfg::launch_fold_x(L, a));
+    if (dx && !solved) HIP_TRY(tfg::launch_fold_x(L, a));
     HIP_TRY(hipEventRecord(h->ev_t1, h->stream));
     State* sf = &h->hst[3];
     HIP_TRY(hipMemcpyAsync(sf, h->st, sizeof(State), hipMemcpyDeviceToHost, h->stream));

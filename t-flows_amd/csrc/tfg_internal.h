@@ -337,6 +337,38 @@ hipError_t launch_diag_sum(const Launch& L, const CgArgs& a);
 hipError_t launch_prologue(const Launch& L, const CgArgs& a, int prec);
 hipError_t launch_start(const Launch& L, const CgArgs& a, int rho_slot = 6);
 hipError_t launch_pupdate(const Launch& L, const CgArgs& a, int prec, int k, bool dx = false);
+// One-launch CG of a small system (tfg_small.hip).
+constexpr int kSmallCopies = 8;           // of the totals, each on a line of its own
+constexpr int kSmallWords = 16 * 64 + 128 + 16 * kSmallCopies + 10 * kBlock;  // slots in all
+struct SmallArgs {
+  int n, nblk;
+  const int *row, *blk, *poff, *plen;
+  const uint8_t* pat;
+  const double* val;
+  double *x, *r, *p, *q;
+  const double* ad;
+  State* st;
+  int g_spmv, g_vec;         // grids of the three-kernel form
+  unsigned long long* flag;  // [64][16] p handed over, one line per workgroup
+  unsigned long long* xcd;   // [128] each workgroup's XCD
+  unsigned long long* out;   // [kSmallCopies][16] totals: (p, q), measure, (z, r)
+  unsigned long long* pq;    // [kBlock][2] partials of (p, q)
+  unsigned long long* upd;   // [4][kBlock][2] partials of the update's sums
+  unsigned tag;              // the launch's first tag
+  unsigned twice;            // product workgroups (of the first 8) with two blocks
+  int kend;                  // last iteration of the launch
+};
+struct SmallPlan {
+  int workgroups;            // 0: the system does not fit; 1: k_tiny_cg
+  int share;                 // slots per thread group (1 or 2)
+  unsigned twice;            // SmallArgs::twice
+};
+SmallPlan small_plan(int nblk, int g_spmv, int g_vec, int cu_per_xcd);
+// mode: 0 relative residual, 1 NRMS with norm, 2 NRMS over the x range.  Runs
+// iterations State::kcur .. kend; State::refine = 1: given up, nothing of the
+// result is valid.
+hipError_t launch_small_cg(hipStream_t stream, const SmallArgs& a, const SmallPlan& s, int prec,
+                           int mode);
 hipError_t launch_fold_x(const Launch& L, const CgArgs& a);
 hipError_t launch_spmv_pq(const Launch& L, const CgArgs& a, int k);
 // Symmetric engine set-up for one val: sd from val, and *flag = 1 when some
