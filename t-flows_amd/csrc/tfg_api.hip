@@ -182,9 +182,8 @@ struct tfg_matrix {
   double* icc_dinv = nullptr;
   double* icc_y = nullptr;
   double* icc_z = nullptr;
-  bool box = false;               // box grid: tiled DIC sweeps (bx, box_toff)
+  bool box = false;               // box grid: tiled DIC sweeps (bx)
   tfg::BoxIcc bx{};
-  std::vector<int> box_toff;
   // graph path: executable chunk of CG iterations and the operands it holds
   hipGraphExec_t cg_graph = nullptr;
   GraphKey cg_key{};
@@ -432,7 +431,7 @@ void free_all(tfg_matrix* h) {
                  h->small,
                  h->loc, h->vmax, h->vrange, h->icc_r64, h->z32, h->icc_rows[0],
                  h->icc_rows[1], h->icc_d, h->icc_dinv, h->icc_y, h->icc_z,
-                 (void*)h->bx.tiles, h->bx.dg, h->bx.lo[0], h->bx.lo[1],
+                 h->bx.dg, h->bx.lo[0], h->bx.lo[1],
                  h->bx.lo[2], h->bx.up[0], h->bx.up[1], h->bx.up[2]};
   for (void* d : dev)
     if (d) (void)hipFree(d);
@@ -780,7 +779,6 @@ tfg::IccArgs icc_args(const tfg_matrix* h) {
   c.off_b_host = h->icc_off[1].data();
   c.box = h->box ? 1 : 0;
   c.bx = h->bx;
-  c.toff_host = h->box_toff.data();
   return c;
 }
 
@@ -889,20 +887,6 @@ int box_setup(tfg_matrix* h, const int* row0, const int* col0) {
   b.ntx = (b.nx + b.tx - 1) / b.tx;
   b.nty = (b.ny + b.ty - 1) / b.ty;
   b.ntz = (b.nz + b.tz - 1) / b.tz;
-  std::vector<int> tiles;
-  h->box_toff.assign(1, 0);
-  for (int l = 0; l <= b.ntx + b.nty + b.ntz - 3; ++l) {
-    for (int X = 0; X < b.ntx; ++X)
-      for (int Y = 0; Y < b.nty; ++Y) {
-        const int Z = l - X - Y;
-        if (Z >= 0 && Z < b.ntz) tiles.push_back((X * b.nty + Y) * b.ntz + Z);
-      }
-    h->box_toff.push_back((int)tiles.size());
-  }
-  int* dt = nullptr;
-  HIP_TRY(hipMalloc(&dt, sizeof(int) * tiles.size()));
-  b.tiles = dt;
-  HIP_TRY(hipMemcpy(dt, tiles.data(), sizeof(int) * tiles.size(), hipMemcpyHostToDevice));
   h->box = true;
   return TFG_OK;
 }

@@ -86,11 +86,11 @@ __global__ __launch_bounds__(kBlock) void k_icc_bwd(IccArgs c, const double* __r
 // coordinates (u, v, w) = (x, y, z) for the form and the forward sweep and
 // (nx-1-x, ny-1-y, nz-1-z) for the backward sweep, a row reads the finished
 // values at u-1, v-1, w-1, in that order.  The grid is cut into tiles of at
-// most kBoxTX x kBoxTY x kBoxTZ cells; a tile needs the tiles before it along u, v and w, so
-// the tiles of one level X + Y + Z run in one launch, one workgroup each
-// (61 launches per sweep at 200^3 instead of 598 row levels).  A workgroup
-// loads the three finished faces next to its tile and its cells' values
-// into LDS, one thread per cell; one wave then runs the tile's own levels
+// most kBoxTX x kBoxTY x kBoxTZ cells; a tile needs the tiles before it along
+// u, v and w, so the tiles of one level X + Y + Z run in one launch, one
+// workgroup each (61 launches per sweep at 200^3 instead of 598 row levels).
+// A workgroup loads the three finished faces next to its tile and its cells'
+// values, one thread per cell; one wave then runs the tile's own levels
 // lu + lv + lw, a lane per (u, v) pencil, with no barrier between them.
 // Every row does the reference's operations in the reference's order; an
 // entry the row lacks is a zero in the diagonals and takes a zero product
@@ -119,157 +119,180 @@ __global__ __launch_bounds__(kBlock) void k_box_pack(IccArgs c, const double* __
   }
 }
 
+// The tiles of level X + Y + Z = l: X = first + x, Y from lo(X) on.
+struct TileLevel {
+  int l, first, rows, span;  // X values, and the most Y values of one of them
+  __host__ __device__ TileLevel(const BoxIcc& b, int level) : l(level) {
+    first = max0(l - (b.nty - 1) - (b.ntz - 1));
+    rows = (l < b.ntx - 1 ? l : b.ntx - 1) - first + 1;
+    span = b.nty < b.ntz ? b.nty : b.ntz;
+  }
+  __host__ __device__ static int max0(int v) { return v > 0 ? v : 0; }
+  __host__ __device__ int lo(const BoxIcc& b, int X) const { return max0(l - X - (b.ntz - 1)); }
+  __host__ __device__ int hi(const BoxIcc& b, int X) const {
+    return l - X < b.nty - 1 ? l - X : b.nty - 1;
+  }
+};
+
+// v of the lane N below in the same 16 lanes; `other` for the first N lanes
+template <int N>
+__device__ __forceinline__ double row_shift(double other, double v) {
+  const long long o = __double_as_longlong(other), b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp((int)o, (int)b, 0x110 + N, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(b >> 32), 0x110 + N, 0xf, 0xf,
+                                             false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
 // MODE 0 form: d_inv, d from a_ii and the lower entries   Prec_Form.f90:68-78
 // MODE 1 forward: y from r                                Prec_Solve.f90:64-75
 // MODE 2 backward: z from y                               Prec_Solve.f90:77-92
-// The value the neighbours read (d, y, z) is `out`.  One tile per call of
-// the pieces below, by a workgroup of kBoxThreads threads: its cells'
-// values into LDS, the three finished faces next to it, the tile's levels
-// on one wave, the results back to HBM.
+// The value the neighbours read (d, y, z) is `out`.
+//
+// A launch is a chain: its loads, the tile's levels, its stores, and each was
+// cut to what it needs.  All loads leave together, before the stop flag is
+// looked at.  The levels run on one wave, a lane per (u, v) pencil, each lane
+// going up its pencil, and a step is bound by the instructions of that wave:
+// - w - 1 is the lane's own last result, u - 1 and every other v - 1 a shift
+//   inside 16 lanes;
+// - the other v - 1 (across the rows of 16 lanes) is read back from LDS, where
+//   the results go anyway: each row of lanes runs one step behind the row
+//   before it, so the value was stored two steps ago; for v = 0 the same read
+//   fetches the face;
+// - the u face is taken off when the values are staged (its entry is the first
+//   of the row; the entry is then zero);
+// - what a step needs leaves LDS two steps before.
+// 100^3, per launch of a sweep: 8.1 us with three loads in turn and the
+// neighbours handed over in LDS, 5.9 now (an empty launch 1.7, loads and
+// stores 1.5, the steps 2.1).
 template <int MODE>
-struct BoxTile {
-  static constexpr int TX = kBoxTX, TY = kBoxTY, TZ = kBoxTZ;
-  static_assert(TX * TY == 64, "one lane of the level wave per (u, v) pencil");
+__global__ __launch_bounds__(kBoxThreads) void k_box_sweep(IccArgs c, const State* st,
+                                                           const double* __restrict__ in,
+                                                           double* __restrict__ out,
+                                                           TileLevel level) {
+  constexpr int TX = kBoxTX, TY = kBoxTY, TZ = kBoxTZ;
+  static_assert(TX == 8 && TY == 8, "a lane per pencil, the v pencils two to 16 lanes");
   static_assert(TX * TY * TZ == kBoxThreads, "one thread per cell when staging");
-  static_assert(TX * TZ >= TY * TZ && TX * TZ >= TX * TY, "the largest face is the v face");
-  // LDS strides of the tile with its faces and the pencil stride of the
-  // staged cell data, padded so that the lanes of one level fall on
-  // different banks
-  static constexpr int SW = 1, SV = TZ + 2, SU = (TY + 1) * SV + 2, P = TZ + 2;
-  struct Smem {
-    double s[(TX + 1) * SU];
-    double cv[5][TX * TY * P];  // c0, c1, c2, a0 (r or y), d; MODE 0: d_inv in slot 4
-  };
-  int u0, v0, w0;
-  int su, sv, sw, sq, si;
-  bool mine;
-
-  __device__ __forceinline__ BoxTile(const BoxIcc& b, int tile) {
-    const int X = tile / (b.nty * b.ntz), Y = (tile / b.ntz) % b.nty, Z = tile % b.ntz;
-    u0 = X * b.tx;
-    v0 = Y * b.ty;
-    w0 = Z * b.tz;
-    const int tid = threadIdx.x;
-    su = tid / (TY * TZ);
-    sv = (tid / TZ) % TY;
-    sw = tid % TZ;
-    mine = in_tile(b, su, sv, sw);
-    sq = (su * TY + sv) * P + sw;
-    si = mine ? row_of(b, u0 + su, v0 + sv, w0 + sw) : 0;
-  }
-  __device__ __forceinline__ static int row_of(const BoxIcc& b, int u, int v, int w) {
+  // Pencil (u, v) starts at P u + S v + v / 2: the lanes of a step, whose w
+  // differ by u + v + v / 2, fall on different banks.  Reads run past a
+  // pencil's ends by up to kPad, where nothing is used.
+  constexpr int P = TZ + 2, S = 169, kPad = 24, kFace = TZ + 3;
+  constexpr int kCells = 7 * S + 3 + 7 * P + TZ + 2 * kPad, kFaces = 7 * kFace + TZ + 2 * kPad;
+  constexpr int kSink = kCells - 1;
+  __shared__ dbl2 m01[kCells], m2d[kCells];  // scaled c0 and c1, c2 and d
+  __shared__ double m[kCells + kFaces];      // r or y, then the result; the v face
+  __shared__ double mw[64];                  // the w face
+  const BoxIcc& b = c.bx;
+  const int X = level.first + blockIdx.y, Y = level.lo(b, X) + blockIdx.x;
+  if (Y > level.hi(b, X)) return;
+  const int u0 = X * b.tx, v0 = Y * b.ty, w0 = (level.l - X - Y) * b.tz;
+  const int tid = threadIdx.x;
+  auto row_of = [&](int u, int v, int w) {
     const int x = MODE == 2 ? b.nx - 1 - u : u;
     const int y = MODE == 2 ? b.ny - 1 - v : v;
     const int z = MODE == 2 ? b.nz - 1 - w : w;
     return (x * b.ny + y) * b.nz + z;
-  }
-  __device__ __forceinline__ bool in_tile(const BoxIcc& b, int lu, int lv, int lw) const {
+  };
+  auto in_tile = [&](int lu, int lv, int lw) {
     return lu < b.tx && lv < b.ty && lw < b.tz && u0 + lu < b.nx && v0 + lv < b.ny &&
            w0 + lw < b.nz;
-  }
-  // this thread's cell (the tile's natural order, w fastest: the loads
-  // coalesce); inputs written by earlier kernels only
-  __device__ __forceinline__ void stage_cells(const IccArgs& c, const double* __restrict__ in,
-                                              Smem& m) const {
-    const BoxIcc& b = c.bx;
+  };
+  // this thread's cell (w fastest: the loads coalesce) and its value of the
+  // three finished faces next to the tile (zero outside the grid)
+  const int su = tid / (TY * TZ), sv = (tid / TZ) % TY, sw = tid % TZ;
+  const bool mine = in_tile(su, sv, sw);
+  const int si = mine ? row_of(u0 + su, v0 + sv, w0 + sw) : 0;
+  const int sq = kPad + su * P + sv * S + sv / 2 + sw;
+  double c0 = 0.0, c1 = 0.0, c2 = 0.0, a0 = 0.0, d0 = 0.0, f0 = 0.0;
+  if (mine) {
     const double* const* cf = MODE == 2 ? b.up : b.lo;
-    if (!mine) return;
-    m.cv[0][sq] = cf[0][si];
-    m.cv[1][sq] = cf[1][si];
-    m.cv[2][sq] = cf[2][si];
-    if (MODE == 0) {
-      m.cv[3][sq] = b.dg[si];
-    } else if (MODE == 1) {
-      m.cv[3][sq] = in[si];
-      m.cv[4][sq] = c.d[si];
-    } else {
-      m.cv[3][sq] = in[si] * c.dinv[si];
-      m.cv[4][sq] = c.d[si];
-    }
+    c0 = cf[0][si];
+    c1 = cf[1][si];
+    c2 = cf[2][si];
+    a0 = MODE == 0 ? b.dg[si] : in[si];
+    if (MODE != 0) d0 = c.d[si];
+    if (MODE == 2) f0 = c.dinv[si];
   }
-  // finished faces at u0-1, v0-1, w0-1 (zero outside the grid)
-  __device__ __forceinline__ void stage_faces(const BoxIcc& b, const double* out, Smem& m) const {
-    const int tid = threadIdx.x;
-    for (int t = tid; t < b.ty * b.tz; t += kBoxThreads) {
-      const int lv = t / b.tz, lw = t % b.tz, v = v0 + lv, w = w0 + lw;
-      m.s[(lv + 1) * SV + (lw + 1) * SW] =
-          (u0 > 0 && v < b.ny && w < b.nz) ? out[row_of(b, u0 - 1, v, w)] : 0.0;
-    }
-    for (int t = tid; t < b.tx * b.tz; t += kBoxThreads) {
-      const int lu = t / b.tz, lw = t % b.tz, u = u0 + lu, w = w0 + lw;
-      m.s[(lu + 1) * SU + (lw + 1) * SW] =
-          (v0 > 0 && u < b.nx && w < b.nz) ? out[row_of(b, u, v0 - 1, w)] : 0.0;
-    }
-    for (int t = tid; t < b.tx * b.ty; t += kBoxThreads) {
-      const int lu = t / b.ty, lv = t % b.ty, u = u0 + lu, v = v0 + lv;
-      m.s[(lu + 1) * SU + (lv + 1) * SV] =
-          (w0 > 0 && u < b.nx && v < b.ny) ? out[row_of(b, u, v, w0 - 1)] : 0.0;
-    }
+  const int side = tid / (TY * TZ), fa = (tid / TZ) % TY, fb = tid % TZ;  // side 2: (u, v) in a row
+  double face = 0.0;
+  {
+    const int lu = side == 0 ? 0 : side == 1 ? fa : (tid / TY) % TX;
+    const int lv = side == 0 ? fa : side == 1 ? 0 : tid % TY;
+    const int lw = side == 2 ? 0 : fb;
+    const bool edge = side == 0 ? u0 > 0 : side == 1 ? v0 > 0 : side == 2 && tid < 2 * TY * TZ + 64 && w0 > 0;
+    if (edge && in_tile(lu, lv, lw))
+      face = out[row_of(u0 + lu - (side == 0), v0 + lv - (side == 1), w0 + lw - (side == 2))];
   }
-  // one wave runs the levels: at level l the lane of pencil (pu, pv)
-  // computes cell w = l - pu - pv, so a level needs no barrier
-  __device__ __forceinline__ void levels(const BoxIcc& b, double fn, Smem& m) const {
-    if (threadIdx.x >= TX * TY) return;
-    const int pu = threadIdx.x / TY, pv = threadIdx.x % TY;
-    const int nlev = b.tx + b.ty + b.tz - 2;
-    for (int l = 0; l < nlev; ++l) {
-      const int lw = l - pu - pv;
-      if (lw >= 0 && in_tile(b, pu, pv, lw)) {
-        const int q = (pu * TY + pv) * P + lw;
-        const int p = (pu + 1) * SU + (pv + 1) * SV + (lw + 1) * SW;
-        const double n0 = m.s[p - SU], n1 = m.s[p - SV], n2 = m.s[p - SW];
-        double r;
-        if (MODE == 0) {
-          double sum = m.cv[3][q] * fn;
-          double a = m.cv[0][q] * fn;
-          sum = sum - n0 * a * a;
-          a = m.cv[1][q] * fn;
-          sum = sum - n1 * a * a;
-          a = m.cv[2][q] * fn;
-          sum = sum - n2 * a * a;
-          m.cv[4][q] = sum;
-          r = 1.0 / sum;
-        } else {
-          double sum = m.cv[3][q];
-          sum = sum - (m.cv[0][q] * fn) * n0;
-          sum = sum - (m.cv[1][q] * fn) * n1;
-          sum = sum - (m.cv[2][q] * fn) * n2;
-          r = sum * m.cv[4][q];
-        }
-        m.s[p] = r;
-      }
-      // the next level reads cells other lanes of this wave stored: release
-      // this level's LDS stores and acquire the others' at wavefront scope
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-  }
-  __device__ __forceinline__ void store(const IccArgs& c, double* out, const Smem& m) const {
-    if (!mine) return;
-    out[si] = m.s[(su + 1) * SU + (sv + 1) * SV + (sw + 1) * SW];
-    if (MODE == 0) c.dinv[si] = m.cv[4][sq];
-  }
-};
-
-// One launch per tile level: the tiles of level toff[l] .. are
-// blockIdx.x + lo.
-template <int MODE>
-__global__ __launch_bounds__(kBoxThreads) void k_box_sweep(IccArgs c, const State* st,
-                                                           const double* __restrict__ in,
-                                                           double* __restrict__ out, int lo) {
-  using T = BoxTile<MODE>;
-  __shared__ typename T::Smem m;
-  if (MODE != 0 && st && st->done) return;
-  const BoxIcc& b = c.bx;
   const double fn = st ? st->fn : 1.0;
-  const T t(b, b.tiles[lo + blockIdx.x]);
-  t.stage_faces(b, out, m);
-  t.stage_cells(c, in, m);
+  const int done = MODE != 0 && st ? st->done : 0;
+  asm volatile("" : "+v"(c0), "+v"(c1), "+v"(c2), "+v"(a0), "+v"(d0), "+v"(f0), "+v"(face));
+  if (done) return;
+  c0 = c0 * fn;
+  a0 = MODE == 0 ? a0 * fn : MODE == 2 ? a0 * f0 : a0;
+  if (side == 0) {  // su = 0, and `face` is this cell's u - 1
+    a0 = a0 - (MODE == 0 ? face * c0 * c0 : c0 * face);
+    c0 = 0.0;
+  }
+  m01[sq] = dbl2{c0, c1 * fn};
+  m2d[sq] = dbl2{c2 * fn, d0};
+  m[sq] = a0;
+  if (side == 1) m[kCells + kPad + fa * kFace + fb] = face;
+  else if (side == 2 && tid < 2 * TY * TZ + 64) mw[tid - 2 * TY * TZ] = face;  // [u][v]
   __syncthreads();
-  t.levels(b, fn, m);
+  if (tid < 64) {
+    const int pu = tid & 7, pv = ((tid >> 4) << 1) | ((tid >> 3) & 1), late = tid >> 4;
+    const int steps = b.tx + b.ty + b.tz - 2 + (b.ty - 1) / 2;
+    const unsigned wend = in_tile(pu, pv, 0) ? min(b.tz, b.nz - w0) : 0;
+    int lw = -(pu + pv + late);
+    const int at = kPad + pu * P + pv * S + pv / 2;
+    const int across = pv == 0 ? kCells + kPad + pu * kFace : (pv & 1) ? at : at - S - 1;
+    struct Ahead { dbl2 c01, c2d; double a, x; };
+    Ahead v[3];
+    double prev = mw[pu * TY + pv];
+    // the compiler may not move these reads: LDS answers in order
+    auto ahead = [&](int w, Ahead& g) {
+      __builtin_amdgcn_sched_barrier(0);
+      g.x = m[across + w];
+      g.a = m[at + w];
+      g.c01 = m01[at + w];
+      g.c2d = m2d[at + w];
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto step = [&](const Ahead& g, Ahead& next) {
+      const double n0 = row_shift<1>(0.0, prev), n1 = row_shift<8>(g.x, prev), n2 = prev;
+      double sum = g.a, r;
+      if (MODE == 0) {
+        sum = sum - n0 * g.c01.x * g.c01.x;
+        sum = sum - n1 * g.c01.y * g.c01.y;
+        sum = sum - n2 * g.c2d.x * g.c2d.x;
+        r = 1.0 / sum;
+      } else {
+        sum = sum - g.c01.x * n0;
+        sum = sum - g.c01.y * n1;
+        sum = sum - g.c2d.x * n2;
+        r = sum * g.c2d.y;
+      }
+      const bool in = (unsigned)lw < wend;
+      prev = in ? r : prev;
+      const int q = in ? at + lw : kSink;   // a store without a branch around it
+      m[q] = r;
+      if (MODE == 0) m2d[q].y = sum;
+      ahead(lw + 2, next);
+      ++lw;
+    };
+    ahead(lw, v[0]);
+    ahead(lw + 1, v[1]);
+    for (int t = 0; t < steps; t += 3) {  // a step more than needed does nothing
+      step(v[0], v[2]);
+      step(v[1], v[0]);
+      step(v[2], v[1]);
+    }
+  }
   __syncthreads();
-  t.store(c, out, m);
+  if (mine) {
+    out[si] = m[sq];
+    if (MODE == 0) c.dinv[si] = m2d[sq].y;
+  }
 }
 
 hipError_t launch_box_sweep(hipStream_t s, const IccArgs& c, int mode, const State* st,
@@ -285,10 +308,11 @@ hipError_t launch_box_sweep(hipStream_t s, const IccArgs& c, int mode, const Sta
   if (wave != 64) return hipErrorInvalidDeviceFunction;
   const int nl = c.bx.ntx + c.bx.nty + c.bx.ntz - 2;
   for (int l = 0; l < nl; ++l) {
-    const int lo = c.toff_host[l], cnt = c.toff_host[l + 1] - lo;
-    if (mode == 0) k_box_sweep<0><<<cnt, kBoxThreads, 0, s>>>(c, st, in, out, lo);
-    else if (mode == 1) k_box_sweep<1><<<cnt, kBoxThreads, 0, s>>>(c, st, in, out, lo);
-    else k_box_sweep<2><<<cnt, kBoxThreads, 0, s>>>(c, st, in, out, lo);
+    const TileLevel t(c.bx, l);
+    const dim3 grid(t.span, t.rows);
+    if (mode == 0) k_box_sweep<0><<<grid, kBoxThreads, 0, s>>>(c, st, in, out, t);
+    else if (mode == 1) k_box_sweep<1><<<grid, kBoxThreads, 0, s>>>(c, st, in, out, t);
+    else k_box_sweep<2><<<grid, kBoxThreads, 0, s>>>(c, st, in, out, t);
   }
   return hipGetLastError();
 }

@@ -219,19 +219,19 @@ struct IrArgs {
 // every entry a box neighbour (offsets 1, nz, ny*nz).  The values sit in
 // seven zero-padded diagonals; the sweeps run over tiles of at most
 // kBoxTX x kBoxTY x kBoxTZ cells (z is the fastest axis), one workgroup
-// per tile (one thread per cell) and one launch per tile level.  Measured at
-// 200^3 (ICC-CG solve): cubes of side 4, 6, 7, 8, 9, 10, 12, 16 ran 1.89,
-// 1.59, 1.52, 1.34, 1.43, 1.35, 1.57, 1.78 s (smaller tiles take more
-// launches, larger ones more barriers); 8x8x16 1.32, 16x8x8 1.33, 8x8x12
-// 1.36, 8x16x16 1.47 s.  The level loop runs on one wave, a lane per (x, y)
-// pencil, so kBoxTX * kBoxTY is 64.
+// per tile (one thread per cell) and one launch per tile level.  The level loop
+// runs on one wave, a lane per (x, y) pencil, so kBoxTX * kBoxTY is 64.  Other
+// tiles take more launches (ICC-CG at 200^3, with the level loop's neighbours
+// still handed over in LDS: cubes of side 4, 6, 8, 10, 16 1.89, 1.59, 1.34,
+// 1.35, 1.78 s, 8x8x12 1.36, 8x8x16 1.32) or more steps: a launch costs some
+// 3.8 us and a step 0.06, so 8x8x32 (28 launches of 50 steps for 31 of 33 at
+// 100^3) would lose.
 constexpr int kBoxTX = 8, kBoxTY = 8, kBoxTZ = 16;
 constexpr int kBoxThreads = 1024;
 struct BoxIcc {
   int nx, ny, nz;
   int tx, ty, tz;           // tile sides (<= kBoxTX, kBoxTY, kBoxTZ)
   int ntx, nty, ntz;        // tiles per side
-  const int* tiles;         // tile ids X * nty * ntz + Y * ntz + Z, sorted by X + Y + Z
   double* dg;               // a_ii
   double* lo[3];            // a(i, i - off) for off = ny*nz, nz, 1 (zero when absent)
   double* up[3];            // a(i, i + off), same order
@@ -251,7 +251,6 @@ struct IccArgs {
   const int* off_b_host;  // host: nlev_b + 1 level starts in rows_b
   int box;                // 1: the tiled sweeps of a box grid
   BoxIcc bx;
-  const int* toff_host;   // host: tile-level starts in bx.tiles (ntx + nty + ntz - 1 levels)
 };
 
 // Each cell's faces in increasing face order (tfg_faces_create).
