@@ -7,7 +7,7 @@
 // Layout: the systems' CSR arrays are concatenated into one block-diagonal
 // matrix (global 0-based rows and columns).  Row blocks (<= 256 rows,
 // <= kCap nonzeros) never straddle two systems.  Every block-level kernel
-// runs one workgroup per block (the vector kernels: one or two blocks) of
+// runs one workgroup per block (the vector kernels: one wavefront) of
 // the ACTIVE list (blocks of systems not yet stopped) and publishes one
 // partial per block; a one-workgroup-per-system kernel then sweeps that
 // system's partials in a fixed order and writes its scalars.  A system that
@@ -116,7 +116,7 @@ struct BatchArgs {
 struct BatchCfg {
   int chunk;      // iterations per replayed graph (FP64)
   int diag_mask;  // bit c: systems of class c on diagonals use the diagonals
-  int rows;       // rows per thread of the vector kernels (1 or 2 blocks per workgroup)
+  int rows;       // rows per thread of the diagonal products (1 or 2 blocks per workgroup)
 };
 
 
@@ -143,6 +143,16 @@ __device__ __forceinline__ void hold(T... v) {
   (hold1(v), ...);
 }
 
+constexpr int kWaves = kBlock / 64;
+
+// lane `lane`'s v, for all lanes
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
 // Entry of this workgroup in a list of nact entries, dealt to the XCDs in
 // contiguous ranges (workgroup g runs on XCD g % 8); false past the list.
 __device__ __forceinline__ bool list_entry(const int4v* list, int nact, ActEntry& e) {
@@ -158,38 +168,64 @@ __device__ __forceinline__ bool active_entry(const BatchArgs& a, ActEntry& e) {
   return list_entry(a.act, a.nact, e);
 }
 
-// The vector kernels (p update, x/r update) take NE consecutive entries of
-// the XCD's range per workgroup, each thread one row of each (NE = 1 or 2,
-// the batch autotuner's rows per thread).  Returns how many exist (0:
-// none); a missing one repeats the last, so its loads stay in bounds, and
-// stores nothing.
-template <int NE>
-__device__ __forceinline__ int active_entries(const BatchArgs& a, ActEntry (&e)[NE]) {
+// The vector kernels (p update, x/r update) give a block to each wavefront:
+// lane l takes rows l, l + 64, l + 128, l + 192 of it, so four rows' loads per
+// lane are in flight, the entry and the system's state are the wavefront's (in
+// scalar registers), and a block's sums need neither LDS nor a barrier; the
+// four wavefronts of a workgroup share nothing.  All running, 48 systems, 4.7M
+// rows: the FP32 update 19.2 us, 5.0 TB/s (24.2 with a workgroup per block and
+// a row per thread), the FP32 p update 23 us, 4.9 TB/s, either way.
+// Returns false past the XCD's range; e is the wavefront's block.
+__device__ __forceinline__ bool wave_entry(const BatchArgs& a, ActEntry& e) {
   const int g = blockIdx.x, x = g % kXcds, l = g / kXcds;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int first = (int)(((long long)a.nact * x) / kXcds);
   const int end = (int)(((long long)a.nact * (x + 1)) / kXcds);
-  const int j = first + l * NE;
-  if (j >= end) return 0;
-  const int n = min(NE, end - j);
-#pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    const int4v v = a.act[j + min(k, n - 1)];
-    e[k] = ActEntry{v.x, v.y, v.z, v.w};
-  }
-  return n;
+  const int j = first + l * kWaves + wave;
+  if (j >= end) return false;
+  const int4v v = a.act[j];
+  e = ActEntry{v.x, v.y, v.z, v.w};
+  return true;
+}
+// row u of this lane (u = 0 .. kWaves-1), and the same clamped for loads
+__device__ __forceinline__ int wave_row(const ActEntry& e, int u) {
+  return e.r0 + u * 64 + ((int)threadIdx.x & 63);
+}
+__device__ __forceinline__ int load_row(const ActEntry& e, int u) {
+  return min(wave_row(e, u), e.r1 - 1);
 }
 
-// Publishes the block totals of the live entries: slot k * NV + c of the
-// reduction holds value c of entry k.  Each slot has its own butterfly, so
-// an entry's totals are those of a one-entry workgroup, bit for bit.
-template <int NV, int NE>
-__device__ __forceinline__ void entries_publish(const BatchArgs& a, int row0,
-                                                const ActEntry (&e)[NE], const bool (&live)[NE],
-                                                double (&v)[NE * NV], const int (&ops)[NE * NV],
-                                                double* s_tmp, double* s_out) {
-  block_reduce<NE * NV>(v, ops, s_tmp, s_out);
-  const int t = (int)threadIdx.x, k = t / NV, c = t % NV;
-  if (t < NE * NV && live[k]) a.part[(size_t)(row0 + c) * a.nblk + e[k].bl] = s_out[t];
+// Publishes a block's NV totals from the lanes' values w[u].  The same bits as
+// block_reduce: w[u] over the wavefront is what wavefront u of a workgroup
+// adds up there (the butterfly 32, 16, .., 1), and the four follow in order.
+// The first two steps halve the values instead of working on all four: the
+// pairs that are added are the same.
+template <int NV>
+__device__ __forceinline__ void wave_publish(const BatchArgs& a, int row0, int bl,
+                                             const double (&w)[kWaves][NV], const int (&ops)[NV]) {
+  const int lane = (int)threadIdx.x & 63;
+  const bool b5 = lane & 32, b4 = lane & 16;
+  double lo[NV], hi[NV], t[NV];
+#pragma unroll
+  for (int c = 0; c < NV; ++c) {  // lanes below 32 keep w[0] and w[2]
+    lo[c] = red_apply(ops[c], b5 ? w[1][c] : w[0][c], xor_lane<32>(b5 ? w[0][c] : w[1][c]));
+    hi[c] = red_apply(ops[c], b5 ? w[3][c] : w[2][c], xor_lane<32>(b5 ? w[2][c] : w[3][c]));
+  }
+#pragma unroll
+  for (int c = 0; c < NV; ++c)
+    t[c] = red_apply(ops[c], b4 ? hi[c] : lo[c], xor_lane<16>(b4 ? lo[c] : hi[c]));
+  butterfly_step<8>(t, ops);
+  butterfly_step<4>(t, ops);
+  butterfly_step<2>(t, ops);
+  butterfly_step<1>(t, ops);
+#pragma unroll
+  for (int c = 0; c < NV; ++c) {
+    double s = lane_value(t[c], 0);
+    s = red_apply(ops[c], s, lane_value(t[c], 32));
+    s = red_apply(ops[c], s, lane_value(t[c], 16));
+    s = red_apply(ops[c], s, lane_value(t[c], 48));
+    if (lane == 0) a.part[(size_t)(row0 + c) * a.nblk + bl] = s;
+  }
 }
 
 // Sum (min, max) of one system's block partials, fixed order; s_out[k].
@@ -317,31 +353,30 @@ __global__ __launch_bounds__(kBlock) void k_bt_start(BatchArgs a) {
 // p = z + beta p (p = z in a system's first iteration)      Cg.f90:145-171
 // (Row loads and the system's state are in flight together; a thread past
 // the block loads the block's last row and stores nothing.)
-template <int PREC, int NE>
+template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bt_pupdate(BatchArgs a) {
-  ActEntry e[NE];
-  const int n = active_entries<NE>(a, e);
-  if (n == 0) return;
-  int i[NE], done[NE], iter[NE];
-  double r[NE], pv[NE], d[NE], beta[NE];
+  ActEntry e;
+  if (!wave_entry(a, e)) return;
+  const State* st = &a.st[e.s];
+  const int done = st->done, iter = st->iter;
+  const double beta = st->aux1;
+  double r[kWaves], pv[kWaves], d[kWaves];
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    i[k] = min(e[k].r0 + (int)threadIdx.x, e[k].r1 - 1);
-    r[k] = a.r[i[k]];
-    pv[k] = a.p[i[k]];
-    d[k] = PREC == PREC_JACOBI ? a.ad[i[k]] : 1.0;
-    const State* st = &a.st[e[k].s];
-    done[k] = st->done;
-    iter[k] = st->iter;
-    beta[k] = st->aux1;
+  for (int u = 0; u < kWaves; ++u) {
+    const int i = load_row(e, u);
+    r[u] = a.r[i];
+    pv[u] = a.p[i];
+    d[u] = PREC == PREC_JACOBI ? a.ad[i] : 1.0;
   }
 #pragma unroll
-  for (int k = 0; k < NE; ++k) hold(r[k], pv[k], d[k], done[k], iter[k], beta[k]);
+  for (int u = 0; u < kWaves; ++u) hold(r[u], pv[u], d[u]);
+  if (done) return;
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    if (k >= n || done[k] || e[k].r0 + (int)threadIdx.x >= e[k].r1) continue;
-    const double z = PREC == PREC_JACOBI ? r[k] * (1.0 / d[k]) : r[k];
-    a.p[i[k]] = iter[k] == 0 ? z : z + beta[k] * pv[k];
+  for (int u = 0; u < kWaves; ++u) {
+    const int i = wave_row(e, u);
+    if (i >= e.r1) continue;
+    const double z = PREC == PREC_JACOBI ? r[u] * (1.0 / d[u]) : r[u];
+    a.p[i] = iter == 0 ? z : z + beta * pv[u];
   }
 }
 
@@ -519,64 +554,51 @@ __global__ __launch_bounds__(kBlock) void k_bt_alpha(BatchArgs a) {
 }
 
 // x += alpha p, r -= alpha q and the block's stopping sums  Cg.f90:204-218
-template <int PREC, int NE>
+template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bt_update(BatchArgs a) {
   constexpr int NV = 5;
-  __shared__ double s_tmp[NE * NV * 4], s_out[NE * NV];
-  ActEntry e[NE];
-  const int n = active_entries<NE>(a, e);
-  if (n == 0) return;
-  int i[NE], done[NE];
-  bool live[NE];
-  double d[NE], x0[NE], p0[NE], r0[NE], q0[NE], alpha[NE];
+  ActEntry e;
+  if (!wave_entry(a, e)) return;
+  const State* st = &a.st[e.s];
+  const int done = st->done;
+  const double alpha = st->alpha;
+  double d[kWaves], x0[kWaves], p0[kWaves], r0[kWaves], q0[kWaves];
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    i[k] = min(e[k].r0 + (int)threadIdx.x, e[k].r1 - 1);
-    d[k] = a.ad[i[k]];
-    x0[k] = a.x[i[k]];
-    p0[k] = a.p[i[k]];
-    r0[k] = a.r[i[k]];
-    q0[k] = a.q[i[k]];
-    const State* st = &a.st[e[k].s];
-    done[k] = st->done;
-    alpha[k] = st->alpha;
+  for (int u = 0; u < kWaves; ++u) {
+    const int i = load_row(e, u);
+    d[u] = a.ad[i];
+    x0[u] = a.x[i];
+    p0[u] = a.p[i];
+    r0[u] = a.r[i];
+    q0[u] = a.q[i];
   }
-  bool any = false;
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    hold(d[k], x0[k], p0[k], r0[k], q0[k], done[k], alpha[k]);
-    live[k] = k < n && !done[k];
-    any = any || live[k];
-  }
-  if (!any) return;
-  double v[NE * NV];
-  int ops[NE * NV];
+  for (int u = 0; u < kWaves; ++u) hold(d[u], x0[u], p0[u], r0[u], q0[u]);
+  if (done) return;
+  double v[kWaves][NV];
+  const int ops[NV] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    double* w = v + k * NV;
+  for (int u = 0; u < kWaves; ++u) {
+    double* w = v[u];
     w[0] = 0.0;
     w[1] = kHuge;
     w[2] = -kHuge;
     w[3] = 0.0;
     w[4] = 0.0;
-    ops[k * NV + 0] = OP_SUM;
-    ops[k * NV + 1] = OP_MIN;
-    ops[k * NV + 2] = OP_MAX;
-    ops[k * NV + 3] = OP_SUM;
-    ops[k * NV + 4] = OP_SUM;
-    if (!live[k] || e[k].r0 + (int)threadIdx.x >= e[k].r1) continue;
-    const double xv = x0[k] + alpha[k] * p0[k];
-    const double rv = r0[k] - alpha[k] * q0[k];
-    a.x[i[k]] = xv;
-    a.r[i[k]] = rv;
-    const double z = PREC == PREC_JACOBI ? rv * (1.0 / d[k]) : rv;
-    w[0] = (rv * rv) / (d[k] * d[k]);
+    const int i = wave_row(e, u);
+    if (i >= e.r1) continue;
+    const double xv = x0[u] + alpha * p0[u];
+    const double rv = r0[u] - alpha * q0[u];
+    a.x[i] = xv;
+    a.r[i] = rv;
+    const double z = PREC == PREC_JACOBI ? rv * (1.0 / d[u]) : rv;
+    w[0] = (rv * rv) / (d[u] * d[u]);
     w[1] = xv;
     w[2] = xv;
     w[3] = z * rv;
     w[4] = rv * rv;
   }
-  entries_publish<NV, NE>(a, BP_UPD, e, live, v, ops, s_tmp, s_out);
+  wave_publish<NV>(a, BP_UPD, e.bl, v, ops);
 }
 
 // stopping test of iteration k (Cg.f90:214-222), next rho and beta
@@ -862,43 +884,35 @@ __global__ __launch_bounds__(kBlock) void k_bt32_rstart(BatchArgs a) {
 
 // p = z + beta p - mu (a fresh start after a restart: p = z - mu), with the
 // deferred e += alpha_{k-1} p_{k-1} on the p read anyway
-template <int PREC, int NE>
+template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bt32_pupdate(BatchArgs a) {
-  ActEntry e[NE];
-  const int n = active_entries<NE>(a, e);
-  if (n == 0) return;
-  int i[NE], done[NE], iter[NE], kref[NE];
-  float r[NE], pv[NE], ev[NE], d[NE];
-  double mu64[NE], beta64[NE], alpha64[NE];
+  ActEntry e;
+  if (!wave_entry(a, e)) return;
+  const State* st = &a.st[e.s];
+  const int done = st->done, iter = st->iter, kref = st->kref;
+  const float mu = (float)st->aux2, beta = (float)st->aux1, ap = (float)st->alpha;
+  float r[kWaves], pv[kWaves], ev[kWaves], d[kWaves];
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    i[k] = min(e[k].r0 + (int)threadIdx.x, e[k].r1 - 1);
-    r[k] = a.f.r32[i[k]];
-    pv[k] = a.f.p32[i[k]];
-    ev[k] = a.f.e32[i[k]];
-    d[k] = PREC == PREC_JACOBI ? a.f.rd32[i[k]] : 1.0f;
-    const State* st = &a.st[e[k].s];
-    done[k] = st->done;
-    iter[k] = st->iter;
-    kref[k] = st->kref;
-    mu64[k] = st->aux2;
-    beta64[k] = st->aux1;
-    alpha64[k] = st->alpha;
+  for (int u = 0; u < kWaves; ++u) {
+    const int i = load_row(e, u);
+    r[u] = a.f.r32[i];
+    pv[u] = a.f.p32[i];
+    ev[u] = a.f.e32[i];
+    d[u] = PREC == PREC_JACOBI ? a.f.rd32[i] : 1.0f;
   }
 #pragma unroll
-  for (int k = 0; k < NE; ++k)
-    hold(r[k], pv[k], ev[k], d[k], done[k], iter[k], kref[k], mu64[k], beta64[k], alpha64[k]);
+  for (int u = 0; u < kWaves; ++u) hold(r[u], pv[u], ev[u], d[u]);
+  if (done) return;
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    if (k >= n || done[k] || e[k].r0 + (int)threadIdx.x >= e[k].r1) continue;
-    const float mu = (float)mu64[k];
-    const float z = PREC == PREC_JACOBI ? r[k] * d[k] : r[k];
-    if (iter[k] == kref[k]) {  // a fresh start after a restart
-      a.f.p32[i[k]] = z - mu;
+  for (int u = 0; u < kWaves; ++u) {
+    const int i = wave_row(e, u);
+    if (i >= e.r1) continue;
+    const float z = PREC == PREC_JACOBI ? r[u] * d[u] : r[u];
+    if (iter == kref) {  // a fresh start after a restart
+      a.f.p32[i] = z - mu;
     } else {
-      const float beta = (float)beta64[k], ap = (float)alpha64[k];
-      a.f.e32[i[k]] = ev[k] + ap * pv[k];
-      a.f.p32[i[k]] = (z + beta * pv[k]) - mu;
+      a.f.e32[i] = ev[u] + ap * pv[u];
+      a.f.p32[i] = (z + beta * pv[u]) - mu;
     }
   }
 }
@@ -1007,62 +1021,48 @@ __global__ __launch_bounds__(kBlock) void k_bt32_alpha(BatchArgs a) {
 }
 
 // r -= alpha q and the sums (z, r), (s, z), (r, r), NRMS of the FP32 residual
-template <int PREC, int NE>
+template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bt32_update(BatchArgs a) {
   constexpr int NV = 4;
-  __shared__ double s_tmp[NE * NV * 4], s_out[NE * NV];
-  ActEntry e[NE];
-  const int n = active_entries<NE>(a, e);
-  if (n == 0) return;
-  int i[NE], crit[NE], done[NE];
-  bool live[NE];
-  float d[NE], r0[NE], q0[NE], sv[NE];
-  double alpha64[NE], defl_e[NE];
+  ActEntry e;
+  if (!wave_entry(a, e)) return;
+  const State* st = &a.st[e.s];
+  const int done = st->done, crit = st->criterion;
+  const double defl_e = st->defl_e;
+  const float a32 = (float)st->alpha;
+  float d[kWaves], r0[kWaves], q0[kWaves], sv[kWaves];
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    i[k] = min(e[k].r0 + (int)threadIdx.x, e[k].r1 - 1);
-    d[k] = a.f.rd32[i[k]];
-    r0[k] = a.f.r32[i[k]];
-    q0[k] = a.f.q32[i[k]];
-    sv[k] = a.f.s32[i[k]];
-    const State* st = &a.st[e[k].s];
-    done[k] = st->done;
-    crit[k] = st->criterion;
-    alpha64[k] = st->alpha;
-    defl_e[k] = st->defl_e;
+  for (int u = 0; u < kWaves; ++u) {
+    const int i = load_row(e, u);
+    d[u] = a.f.rd32[i];
+    r0[u] = a.f.r32[i];
+    q0[u] = a.f.q32[i];
+    sv[u] = a.f.s32[i];
   }
-  bool any = false;
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    hold(d[k], r0[k], q0[k], sv[k], done[k], crit[k], alpha64[k], defl_e[k]);
-    live[k] = k < n && !done[k];
-    any = any || live[k];
-  }
-  if (!any) return;
-  double v[NE * NV];
-  int ops[NE * NV];
+  for (int u = 0; u < kWaves; ++u) hold(d[u], r0[u], q0[u], sv[u]);
+  if (done) return;
+  double v[kWaves][NV];
+  const int ops[NV] = {OP_SUM, OP_SUM, OP_SUM, OP_SUM};
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    double* w = v + k * NV;
+  for (int u = 0; u < kWaves; ++u) {
+    double* w = v[u];
 #pragma unroll
-    for (int c = 0; c < NV; ++c) {
-      w[c] = 0.0;
-      ops[k * NV + c] = OP_SUM;
-    }
-    if (!live[k] || e[k].r0 + (int)threadIdx.x >= e[k].r1) continue;
-    const float a32 = (float)alpha64[k];
-    const float r = r0[k] - a32 * q0[k];
-    a.f.r32[i[k]] = r;
-    const float z = PREC == PREC_JACOBI ? r * d[k] : r;
+    for (int c = 0; c < NV; ++c) w[c] = 0.0;
+    const int i = wave_row(e, u);
+    if (i >= e.r1) continue;
+    const float r = r0[u] - a32 * q0[u];
+    a.f.r32[i] = r;
+    const float z = PREC == PREC_JACOBI ? r * d[u] : r;
     w[0] = (double)z * (double)r;
-    w[1] = defl_e[k] > 0.0 ? (double)sv[k] * (double)z : 0.0;
+    w[1] = defl_e > 0.0 ? (double)sv[u] * (double)z : 0.0;
     w[2] = (double)r * (double)r;
-    if (crit[k] != TFG_CRIT_RELRES) {
-      const double t = (double)(r * d[k]);
+    if (crit != TFG_CRIT_RELRES) {
+      const double t = (double)(r * d[u]);
       w[3] = t * t;
     }
   }
-  entries_publish<NV, NE>(a, BP_UPD, e, live, v, ops, s_tmp, s_out);
+  wave_publish<NV>(a, BP_UPD, e.bl, v, ops);
 }
 
 // Per system, end of iteration k: beta and mu of the next iteration and, at
@@ -1330,9 +1330,8 @@ int batch_run(tfg_batch* h, int pr, bool fp32, const tfg_options& o, const doubl
   // diagonals, the others), rebuilt from the polled state as systems stop.
   std::vector<int4v> act, act_c;
   std::vector<DiaEntry> act_d;
-  // Rows per thread of the block kernels (the autotuner's choice, or
-  // TFG_BATCH_ROWS): two takes two blocks per workgroup in the vector
-  // kernels and two consecutive blocks of a system per diagonal entry.
+  // Rows per thread of the diagonal products (the autotuner's choice, or
+  // TFG_BATCH_ROWS): two takes two consecutive blocks of a system per entry.
   const char* force_rows = getenv("TFG_BATCH_ROWS");
   const bool two = force_rows && (*force_rows == '1' || *force_rows == '2') ? *force_rows == '2'
                                                                             : cfg.rows == 2;
@@ -1410,17 +1409,15 @@ int batch_run(tfg_batch* h, int pr, bool fp32, const tfg_options& o, const doubl
     else k_bt32_restart<PREC_NONE><<<G, B, 0, S>>>(a);
     k_bt32_rstart<<<a.nsys, B, 0, S>>>(a);
   };
-  // the vector kernels with cfg.rows entries per workgroup, grid Gv
-#define TFG_BT_VEC(KERNEL)                                                            \
-  do {                                                                                \
-    if (two && pr == PREC_JACOBI) KERNEL<PREC_JACOBI, 2><<<Gv, B, 0, S>>>(a);          \
-    else if (two) KERNEL<PREC_NONE, 2><<<Gv, B, 0, S>>>(a);                            \
-    else if (pr == PREC_JACOBI) KERNEL<PREC_JACOBI, 1><<<Gv, B, 0, S>>>(a);            \
-    else KERNEL<PREC_NONE, 1><<<Gv, B, 0, S>>>(a);                                     \
+  // the vector kernels, a block per wavefront
+#define TFG_BT_VEC(KERNEL)                                          \
+  do {                                                              \
+    if (pr == PREC_JACOBI) KERNEL<PREC_JACOBI><<<Gv, B, 0, S>>>(a);  \
+    else KERNEL<PREC_NONE><<<Gv, B, 0, S>>>(a);                      \
   } while (0)
   auto enqueue_chunk = [&](int count) -> hipError_t {
     const int per = (a.nact + kXcds - 1) / kXcds;
-    const int G = kXcds * per, Gv = kXcds * (two ? (per + 1) / 2 : per);
+    const int G = kXcds * per, Gv = kXcds * ((per + kWaves - 1) / kWaves);
     const int Gd = kXcds * ((a.nact_dia + kXcds - 1) / kXcds);
     const int Gc = kXcds * ((a.nact_csr + kXcds - 1) / kXcds);
     if (fp32) {
@@ -1578,7 +1575,7 @@ int batch_tune(tfg_batch* h, int pr, bool fp32, const tfg_options& o, const doub
       if (rc != TFG_OK) return rc;
     }
   }
-  {  // two rows per thread in the vector kernels
+  {  // two rows per thread in the diagonal products
     const BatchCfg base = pick;
     const int rc = probe(BatchCfg{base.chunk, base.diag_mask, 2});
     if (rc != TFG_OK) return rc;
