@@ -43,33 +43,51 @@ __device__ __forceinline__ void stop_at(State* st, int k, double res, int status
 }
 
 // Start of iteration k: for k > 1 the stopping test of iteration k-1 on the
-// update partials (Cg.f90:214-220), then rho_k.  Returns false when the solve
-// stops here.  Every workgroup evaluates the same partials, so all agree.
-__device__ __forceinline__ bool begin_iteration(const CgArgs& a, int k, bool check_omega,
-                                                double* s_tmp, double* s_out, double& rho,
-                                                double& rho_old) {
-  State* st = a.st;
-  if (k > 1) {
-    const int ops[5] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
-    gather<5>(a.pt.upd, a.pt.pstride, a.pt.g_upd, ops, s_tmp, s_out);
-    const double res = measure1(st, s_out[0], s_out[1], s_out[2], s_out[4]);
-    if (!isfinite(res)) { stop_at(st, k - 1, res, TFG_EBREAKDOWN); return false; }
-    if (res < st->tol) { stop_at(st, k - 1, res, TFG_OK); return false; }
-    if (check_omega && st->omega == 0.0) { stop_at(st, k - 1, res, TFG_EBREAKDOWN); return false; }
-    rho = s_out[3];
-    rho_old = st->rho[(k - 1) & 1];
-    if (lead1()) {
-      st->rho[k & 1] = rho;
-      st->res = res;
-      st->iter = k - 1;
-    }
-  } else {
-    rho = st->rho[1];
-    rho_old = 1.0;
+// update partials (Cg.f90:214-220), then rho_k.  Every workgroup evaluates the
+// same partials, so all agree.  issue() starts the partials' loads, so that a
+// kernel's own first loads can follow at once; finish() returns false when the
+// solve stops here.
+struct Begin {
+  Sweep<5, 3> sums;
+  __device__ __forceinline__ void issue(const CgArgs& a, int k) {
+#pragma unroll
+    for (int c = 0; c < 5; ++c) sums.row[c] = a.pt.upd + c * a.pt.pstride;
+    if (k > 1) sums.issue(a.pt.g_upd);
   }
-  if (rho == 0.0) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return false; }
-  return true;
-}
+  __device__ __forceinline__ bool finish(const CgArgs& a, int k, bool check_omega, double* s_tmp,
+                                         double* s_out, double& rho, double& rho_old) {
+    State* st = a.st;
+    if (k > 1) {
+      const int ops[5] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
+      sums.finish(a.pt.g_upd, ops, s_tmp, s_out);
+      const double res = measure1(st, s_out[0], s_out[1], s_out[2], s_out[4]);
+      if (!isfinite(res)) { stop_at(st, k - 1, res, TFG_EBREAKDOWN); return false; }
+      if (res < st->tol) { stop_at(st, k - 1, res, TFG_OK); return false; }
+      if (check_omega && st->omega == 0.0) {
+        stop_at(st, k - 1, res, TFG_EBREAKDOWN);
+        return false;
+      }
+      rho = s_out[3];
+      rho_old = st->rho[(k - 1) & 1];
+      if (lead1()) {
+        st->rho[k & 1] = rho;
+        st->res = res;
+        st->iter = k - 1;
+      }
+    } else {
+      rho = st->rho[1];
+      rho_old = 1.0;
+    }
+    if (rho == 0.0) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return false; }
+    return true;
+  }
+};
+
+// Rows per thread and step of the element-wise kernels below: each issues the
+// partials' loads, looks at the stop flag (a chunk's iterations after the stop
+// should cost an empty launch), issues its first rows' loads, then reduces; the
+// next step's rows are loaded while a step is worked on (stream_items).
+constexpr int kNsItems = 4;
 
 template <int PREC>
 __device__ __forceinline__ double mprec(double v, double d) {
@@ -117,7 +135,9 @@ __global__ __launch_bounds__(kBlock) void k_bicg_pupdate(CgArgs a, NsArgs s, int
   __shared__ double s_tmp[5 * 4], s_out[5];
   if (a.st->done) return;
   double rho, rho_old;
-  if (!begin_iteration(a, k, false, s_tmp, s_out, rho, rho_old)) return;
+  Begin begin;
+  begin.issue(a, k);
+  if (!begin.finish(a, k, false, s_tmp, s_out, rho, rho_old)) return;
   const double beta = rho / rho_old;
   const int stride = gridDim.x * kBlock;
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < a.n; i += stride) {
@@ -188,27 +208,42 @@ __global__ __launch_bounds__(kBlock) void k_bicg_update(CgArgs a, NsArgs s, int 
 // ------------------------------------------------------------------ CGS --
 // s.v1 = u, s.v2 = p^, s.v3 = v^, s.v4 = u^, a.q = q, s.rt = r~0
 template <int PREC>
-__global__ __launch_bounds__(kBlock) void k_cgs_pupdate(CgArgs a, NsArgs s, int k) {
+__global__ __launch_bounds__(kBlock, 3) void k_cgs_pupdate(CgArgs a, NsArgs s, int k) {
   __shared__ double s_tmp[5 * 4], s_out[5];
-  if (a.st->done) return;
+  const int done = a.st->done;
+  Begin begin;
+  begin.issue(a, k);
+  struct Item {
+    double r, q, p, d;
+  };
+  auto load = [&](Item& w, int i) {
+    w.r = a.r[i];
+    if (k > 1) {
+      w.q = a.q[i];
+      w.p = a.p[i];
+    }
+    if (PREC == PREC_JACOBI) w.d = a.ad[i];
+  };
+  if (done) return;
+  Item first[kNsItems];
+  first_items<kNsItems>(a.n, first, load);
+  __builtin_amdgcn_sched_barrier(0);
   double rho, rho_old;
-  if (!begin_iteration(a, k, false, s_tmp, s_out, rho, rho_old)) return;
+  if (!begin.finish(a, k, false, s_tmp, s_out, rho, rho_old)) return;
   const double beta = rho / rho_old;
-  const int stride = gridDim.x * kBlock;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < a.n; i += stride) {
+  stream_items<kNsItems>(a.n, first, load, [&](int i, const Item& w) {
     double u, p;
     if (k == 1) {
-      u = a.r[i];
+      u = w.r;
       p = u;
     } else {
-      const double q = a.q[i];
-      u = a.r[i] + beta * q;
-      p = u + beta * (q + beta * a.p[i]);
+      u = w.r + beta * w.q;
+      p = u + beta * (w.q + beta * w.p);
     }
     s.v1[i] = u;
     a.p[i] = p;
-    s.v2[i] = mprec<PREC>(p, a.ad[i]);
-  }
+    s.v2[i] = mprec<PREC>(p, w.d);
+  });
 }
 
 // v = A w and (r~0, v): the first product of CGS and of BiCGSTAB
@@ -231,25 +266,39 @@ __global__ __launch_bounds__(kBlock) void k_ns_spmv_rv(CgArgs a, const double* w
 }
 
 template <int PREC>
-__global__ __launch_bounds__(kBlock) void k_cgs_mid(CgArgs a, NsArgs s, int k) {
+__global__ __launch_bounds__(kBlock, 3) void k_cgs_mid(CgArgs a, NsArgs s, int k) {
   __shared__ double s_tmp[4], s_out[1];
   State* st = a.st;
-  if (st->done) return;
+  const int done = st->done;
+  Sweep<1, 6> sum;
+  sum.row[0] = a.pt.spmv;
+  sum.issue(a.pt.g_spmv);
+  struct Item {
+    double u, v, d, x;
+  };
+  auto load = [&](Item& w, int i) {
+    w.u = s.v1[i];
+    w.v = s.v3[i];
+    if (PREC == PREC_JACOBI) w.d = a.ad[i];
+    w.x = a.x[i];
+  };
+  if (done) return;
+  Item first[kNsItems];
+  first_items<kNsItems>(a.n, first, load);
+  __builtin_amdgcn_sched_barrier(0);
   const int ops1[1] = {OP_SUM};
-  gather<1>(a.pt.spmv, a.pt.pstride, a.pt.g_spmv, ops1, s_tmp, s_out);
+  sum.finish(a.pt.g_spmv, ops1, s_tmp, s_out);
   const double den = s_out[0];
   if (den == 0.0 || !isfinite(den)) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return; }
   const double alpha = st->rho[k & 1] / den;
   if (lead1()) st->alpha = alpha;
-  const int stride = gridDim.x * kBlock;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < a.n; i += stride) {
-    const double u = s.v1[i];
-    const double q = u - alpha * s.v3[i];
-    const double uh = mprec<PREC>(u + q, a.ad[i]);
+  stream_items<kNsItems>(a.n, first, load, [&](int i, const Item& w) {
+    const double q = w.u - alpha * w.v;
+    const double uh = mprec<PREC>(w.u + q, w.d);
     a.q[i] = q;
     s.v4[i] = uh;
-    a.x[i] = a.x[i] + alpha * uh;
-  }
+    a.x[i] = w.x + alpha * uh;
+  });
 }
 
 // q^ = A u^ and r -= alpha q^, with the stopping and rho sums (this kernel
@@ -280,50 +329,83 @@ __global__ __launch_bounds__(kBlock) void k_cgs_spmv_update(CgArgs a, NsArgs s) 
 
 // ------------------------------------------------------------- BiCGSTAB --
 // a.q = v, s.v1 = s, s.v2 = p^, s.v3 = s^, s.v4 = t, s.rt = r~0
+// 120^3 upwind: 20.3 us with the partials reduced first and a row at a time,
+// 16.7 now; k_bcgs_mid 20.5 and 18.7, k_bcgs_update 28.5 and 25.4 (5 TB/s).
 template <int PREC>
-__global__ __launch_bounds__(kBlock) void k_bcgs_pupdate(CgArgs a, NsArgs s, int k) {
+__global__ __launch_bounds__(kBlock, 3) void k_bcgs_pupdate(CgArgs a, NsArgs s, int k) {
   __shared__ double s_tmp[5 * 4], s_out[5];
-  if (a.st->done) return;
+  const int done = a.st->done;
+  Begin begin;
+  begin.issue(a, k);
+  struct Item {
+    double r, p, q, d;
+  };
+  auto load = [&](Item& w, int i) {
+    w.r = a.r[i];
+    if (k > 1) {
+      w.p = a.p[i];
+      w.q = a.q[i];
+    }
+    if (PREC == PREC_JACOBI) w.d = a.ad[i];
+  };
+  if (done) return;
+  Item first[kNsItems];
+  first_items<kNsItems>(a.n, first, load);
+  __builtin_amdgcn_sched_barrier(0);
   double rho, rho_old;
-  if (!begin_iteration(a, k, true, s_tmp, s_out, rho, rho_old)) return;
+  if (!begin.finish(a, k, true, s_tmp, s_out, rho, rho_old)) return;
   const double omega = a.st->omega;
   const double beta = (rho / rho_old) * (a.st->alpha / omega);
-  const int stride = gridDim.x * kBlock;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < a.n; i += stride) {
-    const double p = k == 1 ? a.r[i] : a.r[i] + beta * (a.p[i] - omega * a.q[i]);
+  stream_items<kNsItems>(a.n, first, load, [&](int i, const Item& w) {
+    const double p = k == 1 ? w.r : w.r + beta * (w.p - omega * w.q);
     a.p[i] = p;
-    s.v2[i] = mprec<PREC>(p, a.ad[i]);
-  }
+    s.v2[i] = mprec<PREC>(p, w.d);
+  });
 }
 
 // alpha; s = r - alpha v, s^ = M^-1 s, and the stopping sums of s with the
 // x + alpha p^ it would give (ext rows 0..3)
 template <int PREC>
-__global__ __launch_bounds__(kBlock) void k_bcgs_mid(CgArgs a, NsArgs s, int k) {
+__global__ __launch_bounds__(kBlock, 3) void k_bcgs_mid(CgArgs a, NsArgs s, int k) {
   __shared__ double s_tmp[4 * 4], s_out[4];
   State* st = a.st;
-  if (st->done) return;
+  const int done = st->done;
+  Sweep<1, 6> sum;
+  sum.row[0] = a.pt.spmv;
+  sum.issue(a.pt.g_spmv);
+  struct Item {
+    double d, r, q, x, ph;
+  };
+  auto load = [&](Item& w, int i) {
+    w.d = a.ad[i];
+    w.r = a.r[i];
+    w.q = a.q[i];
+    w.x = a.x[i];
+    w.ph = s.v2[i];
+  };
+  if (done) return;
+  Item first[kNsItems];
+  first_items<kNsItems>(a.n, first, load);
+  __builtin_amdgcn_sched_barrier(0);
   {
     const int ops1[1] = {OP_SUM};
-    gather<1>(a.pt.spmv, a.pt.pstride, a.pt.g_spmv, ops1, s_tmp, s_out);
+    sum.finish(a.pt.g_spmv, ops1, s_tmp, s_out);
   }
   const double den = s_out[0];
   if (den == 0.0 || !isfinite(den)) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return; }
   const double alpha = st->rho[k & 1] / den;
   if (lead1()) st->alpha = alpha;
   double v[4] = {0.0, kHuge, -kHuge, 0.0};
-  const int stride = gridDim.x * kBlock;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < a.n; i += stride) {
-    const double d = a.ad[i];
-    const double sv = a.r[i] - alpha * a.q[i];
-    const double xh = a.x[i] + alpha * s.v2[i];
+  stream_items<kNsItems>(a.n, first, load, [&](int i, const Item& w) {
+    const double sv = w.r - alpha * w.q;
+    const double xh = w.x + alpha * w.ph;
     s.v1[i] = sv;
-    s.v3[i] = mprec<PREC>(sv, d);
-    v[0] = v[0] + (sv * sv) / (d * d);
+    s.v3[i] = mprec<PREC>(sv, w.d);
+    v[0] = v[0] + (sv * sv) / (w.d * w.d);
     v[1] = fmin(v[1], xh);
     v[2] = fmax(v[2], xh);
     v[3] = v[3] + sv * sv;
-  }
+  });
   const int ops[4] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM};
   publish<4>(v, ops, a.pt.ext, a.pt.pstride, s_tmp, s_out);
 }
@@ -356,18 +438,43 @@ __global__ __launch_bounds__(kBlock) void k_bcgs_spmv_t(CgArgs a, NsArgs s) {
 }
 
 template <int PREC>
-__global__ __launch_bounds__(kBlock) void k_bcgs_update(CgArgs a, NsArgs s, int k) {
+__global__ __launch_bounds__(kBlock, 3) void k_bcgs_update(CgArgs a, NsArgs s, int k) {
   __shared__ double s_tmp[5 * 4], s_out[5];
   State* st = a.st;
-  if (st->done) return;
+  const int done = st->done;
+  Sweep<4, 3> exit_sums;
+  Sweep<2, 6> t_sums;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) exit_sums.row[c] = a.pt.ext + c * (size_t)a.pt.pstride;
+#pragma unroll
+  for (int c = 0; c < 2; ++c) t_sums.row[c] = a.pt.ext + (4 + c) * (size_t)a.pt.pstride;
+  exit_sums.issue(a.pt.g_vec);
+  t_sums.issue(a.pt.g_spmv);
+  struct Item {
+    double d, x, ph, sh, sv, t, rt;
+  };
+  auto load = [&](Item& w, int i) {
+    w.d = a.ad[i];
+    w.x = a.x[i];
+    w.ph = s.v2[i];
+    w.sh = s.v3[i];
+    w.sv = s.v1[i];
+    w.t = s.v4[i];
+    w.rt = s.rt[i];
+  };
+  if (done) return;
+  constexpr int kItems = kNsItems / 2;
+  Item first[kItems];
+  first_items<kItems>(a.n, first, load);
+  __builtin_amdgcn_sched_barrier(0);
   const int ops4[4] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM};
-  gather<4>(a.pt.ext, a.pt.pstride, a.pt.g_vec, ops4, s_tmp, s_out);
+  exit_sums.finish(a.pt.g_vec, ops4, s_tmp, s_out);
   const double res_s = measure1(st, s_out[0], s_out[1], s_out[2], s_out[3]);
   const double alpha = st->alpha;
-  const int stride = gridDim.x * kBlock;
   if (!isfinite(res_s)) { stop_at(st, k, res_s, TFG_EBREAKDOWN); return; }
   if (res_s < st->tol) {
     // early exit on s: x += alpha p^, r = s
+    const int stride = gridDim.x * kBlock;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < a.n; i += stride) {
       a.x[i] = a.x[i] + alpha * s.v2[i];
       a.r[i] = s.v1[i];
@@ -378,26 +485,25 @@ __global__ __launch_bounds__(kBlock) void k_bcgs_update(CgArgs a, NsArgs s, int 
   __syncthreads();
   {
     const int ops2[2] = {OP_SUM, OP_SUM};
-    gather<2>(a.pt.ext + 4 * (size_t)a.pt.pstride, a.pt.pstride, a.pt.g_spmv, ops2, s_tmp, s_out);
+    t_sums.finish(a.pt.g_spmv, ops2, s_tmp, s_out);
   }
   const double ts = s_out[0], tt = s_out[1];
   if (tt == 0.0 || !isfinite(tt)) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return; }
   const double omega = ts / tt;
   if (lead1()) st->omega = omega;
   double v[5] = {0.0, kHuge, -kHuge, 0.0, 0.0};
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < a.n; i += stride) {
-    const double d = a.ad[i];
-    const double xh = a.x[i] + alpha * s.v2[i];
-    const double xv = xh + omega * s.v3[i];
-    const double rv = s.v1[i] - omega * s.v4[i];
+  stream_items<kItems>(a.n, first, load, [&](int i, const Item& w) {
+    const double xh = w.x + alpha * w.ph;
+    const double xv = xh + omega * w.sh;
+    const double rv = w.sv - omega * w.t;
     a.x[i] = xv;
     a.r[i] = rv;
-    v[0] = v[0] + (rv * rv) / (d * d);
+    v[0] = v[0] + (rv * rv) / (w.d * w.d);
     v[1] = fmin(v[1], xv);
     v[2] = fmax(v[2], xv);
-    v[3] = v[3] + s.rt[i] * rv;
+    v[3] = v[3] + w.rt * rv;
     v[4] = v[4] + rv * rv;
-  }
+  });
   const int ops[5] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
   publish<5>(v, ops, a.pt.upd, a.pt.pstride, s_tmp, s_out);
 }
