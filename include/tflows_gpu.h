@@ -175,9 +175,10 @@ int tfg_stream_bench(void* d_dst, const void* d_src, long long bytes, int mode, 
 int tfg_sync_bench(int grid, int reps, double* us_barrier, double* us_boundary);
 
 /* SpMV engines: 0 LDS-staged rows (2040 nonzeros per block), 1 the same
- * with 4088, 2/3/4 sub-wavefront rows with 4/8/16 lanes per row, 5 the
- * 2040 stage with the next block's loads in flight, 6 the same reading a
- * 1-byte code per nonzero instead of its int32 column (col = row + table[code];
+ * with 4088, 2/3/4 sub-wavefront rows with 4/8/16 lanes per row, 5 x
+ * gathered once per distinct column of a 2040-nonzero row block (per entry
+ * where blocks have too many of them), 6 the 2040 stage with the next block's
+ * loads in flight and a 1-byte code per nonzero instead of its int32 column (col = row + table[code];
  * available when the matrix has at most 256 distinct col - row offsets, as
  * every structured grid has), 7 the same reading one byte per ROW: the id of
  * its offset sequence in a table of at most 64 sequences of at most 12
