@@ -42,7 +42,8 @@ enum RedOp { OP_SUM = 0, OP_MIN = 1, OP_MAX = 2 };
 // Scalars of one solve, resident in device memory.  Each field is written by
 // one thread (workgroup 0 of a kernel, or a one-workgroup kernel) and read by
 // later kernels; fields read inside the kernel that writes them are never
-// the ones it writes (rho is double-buffered by iteration parity).
+// the ones it writes (rho is double-buffered by iteration parity), but for
+// done (stop_tag).
 struct State {
   double fn;        // 1 / mean(diag)                     (Cg.f90:62-76)
   double rho[2];    // rho_k = (z, r) in rho[k & 1]       (Cg.f90:150-156)
@@ -55,7 +56,8 @@ struct State {
   double aux2;
   int has_norm;
   int criterion;
-  int done;         // 1: stop, every later phase returns at once
+  int done;         // not 0: stop, every later phase returns at once (1, or
+                    // stop_tag of the launch that stopped)
   int niter;        // iteration at which done was raised
   int status;       // TFG_OK or TFG_EBREAKDOWN
   int iter;         // last iteration whose stopping test was evaluated
@@ -84,6 +86,18 @@ struct State {
   double dsum[4];
   double corr;
 };
+
+// State::done as a kernel of a textbook method raises it, when its other
+// workgroups look at the flag too: the launch (iteration k >= 1, phase) that
+// stopped the solve.  A launch does not heed a stop of its own, so a workgroup
+// or wavefront of it that starts late evaluates the same partial sums, takes
+// the same way out and does its rows' share of an early exit; every other
+// kernel stops at any value but 0.
+enum Phase { PH_DIRECTION = 1, PH_MID = 2, PH_UPDATE = 3 };
+__host__ __device__ constexpr int stop_tag(int k, Phase ph) { return 4 * k + ph; }
+__host__ __device__ constexpr bool stopped(int done, int k, Phase ph) {
+  return done != 0 && done != stop_tag(k, ph);
+}
 
 // Partial sums written by one kernel and swept by the next ones.
 struct Partials {

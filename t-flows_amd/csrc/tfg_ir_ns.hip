@@ -23,13 +23,13 @@ typedef float f32;
 
 __device__ __forceinline__ bool lead2() { return blockIdx.x == 0 && threadIdx.x == 0; }
 
-__device__ __forceinline__ void stop2(State* st, int k, double res, int status) {
+__device__ __forceinline__ void stop2(State* st, int k, double res, int status, int done) {
   if (lead2()) {
     st->res = res;
     st->iter = k;
     st->niter = k;
     st->status = status;
-    st->done = 1;
+    st->done = done;
   }
 }
 
@@ -38,13 +38,14 @@ __device__ __forceinline__ void stop2(State* st, int k, double res, int status) 
 __device__ __forceinline__ bool begin32(const CgArgs& a, State* st, int k, bool check_omega,
                                         double* s_tmp, double* s_out, double& rho,
                                         double& rho_old) {
+  const int tag = stop_tag(k, PH_DIRECTION);
   if (k > 1) {
     const int ops[3] = {OP_SUM, OP_SUM, OP_SUM};
     gather<3>(a.pt.upd, a.pt.pstride, a.pt.g_upd, ops, s_tmp, s_out);
     const double res = sqrt(s_out[2]) / st->bnorm;
-    if (!isfinite(res)) { stop2(st, k - 1, res, TFG_EBREAKDOWN); return false; }
-    if (res < st->tol) { stop2(st, k - 1, res, TFG_OK); return false; }
-    if (check_omega && st->omega == 0.0) { stop2(st, k - 1, res, TFG_EBREAKDOWN); return false; }
+    if (!isfinite(res)) { stop2(st, k - 1, res, TFG_EBREAKDOWN, tag); return false; }
+    if (res < st->tol) { stop2(st, k - 1, res, TFG_OK, tag); return false; }
+    if (check_omega && st->omega == 0.0) { stop2(st, k - 1, res, TFG_EBREAKDOWN, tag); return false; }
     rho = s_out[1];
     rho_old = st->rho[(k - 1) & 1];
     if (lead2()) {
@@ -56,7 +57,7 @@ __device__ __forceinline__ bool begin32(const CgArgs& a, State* st, int k, bool 
     rho = st->rho[1];
     rho_old = 1.0;
   }
-  if (rho == 0.0) { stop2(st, k, st->res, TFG_EBREAKDOWN); return false; }
+  if (rho == 0.0) { stop2(st, k, st->res, TFG_EBREAKDOWN, tag); return false; }
   return true;
 }
 
@@ -112,7 +113,7 @@ template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bicg32_pupdate(CgArgs a, IrArgs f, NsArgs32 s,
                                                            State* in, int k) {
   __shared__ double s_tmp[3 * 4], s_out[3];
-  if (in->done) return;
+  if (stopped(in->done, k, PH_DIRECTION)) return;
   double rho, rho_old;
   if (!begin32(a, in, k, false, s_tmp, s_out, rho, rho_old)) return;
   const f32 beta = (f32)(rho / rho_old);
@@ -155,13 +156,13 @@ template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bicg32_update(CgArgs a, IrArgs f, NsArgs32 s,
                                                           State* in, int k) {
   __shared__ double s_tmp[3 * 4], s_out[3];
-  if (in->done) return;
+  if (stopped(in->done, k, PH_UPDATE)) return;
   {
     const int ops1[1] = {OP_SUM};
     gather<1>(a.pt.spmv, a.pt.pstride, a.pt.g_spmv, ops1, s_tmp, s_out);
   }
   const double den = s_out[0];
-  if (den == 0.0 || !isfinite(den)) { stop2(in, k, in->res, TFG_EBREAKDOWN); return; }
+  if (den == 0.0 || !isfinite(den)) { stop2(in, k, in->res, TFG_EBREAKDOWN, stop_tag(k, PH_UPDATE)); return; }
   const f32 alpha = (f32)(in->rho[k & 1] / den);
   double v[3] = {0.0, 0.0, 0.0};
   const int stride = gridDim.x * kBlock;
@@ -185,7 +186,7 @@ template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_cgs32_pupdate(CgArgs a, IrArgs f, NsArgs32 s,
                                                           State* in, int k) {
   __shared__ double s_tmp[3 * 4], s_out[3];
-  if (in->done) return;
+  if (stopped(in->done, k, PH_DIRECTION)) return;
   double rho, rho_old;
   if (!begin32(a, in, k, false, s_tmp, s_out, rho, rho_old)) return;
   const f32 beta = (f32)(rho / rho_old);
@@ -228,11 +229,11 @@ template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_cgs32_mid(CgArgs a, IrArgs f, NsArgs32 s, State* in,
                                                       int k) {
   __shared__ double s_tmp[4], s_out[1];
-  if (in->done) return;
+  if (stopped(in->done, k, PH_MID)) return;
   const int ops1[1] = {OP_SUM};
   gather<1>(a.pt.spmv, a.pt.pstride, a.pt.g_spmv, ops1, s_tmp, s_out);
   const double den = s_out[0];
-  if (den == 0.0 || !isfinite(den)) { stop2(in, k, in->res, TFG_EBREAKDOWN); return; }
+  if (den == 0.0 || !isfinite(den)) { stop2(in, k, in->res, TFG_EBREAKDOWN, stop_tag(k, PH_MID)); return; }
   const double alpha = in->rho[k & 1] / den;
   if (lead2()) in->alpha = alpha;
   const f32 a32 = (f32)alpha;
@@ -275,7 +276,7 @@ template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bcgs32_pupdate(CgArgs a, IrArgs f, NsArgs32 s,
                                                            State* in, int k) {
   __shared__ double s_tmp[3 * 4], s_out[3];
-  if (in->done) return;
+  if (stopped(in->done, k, PH_DIRECTION)) return;
   double rho, rho_old;
   if (!begin32(a, in, k, true, s_tmp, s_out, rho, rho_old)) return;
   const double omega = in->omega;
@@ -294,13 +295,13 @@ template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bcgs32_mid(CgArgs a, IrArgs f, NsArgs32 s, State* in,
                                                        int k) {
   __shared__ double s_tmp[4], s_out[1];
-  if (in->done) return;
+  if (stopped(in->done, k, PH_MID)) return;
   {
     const int ops1[1] = {OP_SUM};
     gather<1>(a.pt.spmv, a.pt.pstride, a.pt.g_spmv, ops1, s_tmp, s_out);
   }
   const double den = s_out[0];
-  if (den == 0.0 || !isfinite(den)) { stop2(in, k, in->res, TFG_EBREAKDOWN); return; }
+  if (den == 0.0 || !isfinite(den)) { stop2(in, k, in->res, TFG_EBREAKDOWN, stop_tag(k, PH_MID)); return; }
   const double alpha = in->rho[k & 1] / den;
   if (lead2()) in->alpha = alpha;
   const f32 a32 = (f32)alpha;
@@ -346,7 +347,7 @@ template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bcgs32_update(CgArgs a, IrArgs f, NsArgs32 s,
                                                           State* in, int k) {
   __shared__ double s_tmp[3 * 4], s_out[3];
-  if (in->done) return;
+  if (stopped(in->done, k, PH_UPDATE)) return;
   {
     const int ops1[1] = {OP_SUM};
     gather<1>(a.pt.ext + 3 * (size_t)a.pt.pstride, a.pt.pstride, a.pt.g_vec, ops1, s_tmp, s_out);
@@ -354,14 +355,14 @@ __global__ __launch_bounds__(kBlock) void k_bcgs32_update(CgArgs a, IrArgs f, Ns
   const double res_s = sqrt(s_out[0]) / in->bnorm;
   const f32 alpha = (f32)in->alpha;
   const int stride = gridDim.x * kBlock;
-  if (!isfinite(res_s)) { stop2(in, k, res_s, TFG_EBREAKDOWN); return; }
+  if (!isfinite(res_s)) { stop2(in, k, res_s, TFG_EBREAKDOWN, stop_tag(k, PH_UPDATE)); return; }
   if (res_s < in->tol) {
     // early exit on s: e += alpha p^, r = s
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < a.n; i += stride) {
       f.e32[i] = f.e32[i] + alpha * s.v2[i];
       f.r32[i] = s.v1[i];
     }
-    stop2(in, k, res_s, TFG_OK);
+    stop2(in, k, res_s, TFG_OK, stop_tag(k, PH_UPDATE));
     return;
   }
   __syncthreads();
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(kBlock) void k_bcgs32_update(CgArgs a, IrArgs f, Ns
     gather<2>(a.pt.ext + 4 * (size_t)a.pt.pstride, a.pt.pstride, a.pt.g_spmv, ops2, s_tmp, s_out);
   }
   const double ts = s_out[0], tt = s_out[1];
-  if (tt == 0.0 || !isfinite(tt)) { stop2(in, k, in->res, TFG_EBREAKDOWN); return; }
+  if (tt == 0.0 || !isfinite(tt)) { stop2(in, k, in->res, TFG_EBREAKDOWN, stop_tag(k, PH_UPDATE)); return; }
   const double omega = ts / tt;
   if (lead2()) in->omega = omega;
   const f32 om = (f32)omega;

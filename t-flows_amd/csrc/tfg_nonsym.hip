@@ -32,13 +32,13 @@ __device__ __forceinline__ double measure1(const State* st, double nrms, double 
   return sqrt(nrms) / range;
 }
 
-__device__ __forceinline__ void stop_at(State* st, int k, double res, int status) {
+__device__ __forceinline__ void stop_at(State* st, int k, double res, int status, int done) {
   if (lead1()) {
     st->res = res;
     st->iter = k;
     st->niter = k;
     st->status = status;
-    st->done = 1;
+    st->done = done;
   }
 }
 
@@ -57,14 +57,15 @@ struct Begin {
   __device__ __forceinline__ bool finish(const CgArgs& a, int k, bool check_omega, double* s_tmp,
                                          double* s_out, double& rho, double& rho_old) {
     State* st = a.st;
+    const int tag = stop_tag(k, PH_DIRECTION);
     if (k > 1) {
       const int ops[5] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
       sums.finish(a.pt.g_upd, ops, s_tmp, s_out);
       const double res = measure1(st, s_out[0], s_out[1], s_out[2], s_out[4]);
-      if (!isfinite(res)) { stop_at(st, k - 1, res, TFG_EBREAKDOWN); return false; }
-      if (res < st->tol) { stop_at(st, k - 1, res, TFG_OK); return false; }
+      if (!isfinite(res)) { stop_at(st, k - 1, res, TFG_EBREAKDOWN, tag); return false; }
+      if (res < st->tol) { stop_at(st, k - 1, res, TFG_OK, tag); return false; }
       if (check_omega && st->omega == 0.0) {
-        stop_at(st, k - 1, res, TFG_EBREAKDOWN);
+        stop_at(st, k - 1, res, TFG_EBREAKDOWN, tag);
         return false;
       }
       rho = s_out[3];
@@ -78,7 +79,7 @@ struct Begin {
       rho = st->rho[1];
       rho_old = 1.0;
     }
-    if (rho == 0.0) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return false; }
+    if (rho == 0.0) { stop_at(st, k, st->res, TFG_EBREAKDOWN, tag); return false; }
     return true;
   }
 };
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_valt(long long nnz, const int
 template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bicg_pupdate(CgArgs a, NsArgs s, int k) {
   __shared__ double s_tmp[5 * 4], s_out[5];
-  if (a.st->done) return;
+  if (stopped(a.st->done, k, PH_DIRECTION)) return;
   double rho, rho_old;
   Begin begin;
   begin.issue(a, k);
@@ -177,13 +178,13 @@ template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bicg_update(CgArgs a, NsArgs s, int k) {
   __shared__ double s_tmp[5 * 4], s_out[5];
   State* st = a.st;
-  if (st->done) return;
+  if (stopped(st->done, k, PH_UPDATE)) return;
   {
     const int ops1[1] = {OP_SUM};
     gather<1>(a.pt.spmv, a.pt.pstride, a.pt.g_spmv, ops1, s_tmp, s_out);
   }
   const double den = s_out[0];
-  if (den == 0.0 || !isfinite(den)) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return; }
+  if (den == 0.0 || !isfinite(den)) { stop_at(st, k, st->res, TFG_EBREAKDOWN, stop_tag(k, PH_UPDATE)); return; }
   const double alpha = st->rho[k & 1] / den;
   double v[5] = {0.0, kHuge, -kHuge, 0.0, 0.0};
   const int stride = gridDim.x * kBlock;
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_cgs_pupdate(CgArgs a, NsArgs s, i
     }
     if (PREC == PREC_JACOBI) w.d = a.ad[i];
   };
-  if (done) return;
+  if (stopped(done, k, PH_DIRECTION)) return;
   Item first[kNsItems];
   first_items<kNsItems>(a.n, first, load);
   __builtin_amdgcn_sched_barrier(0);
@@ -282,14 +283,14 @@ __global__ __launch_bounds__(kBlock, 3) void k_cgs_mid(CgArgs a, NsArgs s, int k
     if (PREC == PREC_JACOBI) w.d = a.ad[i];
     w.x = a.x[i];
   };
-  if (done) return;
+  if (stopped(done, k, PH_MID)) return;
   Item first[kNsItems];
   first_items<kNsItems>(a.n, first, load);
   __builtin_amdgcn_sched_barrier(0);
   const int ops1[1] = {OP_SUM};
   sum.finish(a.pt.g_spmv, ops1, s_tmp, s_out);
   const double den = s_out[0];
-  if (den == 0.0 || !isfinite(den)) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return; }
+  if (den == 0.0 || !isfinite(den)) { stop_at(st, k, st->res, TFG_EBREAKDOWN, stop_tag(k, PH_MID)); return; }
   const double alpha = st->rho[k & 1] / den;
   if (lead1()) st->alpha = alpha;
   stream_items<kNsItems>(a.n, first, load, [&](int i, const Item& w) {
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_bcgs_pupdate(CgArgs a, NsArgs s, 
     }
     if (PREC == PREC_JACOBI) w.d = a.ad[i];
   };
-  if (done) return;
+  if (stopped(done, k, PH_DIRECTION)) return;
   Item first[kNsItems];
   first_items<kNsItems>(a.n, first, load);
   __builtin_amdgcn_sched_barrier(0);
@@ -383,7 +384,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_bcgs_mid(CgArgs a, NsArgs s, int 
     w.x = a.x[i];
     w.ph = s.v2[i];
   };
-  if (done) return;
+  if (stopped(done, k, PH_MID)) return;
   Item first[kNsItems];
   first_items<kNsItems>(a.n, first, load);
   __builtin_amdgcn_sched_barrier(0);
@@ -392,7 +393,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_bcgs_mid(CgArgs a, NsArgs s, int 
     sum.finish(a.pt.g_spmv, ops1, s_tmp, s_out);
   }
   const double den = s_out[0];
-  if (den == 0.0 || !isfinite(den)) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return; }
+  if (den == 0.0 || !isfinite(den)) { stop_at(st, k, st->res, TFG_EBREAKDOWN, stop_tag(k, PH_MID)); return; }
   const double alpha = st->rho[k & 1] / den;
   if (lead1()) st->alpha = alpha;
   double v[4] = {0.0, kHuge, -kHuge, 0.0};
@@ -462,7 +463,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_bcgs_update(CgArgs a, NsArgs s, i
     w.t = s.v4[i];
     w.rt = s.rt[i];
   };
-  if (done) return;
+  if (stopped(done, k, PH_UPDATE)) return;
   constexpr int kItems = kNsItems / 2;
   Item first[kItems];
   first_items<kItems>(a.n, first, load);
@@ -471,7 +472,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_bcgs_update(CgArgs a, NsArgs s, i
   exit_sums.finish(a.pt.g_vec, ops4, s_tmp, s_out);
   const double res_s = measure1(st, s_out[0], s_out[1], s_out[2], s_out[3]);
   const double alpha = st->alpha;
-  if (!isfinite(res_s)) { stop_at(st, k, res_s, TFG_EBREAKDOWN); return; }
+  if (!isfinite(res_s)) { stop_at(st, k, res_s, TFG_EBREAKDOWN, stop_tag(k, PH_UPDATE)); return; }
   if (res_s < st->tol) {
     // early exit on s: x += alpha p^, r = s
     const int stride = gridDim.x * kBlock;
@@ -479,7 +480,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_bcgs_update(CgArgs a, NsArgs s, i
       a.x[i] = a.x[i] + alpha * s.v2[i];
       a.r[i] = s.v1[i];
     }
-    stop_at(st, k, res_s, TFG_OK);
+    stop_at(st, k, res_s, TFG_OK, stop_tag(k, PH_UPDATE));
     return;
   }
   __syncthreads();
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_bcgs_update(CgArgs a, NsArgs s, i
     t_sums.finish(a.pt.g_spmv, ops2, s_tmp, s_out);
   }
   const double ts = s_out[0], tt = s_out[1];
-  if (tt == 0.0 || !isfinite(tt)) { stop_at(st, k, st->res, TFG_EBREAKDOWN); return; }
+  if (tt == 0.0 || !isfinite(tt)) { stop_at(st, k, st->res, TFG_EBREAKDOWN, stop_tag(k, PH_UPDATE)); return; }
   const double omega = ts / tt;
   if (lead1()) st->omega = omega;
   double v[5] = {0.0, kHuge, -kHuge, 0.0, 0.0};
