@@ -7,9 +7,9 @@
 // Layout: the systems' CSR arrays are concatenated into one block-diagonal
 // matrix (global 0-based rows and columns).  Row blocks (<= 256 rows,
 // <= kCap nonzeros) never straddle two systems.  Every block-level kernel
-// runs one workgroup per block (the vector kernels: one wavefront) of
-// the ACTIVE list (blocks of systems not yet stopped) and publishes one
-// partial per block; a one-workgroup-per-system kernel then sweeps that
+// runs one workgroup per block (the vector kernels: one or two blocks, the FP32
+// update of many blocks one wavefront per block) of the ACTIVE list (blocks of
+// systems not yet stopped) and publishes one partial per block; a one-workgroup-per-system kernel then sweeps that
 // system's partials in a fixed order and writes its scalars.  A system that
 // stops is masked at once (its workgroups return) and removed from the
 // active list at the next compaction, so late iterations only launch the
@@ -116,7 +116,8 @@ struct BatchArgs {
 struct BatchCfg {
   int chunk;      // iterations per replayed graph (FP64)
   int diag_mask;  // bit c: systems of class c on diagonals use the diagonals
-  int rows;       // rows per thread of the diagonal products (1 or 2 blocks per workgroup)
+  int rows;       // rows per thread of the diagonal products, and of the vector
+                  // kernels while many blocks run (1 or 2 blocks per workgroup)
 };
 
 
@@ -168,13 +169,56 @@ __device__ __forceinline__ bool active_entry(const BatchArgs& a, ActEntry& e) {
   return list_entry(a.act, a.nact, e);
 }
 
-// The vector kernels (p update, x/r update) give a block to each wavefront:
-// lane l takes rows l, l + 64, l + 128, l + 192 of it, so four rows' loads per
-// lane are in flight, the entry and the system's state are the wavefront's (in
-// scalar registers), and a block's sums need neither LDS nor a barrier; the
-// four wavefronts of a workgroup share nothing.  All running, 48 systems, 4.7M
-// rows: the FP32 update 19.2 us, 5.0 TB/s (24.2 with a workgroup per block and
-// a row per thread), the FP32 p update 23 us, 4.9 TB/s, either way.
+// The vector kernels (p update, x/r update) take NE consecutive entries of
+// the XCD's range per workgroup, each thread one row of each: two where the
+// batch autotuner chose two rows per thread and kManyBlocks blocks are active,
+// else one (16 systems of sides 20 to 44, FP32, which fall below that: 14.0 ms
+// with two to the end, 11.0 with this rule).  Returns how many exist (0:
+// none); a missing one repeats the last, so its loads stay in bounds, and
+// stores nothing.
+constexpr int kManyBlocks = 2048;
+template <int NE>
+__device__ __forceinline__ int active_entries(const BatchArgs& a, ActEntry (&e)[NE]) {
+  const int g = blockIdx.x, x = g % kXcds, l = g / kXcds;
+  const int first = (int)(((long long)a.nact * x) / kXcds);
+  const int end = (int)(((long long)a.nact * (x + 1)) / kXcds);
+  const int j = first + l * NE;
+  if (j >= end) return 0;
+  const int n = min(NE, end - j);
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int4v v = a.act[j + min(k, n - 1)];
+    e[k] = ActEntry{v.x, v.y, v.z, v.w};
+  }
+  return n;
+}
+
+// Publishes the block totals of the live entries: slot k * NV + c of the
+// reduction holds value c of entry k.  Each slot has its own butterfly, so
+// an entry's totals are those of a one-entry workgroup, bit for bit.
+template <int NV, int NE>
+__device__ __forceinline__ void entries_publish(const BatchArgs& a, int row0,
+                                                const ActEntry (&e)[NE], const bool (&live)[NE],
+                                                double (&v)[NE * NV], const int (&ops)[NE * NV],
+                                                double* s_tmp, double* s_out) {
+  block_reduce<NE * NV>(v, ops, s_tmp, s_out);
+  const int t = (int)threadIdx.x, k = t / NV, c = t % NV;
+  if (t < NE * NV && live[k]) a.part[(size_t)(row0 + c) * a.nblk + e[k].bl] = s_out[t];
+}
+
+// The FP32 update of many active blocks gives a block to each wavefront: lane l
+// takes rows l, l + 64, l + 128, l + 192 of it, so four rows' loads per lane are
+// in flight, the entry and the system's state are the wavefront's (in scalar
+// registers), and a block's sums need neither LDS nor a barrier; the four
+// wavefronts of a workgroup share nothing.  48 systems, 4.7M rows, all running:
+// 24.2 us with a workgroup per block and a row per thread, 19.2 us with this
+// form, 5.0 TB/s.  It runs from kManyBlocks active blocks on; below, too few
+// workgroups are left for the chip.  us per iteration with a workgroup and a
+// wavefront per block: 256 blocks 15.3 and 16.1, 512 17.0 and 17.6, 1024 18.3
+// and 18.5, 2048 22.0 and 21.5, 4096 43.0 and 41.3, 20736 86.8 and 78.6, 125184
+// 512 and 494.  The other vector kernels keep their workgroups: the FP64 update
+// gains nothing (20736 blocks 149.2 and 148.4, 256 blocks 15.1 and 16.7), nor
+// does a p update, which has no sums (FP32, 125184 blocks 494 and 498).
 // Returns false past the XCD's range; e is the wavefront's block.
 __device__ __forceinline__ bool wave_entry(const BatchArgs& a, ActEntry& e) {
   const int g = blockIdx.x, x = g % kXcds, l = g / kXcds;
@@ -353,30 +397,31 @@ __global__ __launch_bounds__(kBlock) void k_bt_start(BatchArgs a) {
 // p = z + beta p (p = z in a system's first iteration)      Cg.f90:145-171
 // (Row loads and the system's state are in flight together; a thread past
 // the block loads the block's last row and stores nothing.)
-template <int PREC>
+template <int PREC, int NE>
 __global__ __launch_bounds__(kBlock) void k_bt_pupdate(BatchArgs a) {
-  ActEntry e;
-  if (!wave_entry(a, e)) return;
-  const State* st = &a.st[e.s];
-  const int done = st->done, iter = st->iter;
-  const double beta = st->aux1;
-  double r[kWaves], pv[kWaves], d[kWaves];
+  ActEntry e[NE];
+  const int n = active_entries<NE>(a, e);
+  if (n == 0) return;
+  int i[NE], done[NE], iter[NE];
+  double r[NE], pv[NE], d[NE], beta[NE];
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) {
-    const int i = load_row(e, u);
-    r[u] = a.r[i];
-    pv[u] = a.p[i];
-    d[u] = PREC == PREC_JACOBI ? a.ad[i] : 1.0;
+  for (int k = 0; k < NE; ++k) {
+    i[k] = min(e[k].r0 + (int)threadIdx.x, e[k].r1 - 1);
+    r[k] = a.r[i[k]];
+    pv[k] = a.p[i[k]];
+    d[k] = PREC == PREC_JACOBI ? a.ad[i[k]] : 1.0;
+    const State* st = &a.st[e[k].s];
+    done[k] = st->done;
+    iter[k] = st->iter;
+    beta[k] = st->aux1;
   }
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) hold(r[u], pv[u], d[u]);
-  if (done) return;
+  for (int k = 0; k < NE; ++k) hold(r[k], pv[k], d[k], done[k], iter[k], beta[k]);
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) {
-    const int i = wave_row(e, u);
-    if (i >= e.r1) continue;
-    const double z = PREC == PREC_JACOBI ? r[u] * (1.0 / d[u]) : r[u];
-    a.p[i] = iter == 0 ? z : z + beta * pv[u];
+  for (int k = 0; k < NE; ++k) {
+    if (k >= n || done[k] || e[k].r0 + (int)threadIdx.x >= e[k].r1) continue;
+    const double z = PREC == PREC_JACOBI ? r[k] * (1.0 / d[k]) : r[k];
+    a.p[i[k]] = iter[k] == 0 ? z : z + beta[k] * pv[k];
   }
 }
 
@@ -554,51 +599,64 @@ __global__ __launch_bounds__(kBlock) void k_bt_alpha(BatchArgs a) {
 }
 
 // x += alpha p, r -= alpha q and the block's stopping sums  Cg.f90:204-218
-template <int PREC>
+template <int PREC, int NE>
 __global__ __launch_bounds__(kBlock) void k_bt_update(BatchArgs a) {
   constexpr int NV = 5;
-  ActEntry e;
-  if (!wave_entry(a, e)) return;
-  const State* st = &a.st[e.s];
-  const int done = st->done;
-  const double alpha = st->alpha;
-  double d[kWaves], x0[kWaves], p0[kWaves], r0[kWaves], q0[kWaves];
+  __shared__ double s_tmp[NE * NV * 4], s_out[NE * NV];
+  ActEntry e[NE];
+  const int n = active_entries<NE>(a, e);
+  if (n == 0) return;
+  int i[NE], done[NE];
+  bool live[NE];
+  double d[NE], x0[NE], p0[NE], r0[NE], q0[NE], alpha[NE];
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) {
-    const int i = load_row(e, u);
-    d[u] = a.ad[i];
-    x0[u] = a.x[i];
-    p0[u] = a.p[i];
-    r0[u] = a.r[i];
-    q0[u] = a.q[i];
+  for (int k = 0; k < NE; ++k) {
+    i[k] = min(e[k].r0 + (int)threadIdx.x, e[k].r1 - 1);
+    d[k] = a.ad[i[k]];
+    x0[k] = a.x[i[k]];
+    p0[k] = a.p[i[k]];
+    r0[k] = a.r[i[k]];
+    q0[k] = a.q[i[k]];
+    const State* st = &a.st[e[k].s];
+    done[k] = st->done;
+    alpha[k] = st->alpha;
   }
+  bool any = false;
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) hold(d[u], x0[u], p0[u], r0[u], q0[u]);
-  if (done) return;
-  double v[kWaves][NV];
-  const int ops[NV] = {OP_SUM, OP_MIN, OP_MAX, OP_SUM, OP_SUM};
+  for (int k = 0; k < NE; ++k) {
+    hold(d[k], x0[k], p0[k], r0[k], q0[k], done[k], alpha[k]);
+    live[k] = k < n && !done[k];
+    any = any || live[k];
+  }
+  if (!any) return;
+  double v[NE * NV];
+  int ops[NE * NV];
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) {
-    double* w = v[u];
+  for (int k = 0; k < NE; ++k) {
+    double* w = v + k * NV;
     w[0] = 0.0;
     w[1] = kHuge;
     w[2] = -kHuge;
     w[3] = 0.0;
     w[4] = 0.0;
-    const int i = wave_row(e, u);
-    if (i >= e.r1) continue;
-    const double xv = x0[u] + alpha * p0[u];
-    const double rv = r0[u] - alpha * q0[u];
-    a.x[i] = xv;
-    a.r[i] = rv;
-    const double z = PREC == PREC_JACOBI ? rv * (1.0 / d[u]) : rv;
-    w[0] = (rv * rv) / (d[u] * d[u]);
+    ops[k * NV + 0] = OP_SUM;
+    ops[k * NV + 1] = OP_MIN;
+    ops[k * NV + 2] = OP_MAX;
+    ops[k * NV + 3] = OP_SUM;
+    ops[k * NV + 4] = OP_SUM;
+    if (!live[k] || e[k].r0 + (int)threadIdx.x >= e[k].r1) continue;
+    const double xv = x0[k] + alpha[k] * p0[k];
+    const double rv = r0[k] - alpha[k] * q0[k];
+    a.x[i[k]] = xv;
+    a.r[i[k]] = rv;
+    const double z = PREC == PREC_JACOBI ? rv * (1.0 / d[k]) : rv;
+    w[0] = (rv * rv) / (d[k] * d[k]);
     w[1] = xv;
     w[2] = xv;
     w[3] = z * rv;
     w[4] = rv * rv;
   }
-  wave_publish<NV>(a, BP_UPD, e.bl, v, ops);
+  entries_publish<NV, NE>(a, BP_UPD, e, live, v, ops, s_tmp, s_out);
 }
 
 // stopping test of iteration k (Cg.f90:214-222), next rho and beta
@@ -884,35 +942,43 @@ __global__ __launch_bounds__(kBlock) void k_bt32_rstart(BatchArgs a) {
 
 // p = z + beta p - mu (a fresh start after a restart: p = z - mu), with the
 // deferred e += alpha_{k-1} p_{k-1} on the p read anyway
-template <int PREC>
+template <int PREC, int NE>
 __global__ __launch_bounds__(kBlock) void k_bt32_pupdate(BatchArgs a) {
-  ActEntry e;
-  if (!wave_entry(a, e)) return;
-  const State* st = &a.st[e.s];
-  const int done = st->done, iter = st->iter, kref = st->kref;
-  const float mu = (float)st->aux2, beta = (float)st->aux1, ap = (float)st->alpha;
-  float r[kWaves], pv[kWaves], ev[kWaves], d[kWaves];
+  ActEntry e[NE];
+  const int n = active_entries<NE>(a, e);
+  if (n == 0) return;
+  int i[NE], done[NE], iter[NE], kref[NE];
+  float r[NE], pv[NE], ev[NE], d[NE];
+  double mu64[NE], beta64[NE], alpha64[NE];
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) {
-    const int i = load_row(e, u);
-    r[u] = a.f.r32[i];
-    pv[u] = a.f.p32[i];
-    ev[u] = a.f.e32[i];
-    d[u] = PREC == PREC_JACOBI ? a.f.rd32[i] : 1.0f;
+  for (int k = 0; k < NE; ++k) {
+    i[k] = min(e[k].r0 + (int)threadIdx.x, e[k].r1 - 1);
+    r[k] = a.f.r32[i[k]];
+    pv[k] = a.f.p32[i[k]];
+    ev[k] = a.f.e32[i[k]];
+    d[k] = PREC == PREC_JACOBI ? a.f.rd32[i[k]] : 1.0f;
+    const State* st = &a.st[e[k].s];
+    done[k] = st->done;
+    iter[k] = st->iter;
+    kref[k] = st->kref;
+    mu64[k] = st->aux2;
+    beta64[k] = st->aux1;
+    alpha64[k] = st->alpha;
   }
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) hold(r[u], pv[u], ev[u], d[u]);
-  if (done) return;
+  for (int k = 0; k < NE; ++k)
+    hold(r[k], pv[k], ev[k], d[k], done[k], iter[k], kref[k], mu64[k], beta64[k], alpha64[k]);
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) {
-    const int i = wave_row(e, u);
-    if (i >= e.r1) continue;
-    const float z = PREC == PREC_JACOBI ? r[u] * d[u] : r[u];
-    if (iter == kref) {  // a fresh start after a restart
-      a.f.p32[i] = z - mu;
+  for (int k = 0; k < NE; ++k) {
+    if (k >= n || done[k] || e[k].r0 + (int)threadIdx.x >= e[k].r1) continue;
+    const float mu = (float)mu64[k];
+    const float z = PREC == PREC_JACOBI ? r[k] * d[k] : r[k];
+    if (iter[k] == kref[k]) {  // a fresh start after a restart
+      a.f.p32[i[k]] = z - mu;
     } else {
-      a.f.e32[i] = ev[u] + ap * pv[u];
-      a.f.p32[i] = (z + beta * pv[u]) - mu;
+      const float beta = (float)beta64[k], ap = (float)alpha64[k];
+      a.f.e32[i[k]] = ev[k] + ap * pv[k];
+      a.f.p32[i[k]] = (z + beta * pv[k]) - mu;
     }
   }
 }
@@ -1023,6 +1089,38 @@ __global__ __launch_bounds__(kBlock) void k_bt32_alpha(BatchArgs a) {
 // r -= alpha q and the sums (z, r), (s, z), (r, r), NRMS of the FP32 residual
 template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_bt32_update(BatchArgs a) {
+  constexpr int NV = 4;
+  __shared__ double s_tmp[NV * 4], s_out[NV];
+  ActEntry e[1];
+  if (active_entries<1>(a, e) == 0) return;
+  const int i = min(e[0].r0 + (int)threadIdx.x, e[0].r1 - 1);
+  const float d = a.f.rd32[i], r0 = a.f.r32[i], q0 = a.f.q32[i], sv = a.f.s32[i];
+  const State* st = &a.st[e[0].s];
+  const int done = st->done, crit = st->criterion;
+  const double alpha64 = st->alpha, defl_e = st->defl_e;
+  hold(d, r0, q0, sv, done, crit, alpha64, defl_e);
+  if (done) return;
+  double w[NV] = {0.0, 0.0, 0.0, 0.0};
+  if (e[0].r0 + (int)threadIdx.x < e[0].r1) {
+    const float r = r0 - (float)alpha64 * q0;
+    a.f.r32[i] = r;
+    const float z = PREC == PREC_JACOBI ? r * d : r;
+    w[0] = (double)z * (double)r;
+    w[1] = defl_e > 0.0 ? (double)sv * (double)z : 0.0;
+    w[2] = (double)r * (double)r;
+    if (crit != TFG_CRIT_RELRES) {
+      const double t = (double)(r * d);
+      w[3] = t * t;
+    }
+  }
+  const int ops[NV] = {OP_SUM, OP_SUM, OP_SUM, OP_SUM};
+  const bool live[1] = {true};
+  entries_publish<NV, 1>(a, BP_UPD, e, live, w, ops, s_tmp, s_out);
+}
+
+// The same with a block per wavefront, the same bits.
+template <int PREC>
+__global__ __launch_bounds__(kBlock) void k_bt32_update_waves(BatchArgs a) {
   constexpr int NV = 4;
   ActEntry e;
   if (!wave_entry(a, e)) return;
@@ -1330,8 +1428,9 @@ int batch_run(tfg_batch* h, int pr, bool fp32, const tfg_options& o, const doubl
   // diagonals, the others), rebuilt from the polled state as systems stop.
   std::vector<int4v> act, act_c;
   std::vector<DiaEntry> act_d;
-  // Rows per thread of the diagonal products (the autotuner's choice, or
-  // TFG_BATCH_ROWS): two takes two consecutive blocks of a system per entry.
+  // Rows per thread of the block kernels (the autotuner's choice, or
+  // TFG_BATCH_ROWS): two takes two blocks per workgroup in the vector kernels
+  // (kManyBlocks) and two consecutive blocks of a system per diagonal entry.
   const char* force_rows = getenv("TFG_BATCH_ROWS");
   const bool two = force_rows && (*force_rows == '1' || *force_rows == '2') ? *force_rows == '2'
                                                                             : cfg.rows == 2;
@@ -1409,15 +1508,20 @@ int batch_run(tfg_batch* h, int pr, bool fp32, const tfg_options& o, const doubl
     else k_bt32_restart<PREC_NONE><<<G, B, 0, S>>>(a);
     k_bt32_rstart<<<a.nsys, B, 0, S>>>(a);
   };
-  // the vector kernels, a block per wavefront
-#define TFG_BT_VEC(KERNEL)                                          \
-  do {                                                              \
-    if (pr == PREC_JACOBI) KERNEL<PREC_JACOBI><<<Gv, B, 0, S>>>(a);  \
-    else KERNEL<PREC_NONE><<<Gv, B, 0, S>>>(a);                      \
+  // the vector kernels, grid Gv: one or two entries per workgroup
+#define TFG_BT_VEC(KERNEL)                                                            \
+  do {                                                                                \
+    if (pairs && pr == PREC_JACOBI) KERNEL<PREC_JACOBI, 2><<<Gv, B, 0, S>>>(a);        \
+    else if (pairs) KERNEL<PREC_NONE, 2><<<Gv, B, 0, S>>>(a);                          \
+    else if (pr == PREC_JACOBI) KERNEL<PREC_JACOBI, 1><<<Gv, B, 0, S>>>(a);            \
+    else KERNEL<PREC_NONE, 1><<<Gv, B, 0, S>>>(a);                                     \
   } while (0)
   auto enqueue_chunk = [&](int count) -> hipError_t {
     const int per = (a.nact + kXcds - 1) / kXcds;
-    const int G = kXcds * per, Gv = kXcds * ((per + kWaves - 1) / kWaves);
+    // the forms for many blocks; chosen again when the lists are compacted
+    const bool many = a.nact >= kManyBlocks, pairs = two && many;
+    const int G = kXcds * per, Gv = kXcds * (pairs ? (per + 1) / 2 : per);
+    const int Gw = kXcds * ((per + kWaves - 1) / kWaves);
     const int Gd = kXcds * ((a.nact_dia + kXcds - 1) / kXcds);
     const int Gc = kXcds * ((a.nact_csr + kXcds - 1) / kXcds);
     if (fp32) {
@@ -1427,7 +1531,10 @@ int batch_run(tfg_batch* h, int pr, bool fp32, const tfg_options& o, const doubl
         else if (Gd) k_bt32_spmv_dia<1><<<Gd, B, 0, S>>>(a);
         if (Gc) TFG_BT32_ENGINE((k_bt32_spmv<E><<<Gc, B, 0, S>>>(a)));
         k_bt32_alpha<<<a.nsys, B, 0, S>>>(a);
-        TFG_BT_VEC(k_bt32_update);
+        if (many && pr == PREC_JACOBI) k_bt32_update_waves<PREC_JACOBI><<<Gw, B, 0, S>>>(a);
+        else if (many) k_bt32_update_waves<PREC_NONE><<<Gw, B, 0, S>>>(a);
+        else if (pr == PREC_JACOBI) k_bt32_update<PREC_JACOBI><<<G, B, 0, S>>>(a);
+        else k_bt32_update<PREC_NONE><<<G, B, 0, S>>>(a);
         k_bt32_check<<<a.nsys, B, 0, S>>>(a);
       }
       k_bt32_fold<<<G, B, 0, S>>>(a);
@@ -1575,7 +1682,7 @@ int batch_tune(tfg_batch* h, int pr, bool fp32, const tfg_options& o, const doub
       if (rc != TFG_OK) return rc;
     }
   }
-  {  // two rows per thread in the diagonal products
+  {  // two rows per thread
     const BatchCfg base = pick;
     const int rc = probe(BatchCfg{base.chunk, base.diag_mask, 2});
     if (rc != TFG_OK) return rc;
