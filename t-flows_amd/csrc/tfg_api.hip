@@ -309,6 +309,22 @@ long long iteration_bytes(const tfg_matrix* h, int kind) {
   return matrix + 40 * n;
 }
 
+// Whether an iteration's data (the FP32 forms: half of them) exceed what stays
+// in the Infinity Cache.  Non-temporal loads of the matrix keep it out of there,
+// which costs when everything would have stayed and gains when the vectors
+// alone do.  Products with plain / non-temporal loads, us: 131x117x97 (107 MB)
+// 14.2 / 18.1, kNN 1M by its windows (215 MB) 35.9 / 51.8, upwind 120^3 (165 MB)
+// 20.1 / 23.9; 160^3 (300 MB) 37.6 / 34.8, upwind 200^3 (766 MB) 112 / 104.
+// Scattered reads of x take lines from the matrix, so a product that makes them
+// crosses over at two thirds: a kNN system in random numbering, ms a solve, FP64
+// 86^3 (157 MB) 17.57 / 17.94, 92^3 (191 MB) 25.4 / 24.5, 100^3 41.8 / 40.3; FP32
+// form 110^3 (163 MB) 25.4 / 25.7, 116^3 (191 MB) 43.3 / 41.4.
+bool beyond_cache(const tfg_matrix* h, int kind, bool fp32) {
+  const long long bytes = iteration_bytes(h, kind) / (fp32 ? 2 : 1);
+  const bool scattered = kind == tfg::K_PIPE2048 && !h->ucol;
+  return bytes > (scattered ? tfg::kInfinityCache / 3 * 2 : tfg::kInfinityCache);
+}
+
 tfg::Launch launch_of(const tfg_matrix* h, const void* val, int kind) {
   tfg::Launch L;
   L.stream = h->stream;
@@ -318,12 +334,13 @@ tfg::Launch launch_of(const tfg_matrix* h, const void* val, int kind) {
   L.vec_val = ((uintptr_t)val % 16) == 0 && h->nnz >= 4;
   L.sym = false;
   L.window = h->ucol != nullptr;
-  // Non-temporal loads of the matrix keep it out of the Infinity Cache, which
-  // costs when everything would have stayed there and gains when the vectors
-  // alone do.  Products with plain / non-temporal loads, us: 131x117x97 (107
-  // MB) 14.2 / 18.1, kNN 1M (215 MB) 35.9 / 51.8, upwind 120^3 (165 MB)
-  // 20.1 / 23.9; 160^3 (300 MB) 37.6 / 34.8, upwind 200^3 (766 MB) 112 / 104.
-  L.nt = iteration_bytes(h, kind) > tfg::kInfinityCache;
+  // GatherEngine or the pipelined StreamEngine for kind 5 without windows; ms a
+  // solve of a kNN system in random numbering, entries dealt out / a row per
+  // thread: FP64 20^3 2.68 / 3.23, 48^3 9.43 / 9.90, 64^3 (262144 rows) 9.44 / 9.64,
+  // 70^3 7.89 / 7.68, 80^3 13.0 / 12.2, 100^3 43.2 / 40.3 (non-temporal); FP32 form
+  // 48^3 6.07 / 6.10, 80^3 11.35 / 11.20, 100^3 29.0 / 27.3.
+  L.gather = h->nt <= (1 << 18);
+  L.nt = beyond_cache(h, kind, false);
   return L;
 }
 
@@ -449,12 +466,11 @@ void free_all(tfg_matrix* h) {
   delete h;
 }
 
-// Engine choice.  By default the pipelined ~2K-nonzero stream engine (the
-// fastest on every T-Flows-like structure measured).  The choice fixes the
-// SpMV launch grid and with it the tree of the fused dot products, so a
-// timed choice could differ between two runs on the same matrix and move
-// the last bits of the result; timing is therefore opt-in: tfg_spmv_tune(),
-// or TFG_SPMV_AUTOTUNE=1 in the environment (times every engine, 2 warm-up +
+// Engine choice.  By default by the formats that the matrix offers
+// (default_kind).  The choice fixes the SpMV launch grid and with it the tree of
+// the fused dot products, so a timed choice could differ between two runs on the
+// same matrix and move the last bits of the result; timing is therefore opt-in:
+// tfg_spmv_tune(), or TFG_SPMV_AUTOTUNE=1 in the environment (times every engine, 2 warm-up +
 // 5 timed launches each, keeps the fastest).  TFG_SPMV_KIND=<0..5> forces one.
 int tune_all(tfg_matrix* h, const double* val);
 
@@ -542,7 +558,7 @@ int tune_all(tfg_matrix* h, const double* val) {
 // The window engine's tables for a handle whose products run kind 5 (made
 // with the handle, so that no product or solve allocates them).  Without the
 // memory for them, or when more than an eighth of the blocks have too many
-// different columns, kind 5 gathers x entry by entry.
+// different columns, kind 5 reads x entry by entry.
 int window_setup(tfg_matrix* h) {
   const int nb = h->nblk[0];
   if (h->nnz < 4) return TFG_OK;
@@ -952,14 +968,14 @@ int solve_ir(tfg_matrix* h, int prec, const double* val, const double* b, int mi
   if (sym) {
     L32.kind = tfg::K_SYM_DIA;
     L32.grid_spmv = h->grid32;
-    L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
+    L32.nt = beyond_cache(h, L32.kind, true);
   } else {
     if (L32.kind != tfg::K_STAGE2048 && L32.kind != tfg::K_PIPE2048_CODED &&
         L32.kind != tfg::K_PIPE_PATTERN)
       L32.kind = tfg::K_PIPE2048;
     L32.grid_spmv = h->grid[L32.kind];
     L32.vec_val = h->nnz >= 4;
-    L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
+    L32.nt = beyond_cache(h, L32.kind, true);
   }
   // one grid for every product-shaped kernel of this solve (their partials
   // are swept with it)
@@ -1156,7 +1172,7 @@ int solve_ir_ns(tfg_matrix* h, int method, int prec, const double* val, const do
     L32.kind = tfg::K_PIPE2048;
   L32.grid_spmv = h->grid[L32.kind];
   L32.vec_val = h->nnz >= 4;
-  L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
+  L32.nt = beyond_cache(h, L32.kind, true);
   tfg::Launch L = launch_of(h, val, h->kind);
   L.grid_spmv = L32.grid_spmv;
   tfg::CgArgs a = args_of(h, h->kind);
@@ -2818,14 +2834,14 @@ int tfg_spmv_fp32(tfg_matrix* h, const double* d_val, double fn, const float* d_
   if (sym) {
     L32.kind = tfg::K_SYM_DIA;
     L32.grid_spmv = h->grid32;
-    L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
+    L32.nt = beyond_cache(h, L32.kind, true);
   } else {
     if (L32.kind != tfg::K_STAGE2048 && L32.kind != tfg::K_PIPE2048_CODED &&
         L32.kind != tfg::K_PIPE_PATTERN)
       L32.kind = tfg::K_PIPE2048;
     L32.grid_spmv = h->grid[L32.kind];
     L32.vec_val = h->nnz >= 4;
-    L32.nt = iteration_bytes(h, L32.kind) / 2 > tfg::kInfinityCache;
+    L32.nt = beyond_cache(h, L32.kind, true);
   }
   tfg::Launch L = launch_of(h, d_val, h->kind);
   tfg::CgArgs a = args_of(h, h->kind);

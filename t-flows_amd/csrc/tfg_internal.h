@@ -339,8 +339,9 @@ struct Launch {
   bool vec_val;    // val is 16-byte aligned (wide nontemporal loads)
   bool sym;        // products by the symmetric engine (val checked symmetric)
   bool nt;         // non-temporal loads of what a product reads once: the data that
-                   // one iteration touches exceed the Infinity Cache (launch_of)
+                   // one iteration touches exceed the Infinity Cache (beyond_cache)
   bool window;     // kind 5 has the columns of its row blocks (WindowEngine)
+  bool gather;     // kind 5 without them deals its entries out (GatherEngine)
 };
 
 // Resident SpMV workgroups per CU for an engine (occupancy query).

@@ -567,7 +567,12 @@ void k_spmv_lap32_sym(SymDiag g, int n, IrArgs f, const float* __restrict__ x,
         } else if ((L).vec_val && (L).window) {                                  \
           using E = WindowEngine<kCap, float, false>; CALL;                      \
         }                                                                        \
-        else if ((L).vec_val) { using E = GatherEngine<kCap, float>; CALL; }     \
+        else if ((L).vec_val && (L).gather) { using E = GatherEngine<kCap, float>; CALL; }\
+        else if ((L).vec_val && (L).nt) {                                        \
+          using E = StreamEngine<kCap, true, float, false, true>; CALL;          \
+        } else if ((L).vec_val) {                                                \
+          using E = StreamEngine<kCap, true, float, false, false>; CALL;         \
+        }                                                                        \
         else { using E = ScalarStage<kCap, float>; CALL; }                       \
         break;                                                                   \
     }                                                                            \

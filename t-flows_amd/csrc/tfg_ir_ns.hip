@@ -469,7 +469,12 @@ __global__ __launch_bounds__(kBlock) void k_ns32_valt(CgArgs a, const int* __res
         } else if ((L).vec_val && (L).window) {                                  \
           using E = WindowEngine<kCap, float, false>; CALL;                      \
         }                                                                        \
-        else if ((L).vec_val) { using E = GatherEngine<kCap, float>; CALL; }     \
+        else if ((L).vec_val && (L).gather) { using E = GatherEngine<kCap, float>; CALL; }\
+        else if ((L).vec_val && (L).nt) {                                        \
+          using E = StreamEngine<kCap, true, float, false, true>; CALL;          \
+        } else if ((L).vec_val) {                                                \
+          using E = StreamEngine<kCap, true, float, false, false>; CALL;         \
+        }                                                                        \
         else { using E = ScalarStage<kCap, float>; CALL; }                       \
         break;                                                                   \
     }                                                                            \

@@ -578,8 +578,8 @@ int spmv_blocks_per_cu(int kind) {
     default: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_spmv_pq<WaveEngine<16, double>>, kBlock, 0); break;
   }
   if (e != hipSuccess || nb < 1) return 1;
-  // kind 5: five, as its row-per-thread form had.  The grid fixes the tree of
-  // the dot products, so a solve keeps its bits.
+  // kind 5: five, as its row-per-thread form has.  The grid fixes the tree of
+  // the dot products, so all its forms give a solve the same bits.
   return kind == 5 ? std::min(nb, 5) : nb;
 }
 

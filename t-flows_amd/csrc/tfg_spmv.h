@@ -85,7 +85,7 @@ struct XcdWalk {
 
 // A load of data that one sweep reads once: non-temporal (NT) when a solve's
 // data exceed the Infinity Cache, so that it does not push out what the next
-// kernel reads again, a plain load when they fit it (launch_of).
+// kernel reads again, a plain load when they fit it (beyond_cache).
 template <bool NT, typename V>
 __device__ __forceinline__ V stream_load(const V* p) {
   if constexpr (NT) return __builtin_nontemporal_load(p);
@@ -317,8 +317,9 @@ struct StreamEngine {
 // row-excess form (LAP) needs the row's own x, so LDS holds a_ij and x_j.
 // While a block is summed the next block's values and columns are in flight
 // into registers.  One line of the L1 per gathered entry is what it takes most
-// time for: 1M rows, 16.8M entries 58 us (63 us with a row per thread); a
-// matrix whose blocks share columns runs WindowEngine instead.
+// time for, so a matrix whose blocks share columns runs WindowEngine instead; and
+// where x is more than half an XCD's L2, many gathers in flight gain nothing over
+// a row per thread (StreamEngine with PIPE): see launch_of.
 template <int CAP, typename T>
 struct GatherEngine {
   static constexpr int NCH = (CAP / 4 + 1 + kBlock - 1) / kBlock;  // 4-entry chunks per thread
@@ -470,7 +471,7 @@ struct GatherEngine {
 // LDS, and each row adds its terms in CSR order.  In flight while a block is
 // summed: the next block's values, places and x entries, and the columns of
 // the one after.  1M rows, 16.8M entries (215 MB, from the Infinity Cache): 36 us,
-// GatherEngine 58 us; 4M rows 181 and 200 us.
+// 58 us entry by entry (GatherEngine); 4M rows 181 and 200 us.
 template <int CAP, typename T, bool NT>
 struct WindowEngine {
   static constexpr int NCH = (CAP / 4 + 1 + kBlock - 1) / kBlock;  // 4-entry chunks per thread
@@ -1195,8 +1196,9 @@ struct WaveEngine {
 };
 
 // kind: 0 stage/kCap, 1 stage/kCap2, 2 wave/4, 3 wave/8, 4 wave/16,
-// 5 entries dealt to the threads (GatherEngine, or WindowEngine where the handle
-// holds the blocks' columns), 6 pipelined stage/kCap with offset-coded columns,
+// 5 entries dealt to the threads (WindowEngine where the handle holds the
+// blocks' columns, else GatherEngine, or the pipelined stage from 262145 rows
+// on), 6 pipelined stage/kCap with offset-coded columns,
 // 7 the same with row patterns (also kind 8: the symmetric engine serves only the CG
 // product and the plain product, when Launch::sym is set; every other
 // kernel uses the row-pattern engine).  The stage engines fall back to scalar staging
@@ -1218,7 +1220,12 @@ struct WaveEngine {
         } else if ((L).vec_val && (L).window) {                                    \
           using E = WindowEngine<kCap, T, false>; CALL;                            \
         }                                                                          \
-        else if ((L).vec_val) { using E = GatherEngine<kCap, T>; CALL; }           \
+        else if ((L).vec_val && (L).gather) { using E = GatherEngine<kCap, T>; CALL; }\
+        else if ((L).vec_val && (L).nt) {                                          \
+          using E = StreamEngine<kCap, true, T, false, true>; CALL;                \
+        } else if ((L).vec_val) {                                                  \
+          using E = StreamEngine<kCap, true, T, false, false>; CALL;               \
+        }                                                                          \
         else { using E = ScalarStage<kCap, T>; CALL; }                             \
         break;                                                                     \
       case 6:                                                                      \
