@@ -20,6 +20,8 @@
 // region loop's order when each region's faces are one range and the ranges
 // ascend with the region number (Faces_In_Region, as T-Flows numbers its
 // boundary faces).  Every value is bit-identical to the serial assembly.
+#include <algorithm>
+
 #include "tflows_gpu.h"
 #include "tfg_spmv.h"
 
@@ -541,8 +543,13 @@ __device__ __forceinline__ RcCell rc_cell(const tfg_rhie_chow& r, int c) {
 // grid's faces swept all cell arrays once each.  Bound by the memory behind
 // the L2: 128x112x96 with Choi's and Gu's corrections 253 us in face order,
 // 196 us now (1.35 GB fetched).  The corrections are template arguments, so
-// that their loads are issued with the others.
-template <bool VOF, bool CHOI, bool GU>
+// that their loads are issued with the others.  On small grids a thread's three
+// faces in turn are all the time there is, so there a cell's faces are dealt to
+// up to six threads (SPLIT: gridDim.y) while the chip has room for them; us a call in
+// face order, with one thread and with this rule: 12^3 15.4, 18.5, 14.7; 26^3 15.6,
+// 18.5, 16.1; 32^3 18.2, 18.5, 16.9; from 64^3 on more threads only cost (48.7, and
+// 56.6 with two).
+template <bool VOF, bool CHOI, bool GU, bool SPLIT>
 __global__ __launch_bounds__(kBlock) void k_rhie_chow(RcArgs a) {
   const CellFaces& t = a.t;
   const int blk = cell_block((t.n + kBlock - 1) / kBlock);
@@ -552,7 +559,8 @@ __global__ __launch_bounds__(kBlock) void k_rhie_chow(RcArgs a) {
   const tfg_rhie_chow& r = a.r;
   const RcCell A = rc_cell<VOF, CHOI, GU>(r, c1);
   const int f1 = t.off[c1 + 1];
-  for (int f = t.off[c1]; f < f1; ++f) {
+  const int first = SPLIT ? (int)blockIdx.y : 0, step = SPLIT ? (int)gridDim.y : 1;
+  for (int f = t.off[c1] + first; f < f1; f += step) {
     const int e = t.face[f], s = e >> 1, c2 = t.nbr[f] - 1;
     if ((e & 1) || c2 < 0) continue;                        // its own domain faces only
     const RcCell B = rc_cell<VOF, CHOI, GU>(r, c2);
@@ -583,18 +591,26 @@ __global__ __launch_bounds__(kBlock) void k_rhie_chow(RcArgs a) {
   }
 }
 
+template <bool VOF, bool CHOI, bool GU>
+void run_rhie_chow(hipStream_t stream, const RcArgs& a) {
+  // two workgroups for each of the 256 CUs, and six faces for a hexahedron
+  const int nblk = std::max(1, (a.t.n + kBlock - 1) / kBlock);
+  const int split = std::min(6, 512 / nblk), grid = cell_grid(a.t.n);
+  if (split > 1) k_rhie_chow<VOF, CHOI, GU, true><<<dim3(grid, split), kBlock, 0, stream>>>(a);
+  else k_rhie_chow<VOF, CHOI, GU, false><<<grid, kBlock, 0, stream>>>(a);
+}
+
 hipError_t launch_rhie_chow(hipStream_t stream, const RcArgs& a) {
-  const int grid = cell_grid(a.t.n);
   const int terms = (a.vof ? 4 : 0) | (a.r.choi ? 2 : 0) | (a.r.gu ? 1 : 0);
   switch (terms) {
-    case 0: k_rhie_chow<false, false, false><<<grid, kBlock, 0, stream>>>(a); break;
-    case 1: k_rhie_chow<false, false, true><<<grid, kBlock, 0, stream>>>(a); break;
-    case 2: k_rhie_chow<false, true, false><<<grid, kBlock, 0, stream>>>(a); break;
-    case 3: k_rhie_chow<false, true, true><<<grid, kBlock, 0, stream>>>(a); break;
-    case 4: k_rhie_chow<true, false, false><<<grid, kBlock, 0, stream>>>(a); break;
-    case 5: k_rhie_chow<true, false, true><<<grid, kBlock, 0, stream>>>(a); break;
-    case 6: k_rhie_chow<true, true, false><<<grid, kBlock, 0, stream>>>(a); break;
-    default: k_rhie_chow<true, true, true><<<grid, kBlock, 0, stream>>>(a); break;
+    case 0: run_rhie_chow<false, false, false>(stream, a); break;
+    case 1: run_rhie_chow<false, false, true>(stream, a); break;
+    case 2: run_rhie_chow<false, true, false>(stream, a); break;
+    case 3: run_rhie_chow<false, true, true>(stream, a); break;
+    case 4: run_rhie_chow<true, false, false>(stream, a); break;
+    case 5: run_rhie_chow<true, false, true>(stream, a); break;
+    case 6: run_rhie_chow<true, true, false>(stream, a); break;
+    default: run_rhie_chow<true, true, true>(stream, a); break;
   }
   return hipGetLastError();
 }
