@@ -216,6 +216,26 @@ int tfg_matrix_info(tfg_matrix* h, int* n, int* nnz, int* spmv_kind,
                     int* spmv_grid, int* stage_blocks, int* offsets, int* patterns,
                     int* sym_diagonals, int* sym_state, int* ordering, int* icc_tiles);
 
+/* The one-launch CG of small systems (TFG_PATH_AUTO) on this handle so far:
+ * its workgroups (-1: no solve has asked yet, or the rows have no patterns, 0:
+ * the system does not fit), its launches, the solves it ran to their end, those that took the other form
+ * because another solve had the device's XCD (busy), and those that could not
+ * hand over between workgroups in time and were solved again in the other form
+ * (given_up).  All forms give the same bits. */
+typedef struct {
+  int workgroups;
+  int launches;
+  int solves;
+  int busy;
+  int given_up;
+} tfg_small_counts;
+int tfg_small_info(tfg_matrix* h, tfg_small_counts* counts);
+/* Its limits: iterations per launch (1 .. 16384, the default), how many more
+ * launches get the time to hand over between their workgroups (negative: all,
+ * the default; a later one gives up at once), and the tag of the next hand-over
+ * (0: unchanged; it can only grow, up to 0xf0000000). */
+int tfg_small_limits(tfg_matrix* h, int iterations, int launches, unsigned next_tag);
+
 /* ---- internal ordering ----------------------------------------------------
  * No counterpart in the reference.  A matrix whose numbering has no locality
  * (randomly numbered cells, as a permuted kNN or a badly ordered unstructured

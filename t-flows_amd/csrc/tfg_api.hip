@@ -194,6 +194,8 @@ struct tfg_matrix {
   unsigned small_tag = 1;
   int small_state = 0;
   tfg::SmallPlan small_plan{};
+  int small_iters = tfg::kSmallLaunch, small_left = -1;  // tfg_small_limits
+  tfg_small_counts small_counts{};
   int pat_len = 0;
   // multi-rank hooks
   tfg_allreduce_fn allreduce = nullptr;
@@ -656,12 +658,12 @@ class XcdLease {
 };
 std::atomic<bool> XcdLease::taken_[XcdLease::kDevices];
 
-// Runs the one-launch CG to its end (some thousand iterations per launch).
+// Runs the one-launch CG to its end, small_iters iterations per launch.
 // *given_up: the kernel could not hand over in time; the solve has to start
 // again with the three-kernel form.
 int small_solve(tfg_matrix* h, const tfg::CgArgs& a, int prec, int mode, int miter,
                 bool* given_up) {
-  constexpr int kLaunch = 1 << 14;
+  const int len = h->small_iters;
   *given_up = false;
   tfg::SmallArgs q{};
   q.n = a.n;
@@ -685,26 +687,31 @@ int small_solve(tfg_matrix* h, const tfg::CgArgs& a, int prec, int mode, int mit
   q.out = q.xcd + 128;
   q.pq = q.out + 16 * tfg::kSmallCopies;
   q.upd = q.pq + 2 * tfg::kBlock;
-  for (int k = 1; k <= miter; k += kLaunch) {
-    if (h->small_tag > 0xf0000000u) {  // the tags start again on cleared slots
+  for (int k = 1; k <= miter; k += len) {
+    if (h->small_tag > tfg::kSmallTags) {  // the tags start again on cleared slots
       HIP_TRY(hipMemsetAsync(h->small, 0, sizeof(unsigned long long) * tfg::kSmallWords, h->stream));
       h->small_tag = 1;
     }
-    q.kend = std::min(miter, k + kLaunch - 1);
+    q.kend = std::min(miter, k + len - 1);
     q.tag = h->small_tag;
+    q.polls = h->small_left != 0 ? tfg::kSmallPolls : 0;
+    if (h->small_left > 0) --h->small_left;
     h->small_tag += (unsigned)(q.kend - k) + 3u;
     HIP_TRY(tfg::launch_small_cg(h->stream, q, h->small_plan, prec, mode));
+    ++h->small_counts.launches;
     State* s = &h->hst[1];
     HIP_TRY(hipMemcpyAsync(s, h->st, sizeof(State), hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
     if (s->refine) {
       h->small_state = -1;
+      ++h->small_counts.given_up;
       *given_up = true;
       return TFG_OK;
     }
     if (s->done) break;
-    if (k > INT_MAX - kLaunch) break;
+    if (k > INT_MAX - len) break;
   }
+  ++h->small_counts.solves;
   return TFG_OK;
 }
 
@@ -2290,6 +2297,28 @@ int tfg_matrix_info(tfg_matrix* h, int* n, int* nnz, int* spmv_kind, int* spmv_g
   return TFG_OK;
 }
 
+int tfg_small_info(tfg_matrix* h, tfg_small_counts* counts) {
+  if (!h || !counts) return fail(TFG_EINVAL, "null argument");
+  if (h->inner) return tfg_small_info(h->inner, counts);
+  *counts = h->small_counts;
+  counts->workgroups = h->small_state == 0 ? -1 : h->small_plan.workgroups;
+  return TFG_OK;
+}
+
+int tfg_small_limits(tfg_matrix* h, int iterations, int launches, unsigned next_tag) {
+  if (!h) return fail(TFG_EINVAL, "null handle");
+  if (h->inner) return tfg_small_limits(h->inner, iterations, launches, next_tag);
+  if (iterations < 1 || iterations > tfg::kSmallLaunch)
+    return fail(TFG_EINVAL, "iterations of a launch: %d", iterations);
+  // the slots may hold any tag below the next one
+  if (next_tag && (next_tag < h->small_tag || next_tag > tfg::kSmallTags))
+    return fail(TFG_EINVAL, "tag %u after %u", next_tag, h->small_tag);
+  h->small_iters = iterations;
+  h->small_left = std::max(launches, -1);
+  if (next_tag) h->small_tag = next_tag;
+  return TFG_OK;
+}
+
 int tfg_spmv_select(tfg_matrix* h, int kind) {
   if (!h) return fail(TFG_EINVAL, "null handle");
   if (h->inner) return tfg_spmv_select(h->inner, kind);
@@ -2496,8 +2525,12 @@ int tfg_solve_native_ex(tfg_matrix* h, const char* solver, int solver_len, const
     // SpMV advances: three launches per iteration.  The executable graph is
     // kept per handle for the same operands.
     XcdLease lease;
-    const bool small = method == tfg::NS_NONE && !icc && !timing && o.path == TFG_PATH_AUTO &&
-                       small_fits(h, L) && lease.take(h->device, h->small_plan);
+    bool small = method == tfg::NS_NONE && !icc && !timing && o.path == TFG_PATH_AUTO &&
+                 small_fits(h, L);
+    if (small && !lease.take(h->device, h->small_plan)) {
+      ++h->small_counts.busy;
+      small = false;
+    }
     bool solved = false;
     if (small) {
       bool given_up = false;

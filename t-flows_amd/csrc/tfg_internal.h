@@ -353,6 +353,9 @@ hipError_t launch_start(const Launch& L, const CgArgs& a, int rho_slot = 6);
 hipError_t launch_pupdate(const Launch& L, const CgArgs& a, int prec, int k, bool dx = false);
 // One-launch CG of a small system (tfg_small.hip).
 constexpr int kSmallCopies = 8;           // of the totals, each on a line of its own
+constexpr int kSmallPolls = 1 << 17;      // reads of one wait, some 50 ms
+constexpr int kSmallLaunch = 1 << 14;     // iterations of one launch
+constexpr unsigned kSmallTags = 0xf0000000u;  // above it the tags start again
 constexpr int kSmallWords = 16 * 64 + 128 + 16 * kSmallCopies + 10 * kBlock;  // slots in all
 struct SmallArgs {
   int n, nblk;
@@ -371,6 +374,7 @@ struct SmallArgs {
   unsigned tag;              // the launch's first tag
   unsigned twice;            // product workgroups (of the first 8) with two blocks
   int kend;                  // last iteration of the launch
+  int polls;                 // of the launch's first wait: kSmallPolls, or 0 (gives up)
 };
 struct SmallPlan {
   int workgroups;            // 0: the system does not fit; 1: k_tiny_cg

@@ -308,7 +308,7 @@ __global__ __launch_bounds__(kTinyGroups* kBlock) void k_tiny_cg(SmallArgs a) {
 // The workgroups have to be resident together.  They fit on the idle XCD
 // (small_plan), one process runs one such launch per device at a time
 // (XcdLease), and other kernels end.  Where another process's launch is in the
-// way all the same, every wait is bounded (kMaxPolls): a workgroup whose wait
+// way all the same, every wait is bounded (kSmallPolls): a workgroup whose wait
 // ends without the tag, or that finds itself on another XCD than the others,
 // raises State::refine and leaves, the others follow by their own bounds, and
 // the host runs the solve again with the three-kernel form.  A cooperative
@@ -316,7 +316,6 @@ __global__ __launch_bounds__(kTinyGroups* kBlock) void k_tiny_cg(SmallArgs a) {
 // process's launch fails.
 namespace {
 
-constexpr int kMaxPolls = 1 << 17;  // some 50 ms
 constexpr int kGroups = 2;          // thread groups of a workgroup
 constexpr int kLine = 16;           // words of a 128-byte line
 
@@ -346,7 +345,7 @@ template <int NV>
 __device__ __forceinline__ bool poll_slots(const u64* slot, int apart, unsigned tag,
                                            double (&v)[NV]) {
 #pragma unroll 1
-  for (int n = 0; n < kMaxPolls; ++n) {
+  for (int n = 0; n < kSmallPolls; ++n) {
     bool all = true;
     u64 hi[NV], lo[NV];
 #pragma unroll
@@ -422,7 +421,7 @@ __global__ __launch_bounds__(kGroups* kBlock, 4) void k_small_cg(SmallArgs a) {
   if (tid < NW) {
     u64 f = 0;
 #pragma unroll 1
-    for (int n = 0; n < kMaxPolls && (unsigned)f != a.tag; ++n) f = load_shared(a.xcd + tid);
+    for (int n = 0; n < a.polls && (unsigned)f != a.tag; ++n) f = load_shared(a.xcd + tid);
     if (f != here) s_bad = 1;
   }
   __syncthreads();
@@ -487,7 +486,7 @@ __global__ __launch_bounds__(kGroups* kBlock, 4) void k_small_cg(SmallArgs a) {
     if (tid < NWV) {
       bool ok = false;
 #pragma unroll 1
-      for (int n = 0; n < kMaxPolls && !ok; ++n)
+      for (int n = 0; n < kSmallPolls && !ok; ++n)
         ok = (unsigned)load_shared(a.flag + tid * kLine) == tag;
       if (!ok) s_bad = 1;
     }

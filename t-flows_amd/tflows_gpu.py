@@ -53,6 +53,10 @@ class Report(ctypes.Structure):
         return {k: getattr(self, k) for k, _ in self._fields_}
 
 
+class SmallCounts(ctypes.Structure):
+    _fields_ = [(k, ctypes.c_int) for k in ("workgroups", "launches", "solves", "busy", "given_up")]
+
+
 _lib = None
 
 
@@ -74,6 +78,8 @@ def lib():
         P, I, D, LL = ctypes.c_void_p, ctypes.c_int, ctypes.c_double, ctypes.c_longlong
         L.tfg_matrix_create.argtypes = [I, I, I, P, P, P, ctypes.POINTER(P)]
         L.tfg_matrix_destroy.argtypes = [P]
+        L.tfg_small_info.argtypes = [P, P]
+        L.tfg_small_limits.argtypes = [P, I, I, ctypes.c_uint]
         L.tfg_matrix_info.argtypes = [P, P, P, P, P, P, P, P, P, P, P, P]
         L.tfg_solve_native.argtypes = [P, ctypes.c_char_p, I, ctypes.c_char_p, I, P, P, P, I,
                                        P, D, P, P]
@@ -225,6 +231,16 @@ class Native:
         return dict(zip(["n", "nnz", "spmv_kind", "spmv_grid", "stage_blocks", "offsets",
                          "patterns", "sym_diagonals", "sym_state", "ordering", "icc_tiles"],
                         [v.value for v in vals]))
+
+    def small_info(self):
+        """How often the one-launch CG of small systems ran on this handle."""
+        c = SmallCounts()
+        _check(lib().tfg_small_info(self.h, ctypes.byref(c)))
+        return {k: getattr(c, k) for k, _ in SmallCounts._fields_}
+
+    def small_limits(self, iterations=1 << 14, launches=-1, next_tag=0):
+        """Its iterations per launch, launches before one gives up, and next tag."""
+        _check(lib().tfg_small_limits(self.h, int(iterations), int(launches), int(next_tag)))
 
     def reorder(self, order):
         """Internal ordering: ORDER_NATURAL or ORDER_RCM (tfg_matrix_reorder)."""
