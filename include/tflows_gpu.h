@@ -221,7 +221,8 @@ int tfg_matrix_info(tfg_matrix* h, int* n, int* nnz, int* spmv_kind,
  * the system does not fit), its launches, the solves it ran to their end, those that took the other form
  * because another solve had the device's XCD (busy), and those that could not
  * hand over between workgroups in time and were solved again in the other form
- * (given_up).  All forms give the same bits. */
+ * (given_up; the next 16 solves, or 32 and so on to 1024 when it happens again,
+ * then do not try).  All forms give the same bits. */
 typedef struct {
   int workgroups;
   int launches;

@@ -188,14 +188,15 @@ struct tfg_matrix {
   hipGraphExec_t cg_graph = nullptr;
   GraphKey cg_key{};
   // one-launch CG of a small system: slots, the next tag, the plan (state 0 not
-  // asked yet, 1 made, -1 the system does not fit, or a launch gave up), longest
-  // row
+  // asked yet, 1 made, -1 the system does not fit), solves to leave out after a
+  // launch gave up, longest row
   unsigned long long* small = nullptr;
   unsigned small_tag = 1;
   int small_state = 0;
   tfg::SmallPlan small_plan{};
   int small_iters = tfg::kSmallLaunch, small_left = -1;  // tfg_small_limits
   tfg_small_counts small_counts{};
+  int small_pause = 0, small_wait = 0;
   int pat_len = 0;
   // multi-rank hooks
   tfg_allreduce_fn allreduce = nullptr;
@@ -631,7 +632,15 @@ bool small_fits(tfg_matrix* h, const tfg::Launch& L) {
     h->small_state = ok ? 1 : -1;
     (void)hipGetLastError();
   }
-  return h->small_state > 0;
+  if (h->small_state < 0) return false;
+  // A launch that gave up cost some 50 ms, and what was in its way (another
+  // process on the card) may stay: the next 16 solves go another way, twice as
+  // many after each further one in a row, at most 1024.
+  if (h->small_wait > 0) {
+    --h->small_wait;
+    return false;
+  }
+  return true;
 }
 
 // One launch at a time of several workgroups that wait for each other, per
@@ -703,7 +712,8 @@ int small_solve(tfg_matrix* h, const tfg::CgArgs& a, int prec, int mode, int mit
     HIP_TRY(hipMemcpyAsync(s, h->st, sizeof(State), hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
     if (s->refine) {
-      h->small_state = -1;
+      h->small_pause = std::min(1024, std::max(16, 2 * h->small_pause));
+      h->small_wait = h->small_pause;
       ++h->small_counts.given_up;
       *given_up = true;
       return TFG_OK;
@@ -711,6 +721,7 @@ int small_solve(tfg_matrix* h, const tfg::CgArgs& a, int prec, int mode, int mit
     if (s->done) break;
     if (k > INT_MAX - len) break;
   }
+  h->small_pause = 0;
   ++h->small_counts.solves;
   return TFG_OK;
 }

@@ -101,6 +101,29 @@ def test_given_up(cases, gpu, dims, mode, device, good):
     assert (i["launches"], i["solves"], i["given_up"]) == (good + 1, 0, 1)
 
 
+def test_tried_again(cases, gpu):
+    """After a launch gave up, 16 solves go another way, 32 when the next one
+    gives up too, then the one launch is back, and a later pause starts at 16."""
+    nat, solve = _solver(cases, gpu, SMALL[0], *MODES[0])
+    want = solve(gpu.PATH_KERNELS)
+
+    def run(n):
+        for _ in range(n):
+            assert solve(gpu.PATH_AUTO) == want
+        i = nat.small_info()
+        return i["solves"], i["given_up"]
+
+    nat.small_limits(launches=0)
+    assert run(1) == (0, 1)
+    assert run(16) == (0, 1) and run(1) == (0, 2)
+    nat.small_limits()
+    assert run(32) == (0, 2) and run(1) == (1, 2) and run(3) == (4, 2)
+    nat.small_limits(launches=0)
+    assert run(1) == (4, 3)
+    nat.small_limits()
+    assert run(16) == (4, 3) and run(1) == (5, 3)
+
+
 def test_two_at_once(cases, gpu):
     """Each solve runs in the one launch or finds the device's XCD taken; none
     gives up, and the bits are the same."""
