@@ -269,10 +269,13 @@ __global__ __launch_bounds__(kBlock) void k_spmv_pq(CgArgs a, int k) {
 // and ||r||^2 on the new r and x.  REL (as in k_pupdate): of these only (z, r)
 // and ||r||^2, and no division; the others are what NRMS measures.  Loads
 // ordered as in k_pupdate: 131x117x97 12.5 us before, 10.2 us now (100^3 10.7 and
-// 8.5, 160^3 23.6 and 20.9).
-template <int PREC, bool DX, bool REL>
+// 8.5, 160^3 23.6 and 20.9).  ITEMS pairs per thread and step: two, but one up to
+// a million rows where x is updated here (!DX), since five vectors' loads for a
+// pair that most threads do not have cost more there than they hide; ms a solve
+// with one load order for all, two and one: 42^3 7.12, 7.24, 7.14; 80^3 22.4, 21.2,
+// 20.8; 100^3 42.5, 37.7, 37.8; 131x117x97 58.7, 49.9, 50.7.
+template <int PREC, bool DX, bool REL, int ITEMS>
 __global__ __launch_bounds__(kBlock, 3) void k_update(CgArgs a, int k) {
-  constexpr int kItems = 2;
   __shared__ double s_tmp[5 * 4], s_out[5];
   State* st = a.st;
   const int done = st->done;
@@ -299,8 +302,8 @@ __global__ __launch_bounds__(kBlock, 3) void k_update(CgArgs a, int k) {
       w.p = p2[t];
     }
   };
-  Item first[kItems];
-  if (npair > 0) first_items<kItems>(npair, first, load);
+  Item first[ITEMS];
+  if (npair > 0) first_items<ITEMS>(npair, first, load);
   __builtin_amdgcn_sched_barrier(0);
   {
     const int ops1[1] = {OP_SUM};
@@ -350,7 +353,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_update(CgArgs a, int k) {
       x2[t] = xo;
     }
   };
-  if (npair > 0) stream_items<kItems>(npair, first, load, pair);
+  if (npair > 0) stream_items<ITEMS>(npair, first, load, pair);
   if ((a.n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
     const int i = a.n - 1;
     double xv = DX ? 0.0 : a.x[i], rv = a.r[i];
@@ -653,7 +656,8 @@ hipError_t launch_update(const Launch& L, const CgArgs& a, int prec, int k, bool
   update_dispatch(prec, dx, a.rel, [&](auto pc, auto dc, auto rc) {
     constexpr int P = decltype(pc)::value;
     constexpr bool D = decltype(dc)::value, R = decltype(rc)::value;
-    k_update<P, D, R><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
+    if (!D && a.n <= (1 << 20)) k_update<P, D, R, D ? 2 : 1><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
+    else k_update<P, D, R, 2><<<L.grid_vec, kBlock, 0, L.stream>>>(a, k);
   });
   return hipGetLastError();
 }
