@@ -34,7 +34,7 @@ __device__ __forceinline__ void stop2(State* st, int k, double res, int status, 
 }
 
 // Start of inner iteration k: for k > 1 the relres test of iteration k-1 on
-// the update partials, then rho_k (as tfg_nonsym.hip's Begin).
+// the update partials, then rho_k (as tfg_nonsym.hip's begin_iteration).
 __device__ __forceinline__ bool begin32(const CgArgs& a, State* st, int k, bool check_omega,
                                         double* s_tmp, double* s_out, double& rho,
                                         double& rho_old) {
