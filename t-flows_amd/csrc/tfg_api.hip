@@ -1503,6 +1503,8 @@ struct tfg_faces {
   int n_ambient = 0;         // boundary faces of ambient regions
   // each cell's faces (tfg::CellFaces)
   int *cf_off = nullptr, *cf_face = nullptr, *cf_nbr = nullptr;
+  int* own = nullptr;        // RcArgs: starts (nt + 1), faces, other cells (n_inner each)
+  int n_inner = 0;           // domain faces
   void* cf_slot = nullptr;
   uint8_t* late = nullptr;
   bool wide = false;         // some row is longer than 256 entries
@@ -1534,7 +1536,7 @@ static tfg::CellFaces cell_faces(const tfg_faces* f) {
 static void faces_free(tfg_faces* f) {
   if (!f) return;
   (void)hipSetDevice(f->device);
-  void* dev[] = {f->cf_off, f->cf_face, f->cf_nbr, f->cf_slot, f->late, f->flags, f->mm};
+  void* dev[] = {f->cf_off, f->cf_face, f->cf_nbr, f->cf_slot, f->late, f->flags, f->mm, f->own};
   for (void* d : dev)
     if (d) (void)hipFree(d);
   (void)hipGetLastError();
@@ -1554,9 +1556,11 @@ int tfg_faces_create(tfg_matrix* h, int n_faces, const int* c1, const int* c2, c
   HIP_TRY(hipMemcpy(col.data(), h->col, sizeof(int) * (size_t)h->nnz, hipMemcpyDeviceToHost));
   std::vector<int> cnt(n + 1, 0);
   std::vector<char> set(h->nnz, 0);   // entries some face sets
+  // the domain faces each cell is c1 of: starts, faces, other cells (RcArgs)
+  std::vector<int> own(n + 1, 0);
   std::vector<uint8_t> fl(n_faces);
   bool shared_entry = false;
-  int max_bnd = 0;
+  int max_bnd = 0, n_set = 0, n_inner = 0;
   for (int s = 0; s < n_faces; ++s)
     if (c2[s] < 0) max_bnd = std::max(max_bnd, -c2[s]);
   std::vector<char> bnd_seen((size_t)max_bnd + 1, 0);
@@ -1581,19 +1585,27 @@ int tfg_faces_create(tfg_matrix* h, int n_faces, const int* c1, const int* c2, c
           col[j2] != p)
         return fail(TFG_EINVAL, "face %d: pos does not point at (c1,c2) / (c2,c1)", s + 1);
       if (set[j1] || set[j2]) shared_entry = true;
+      n_set += !set[j1];
       set[j1] = 1;
+      n_set += !set[j2];
       set[j2] = 1;
+      ++own[p + 1];
+      ++n_inner;
     } else if (c2[s] < 0) {
       if (bnd_seen[-c2[s]]) shared_bnd = true;
       bnd_seen[-c2[s]] = 1;
     }
   }
-  bool wide = false, unset = false;
+  bool wide = false;
+  const bool unset = n_set < h->nnz - n;
   for (int c = 0; c < n; ++c) {
     wide = wide || row[c + 1] - row[c] > 256;
     cnt[c + 1] += cnt[c];
-    for (int j = row[c] + 1; j < row[c + 1]; ++j) unset = unset || !set[j];
+    own[c + 1] += own[c];
   }
+  std::vector<int> own_fill(own.begin(), own.end() - 1);
+  own.resize(n + 1 + 2 * (size_t)n_inner);
+  int *own_face = own.data() + n + 1, *own_nbr = own_face + n_inner;
   // increasing face order within each cell; a face that shares an entry with
   // an earlier one overwrites it, as in the loop
   std::vector<int> cf(cnt[n]), nbr(cnt[n]), fill(cnt.begin(), cnt.end() - 1);
@@ -1611,7 +1623,12 @@ int tfg_faces_create(tfg_matrix* h, int n_faces, const int* c1, const int* c2, c
     const int p = c1[s] - 1, q = c2[s] - 1;
     const bool inner = c2[s] > 0;
     list(p, s << 1, c2[s], inner ? pos[2 * s] - 1 - row[p] : 0);
-    if (inner) list(q, (s << 1) | 1, c1[s], pos[2 * s + 1] - 1 - row[q]);
+    if (inner) {
+      list(q, (s << 1) | 1, c1[s], pos[2 * s + 1] - 1 - row[q]);
+      const int t = own_fill[p]++;
+      own_face[t] = s;
+      own_nbr[t] = q;
+    }
   }
   tfg_faces* f = new tfg_faces();
   f->h = h;
@@ -1627,6 +1644,8 @@ int tfg_faces_create(tfg_matrix* h, int n_faces, const int* c1, const int* c2, c
   up((void**)&f->cf_nbr, nbr.data(), sizeof(int) * nbr.size());
   if (wide) up(&f->cf_slot, slot32.data(), sizeof(int) * slot32.size());
   else up(&f->cf_slot, slot8.data(), slot8.size());
+  up((void**)&f->own, own.data(), sizeof(int) * own.size());
+  f->n_inner = n_inner;
   up((void**)&f->late, late.data(), late.size());
   up((void**)&f->flags, fl.data(), fl.size());
   f->wide = wide;
@@ -1734,7 +1753,10 @@ int tfg_rhie_chow_fluxes(tfg_faces* f, const tfg_rhie_chow* r, double* v_flux) {
   }
   HIP_TRY(hipSetDevice(f->device));
   tfg::RcArgs a{};
-  a.t = cell_faces(f);
+  a.n = f->h->nt;
+  a.off = f->own;
+  a.face = a.off + f->h->nt + 1;
+  a.nbr = a.face + f->n_inner;
   a.r = *r;
   a.vof = vof ? 1 : 0;
   a.v_flux = v_flux;

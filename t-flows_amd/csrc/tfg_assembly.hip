@@ -537,65 +537,76 @@ __device__ __forceinline__ RcCell rc_cell(const tfg_rhie_chow& r, int c) {
 
 }  // namespace
 
-// One thread per cell takes the faces it is c1 of, so a cell's 8 to 18
-// values are read once for its faces, and its neighbours' from the lines that
-// nearby threads read as their own; in face order the three directions of a
-// grid's faces swept all cell arrays once each.  Bound by the memory behind
-// the L2: 128x112x96 with Choi's and Gu's corrections 253 us in face order,
-// 196 us now (1.35 GB fetched).  The corrections are template arguments, so
-// that their loads are issued with the others.  On small grids a thread's three
-// faces in turn are all the time there is, so there a cell's faces are dealt to
-// up to six threads (SPLIT: gridDim.y) while the chip has room for them; us a call in
-// face order, with one thread and with this rule: 12^3 15.4, 18.5, 14.7; 26^3 15.6,
-// 18.5, 16.1; 32^3 18.2, 18.5, 16.9; from 64^3 on more threads only cost (48.7, and
-// 56.6 with two).
+// One thread per cell takes the domain faces it is c1 of (a list of their own:
+// with a cell's whole list walked for them, half the indices were read for
+// nothing and each face waited for its own), so a cell's 8 to 18 values are read
+// once for its faces, and its neighbours' from the lines that nearby threads read
+// as their own; in face order the three directions of a grid's faces swept all
+// cell arrays once each.  Bound by the memory behind the L2.  The corrections are
+// template arguments, so that their loads are issued with the others.  us a call
+// in face order, by the cells' whole lists, by this list: 120^3 with Choi's and
+// Gu's corrections 312, 262, 221; without 134, 155, 131; 80^3 without 53, 52, 40.
+// On small grids a thread's three faces in turn are all the time there is, so
+// there they are dealt to up to three threads (SPLIT: gridDim.y) while the chip
+// has room for them: 12^3 15.5, 18.5, 15.3; from 64^3 on that only costs.
 template <bool VOF, bool CHOI, bool GU, bool SPLIT>
 __global__ __launch_bounds__(kBlock) void k_rhie_chow(RcArgs a) {
-  const CellFaces& t = a.t;
-  const int blk = cell_block((t.n + kBlock - 1) / kBlock);
+  const int blk = cell_block((a.n + kBlock - 1) / kBlock);
   if (blk < 0) return;
   const int c1 = blk * kBlock + (int)threadIdx.x;
-  if (c1 >= t.n) return;
+  if (c1 >= a.n) return;
   const tfg_rhie_chow& r = a.r;
   const RcCell A = rc_cell<VOF, CHOI, GU>(r, c1);
-  const int f1 = t.off[c1 + 1];
-  const int first = SPLIT ? (int)blockIdx.y : 0, step = SPLIT ? (int)gridDim.y : 1;
-  for (int f = t.off[c1] + first; f < f1; f += step) {
-    const int e = t.face[f], s = e >> 1, c2 = t.nbr[f] - 1;
-    if ((e & 1) || c2 < 0) continue;                        // its own domain faces only
-    const RcCell B = rc_cell<VOF, CHOI, GU>(r, c2);
-    const double fs = r.f[s], fc = r.fc[s], sx = r.sx[s], sy = r.sy[s], sz = r.sz[s];
-    const double dx = r.dx[s], dy = r.dy[s], dz = r.dz[s];
-    const double fo = CHOI ? r.flux_o[s] : 0.0, foo = CHOI ? r.flux_oo[s] : 0.0;
-    const double fx = GU ? r.face_fx[s] : 0.0, fy = GU ? r.face_fy[s] : 0.0;
-    const double fz = GU ? r.face_fz[s] : 0.0;
-    double pst_d = A.p - B.p;                               // :94-98
-    if (VOF) {                                              // :115-123
-      const double curv_f = fs * A.curv + (1.0 - fs) * B.curv;
-      pst_d = pst_d - r.sigma * curv_f * (A.col - B.col);
+  // kIndex faces' indices together, then each face
+  constexpr int kIndex = SPLIT ? 1 : 3;
+  const int f1 = a.off[c1 + 1];
+  const int first = SPLIT ? (int)blockIdx.y : 0, step = SPLIT ? (int)gridDim.y : kIndex;
+  for (int f0 = a.off[c1] + first; f0 < f1; f0 += step) {
+    int face[kIndex], nbr[kIndex];
+#pragma unroll
+    for (int k = 0; k < kIndex; ++k) {
+      const int f = min(f0 + k, f1 - 1);
+      face[k] = a.face[f];
+      nbr[k] = a.nbr[f];
     }
-    const double u_f = fs * A.u + (1.0 - fs) * B.u;
-    const double v_f = fs * A.v + (1.0 - fs) * B.v;
-    const double w_f = fs * A.w + (1.0 - fs) * B.w;
-    const double a12 = fc * (fs * A.vm + (1.0 - fs) * B.vm);
-    const double px_f = (fs * (A.px * A.vm) + (1.0 - fs) * (B.px * B.vm)) * dx;
-    const double py_f = (fs * (A.py * A.vm) + (1.0 - fs) * (B.py * B.vm)) * dy;
-    const double pz_f = (fs * (A.pz * A.vm) + (1.0 - fs) * (B.pz * B.vm)) * dz;
-    double fl = (u_f * sx + v_f * sy + w_f * sz) + a12 * pst_d +
-                fc * (px_f + py_f + pz_f);                  // :226-230
-    if (CHOI)                                               // :235-246
-      fl = fl + (fs * A.tm + (1.0 - fs) * B.tm) * (r.w_o * fo + r.w_oo * foo);
-    if (GU)                                                 // :250-256
-      fl = fl + (fs * A.vm + (1.0 - fs) * B.vm) * (fx * sx + fy * sy + fz * sz);
-    a.v_flux[s] = fl;
+#pragma unroll
+    for (int k = 0; k < kIndex; ++k) {
+      if (f0 + k >= f1) continue;
+      const int s = face[k], c2 = nbr[k];
+      const RcCell B = rc_cell<VOF, CHOI, GU>(r, c2);
+      const double fs = r.f[s], fc = r.fc[s], sx = r.sx[s], sy = r.sy[s], sz = r.sz[s];
+      const double dx = r.dx[s], dy = r.dy[s], dz = r.dz[s];
+      const double fo = CHOI ? r.flux_o[s] : 0.0, foo = CHOI ? r.flux_oo[s] : 0.0;
+      const double fx = GU ? r.face_fx[s] : 0.0, fy = GU ? r.face_fy[s] : 0.0;
+      const double fz = GU ? r.face_fz[s] : 0.0;
+      double pst_d = A.p - B.p;                               // :94-98
+      if (VOF) {                                              // :115-123
+        const double curv_f = fs * A.curv + (1.0 - fs) * B.curv;
+        pst_d = pst_d - r.sigma * curv_f * (A.col - B.col);
+      }
+      const double u_f = fs * A.u + (1.0 - fs) * B.u;
+      const double v_f = fs * A.v + (1.0 - fs) * B.v;
+      const double w_f = fs * A.w + (1.0 - fs) * B.w;
+      const double a12 = fc * (fs * A.vm + (1.0 - fs) * B.vm);
+      const double px_f = (fs * (A.px * A.vm) + (1.0 - fs) * (B.px * B.vm)) * dx;
+      const double py_f = (fs * (A.py * A.vm) + (1.0 - fs) * (B.py * B.vm)) * dy;
+      const double pz_f = (fs * (A.pz * A.vm) + (1.0 - fs) * (B.pz * B.vm)) * dz;
+      double fl = (u_f * sx + v_f * sy + w_f * sz) + a12 * pst_d +
+                  fc * (px_f + py_f + pz_f);                  // :226-230
+      if (CHOI)                                               // :235-246
+        fl = fl + (fs * A.tm + (1.0 - fs) * B.tm) * (r.w_o * fo + r.w_oo * foo);
+      if (GU)                                                 // :250-256
+        fl = fl + (fs * A.vm + (1.0 - fs) * B.vm) * (fx * sx + fy * sy + fz * sz);
+      a.v_flux[s] = fl;
+    }
   }
 }
 
 template <bool VOF, bool CHOI, bool GU>
 void run_rhie_chow(hipStream_t stream, const RcArgs& a) {
-  // two workgroups for each of the 256 CUs, and six faces for a hexahedron
-  const int nblk = std::max(1, (a.t.n + kBlock - 1) / kBlock);
-  const int split = std::min(6, 512 / nblk), grid = cell_grid(a.t.n);
+  // two workgroups for each of the 256 CUs, and three faces for a hexahedron
+  const int nblk = std::max(1, (a.n + kBlock - 1) / kBlock);
+  const int split = std::min(3, 512 / nblk), grid = cell_grid(a.n);
   if (split > 1) k_rhie_chow<VOF, CHOI, GU, true><<<dim3(grid, split), kBlock, 0, stream>>>(a);
   else k_rhie_chow<VOF, CHOI, GU, false><<<grid, kBlock, 0, stream>>>(a);
 }

@@ -313,7 +313,10 @@ hipError_t launch_momentum(hipStream_t stream, const MomArgs& m);
 
 // Rhie-Chow face fluxes (tfg_assembly.hip).
 struct RcArgs {
-  CellFaces t;
+  int n;                 // cells
+  const int* off;        // n+1: the domain faces each cell is c1 of, in the lists below
+  const int* face;       // face index
+  const int* nbr;        // the other cell, 0-based
   tfg_rhie_chow r;
   int vof;               // surface tension term active
   double* v_flux;

@@ -1,8 +1,7 @@
 """The per-cell walk of the Rhie-Chow fluxes where it can go wrong: block
 remainders, boundary faces before, between and after the domain faces, faces
 whose c1 is the larger cell, cells of many faces and of none, and a cell's
-faces dealt to six threads, to five, three, two and one (by the number of
-cells).  Bit for bit against the oracle's serial loop; every domain face is
+faces dealt to three threads, to two and to one (by the number of cells).  Bit for bit against the oracle's serial loop; every domain face is
 written (NaN before), no boundary face is."""
 import numpy as np
 import pytest
