@@ -300,32 +300,46 @@ int grid_vec_of(const tfg_matrix* h) {
   return std::max(1, std::min(gv, std::max(1, h->cu_count) * 3));
 }
 
-// Bytes that one FP64 iteration touches: the matrix as the engine reads it
-// and five vectors (x, r, p, q, the diagonal).  The FP32 forms touch half.
-long long iteration_bytes(const tfg_matrix* h, int kind) {
-  const long long n = h->nt, nnz = h->nnz;
-  const long long matrix = kind == tfg::K_SYM_DIA          ? 8 * (h->nsym + 1) * n
-                           : kind == tfg::K_PIPE_PATTERN   ? 8 * nnz + n
-                           : kind == tfg::K_PIPE2048_CODED ? 9 * nnz + 4 * n
-                           : kind == tfg::K_PIPE2048 && h->ucol ? 10 * nnz + 4 * n
-                                                                : 12 * nnz + 4 * n;
-  return matrix + 40 * n;
+int default_kind(const tfg_matrix* h);
+
+// Vectors that an iteration touches: CG x, r, p, q and the diagonal; its FP32
+// form e, r, p, q, the diagonal and the row sums; CGS and BiCGSTAB twice CG's.
+// BiCG (with the transposed values) and the textbook methods' FP32 forms count
+// for twelve, by where their solves cross over: BiCG 120^3 4.07 / 4.13 ms with
+// plain and non-temporal loads, 125^3 4.26 / 4.14; CGS in FP32 132^3 2.15 / 2.31,
+// 137^3 2.57 / 2.45.
+constexpr int kCgVectors = 5, kCg32Vectors = 6, kNsVectors = 10, kNsMoreVectors = 12;
+
+// Whether an iteration's data, the matrix as the engine reads it and the
+// vectors, exceed the Infinity Cache.  Non-temporal loads of the matrix keep it
+// out of there, which costs when everything would have stayed and gains when the
+// vectors alone do.  Products with plain / non-temporal loads, us: 131x117x97
+// (107 MB) 14.2 / 18.1, kNN 1M by its windows (215 MB) 35.9 / 51.8, 160^3 (295 MB)
+// 37.6 / 34.8, upwind 200^3 112 / 104.  ms a solve: FP32 form 182^3 (241 MB) 7.49 /
+// 8.22, 190^3 (274 MB) 16.3 / 16.0; CGS 124^3 (261 MB) 2.19 / 2.30, 132^3 (315 MB)
+// 2.70 / 2.65, 142^3 3.60 / 3.31.
+// Reads of x scattered by a random numbering find it in the L2s up to some 5 MB;
+// beyond, they take the cache, and the matrix is better left out of it: kNN
+// systems in random numbering, ms a solve, FP64 86^3 (x of 5.1 MB) 17.57 / 17.94,
+// 92^3 (6.2 MB) 25.4 / 24.5, 100^3 41.8 / 40.3; FP32 form 110^3 (5.3 MB) 25.4 /
+// 25.7, 116^3 (6.2 MB) 43.3 / 41.4.
+bool beyond_cache(const tfg_matrix* h, int kind, int vectors, bool fp32) {
+  const long long n = h->nt, nnz = h->nnz, v = fp32 ? 4 : 8;
+  if (kind == tfg::K_PIPE2048 && !h->ucol && default_kind(h) == tfg::K_PIPE2048)
+    return v * n > 11LL << 19;
+  const long long matrix = kind == tfg::K_SYM_DIA          ? v * (h->nsym + 1) * n
+                           : kind == tfg::K_PIPE_PATTERN   ? v * nnz + n
+                           : kind == tfg::K_PIPE2048_CODED ? (v + 1) * nnz + 4 * n
+                           : kind == tfg::K_PIPE2048 && h->ucol ? (v + 2) * nnz + 4 * n
+                                                                : (v + 4) * nnz + 4 * n;
+  return matrix + v * vectors * n > tfg::kInfinityCache;
 }
 
-// Whether an iteration's data (the FP32 forms: half of them) exceed what stays
-// in the Infinity Cache.  Non-temporal loads of the matrix keep it out of there,
-// which costs when everything would have stayed and gains when the vectors
-// alone do.  Products with plain / non-temporal loads, us: 131x117x97 (107 MB)
-// 14.2 / 18.1, kNN 1M by its windows (215 MB) 35.9 / 51.8, upwind 120^3 (165 MB)
-// 20.1 / 23.9; 160^3 (300 MB) 37.6 / 34.8, upwind 200^3 (766 MB) 112 / 104.
-// Scattered reads of x take lines from the matrix, so a product that makes them
-// crosses over at two thirds: a kNN system in random numbering, ms a solve, FP64
-// 86^3 (157 MB) 17.57 / 17.94, 92^3 (191 MB) 25.4 / 24.5, 100^3 41.8 / 40.3; FP32
-// form 110^3 (163 MB) 25.4 / 25.7, 116^3 (191 MB) 43.3 / 41.4.
-bool beyond_cache(const tfg_matrix* h, int kind, bool fp32) {
-  const long long bytes = iteration_bytes(h, kind) / (fp32 ? 2 : 1);
-  const bool scattered = kind == tfg::K_PIPE2048 && !h->ucol;
-  return bytes > (scattered ? tfg::kInfinityCache / 3 * 2 : tfg::kInfinityCache);
+// The matrix loads of a launch whose engine is settled: kind 8 runs the row
+// patterns where val is not symmetric.
+void set_loads(const tfg_matrix* h, tfg::Launch* L, int vectors) {
+  const int kind = L->kind == tfg::K_SYM_DIA && !L->sym ? (int)tfg::K_PIPE_PATTERN : L->kind;
+  L->nt = beyond_cache(h, kind, vectors, false);
 }
 
 tfg::Launch launch_of(const tfg_matrix* h, const void* val, int kind) {
@@ -343,7 +357,7 @@ tfg::Launch launch_of(const tfg_matrix* h, const void* val, int kind) {
   // 70^3 7.89 / 7.68, 80^3 13.0 / 12.2, 100^3 43.2 / 40.3 (non-temporal); FP32 form
   // 48^3 6.07 / 6.10, 80^3 11.35 / 11.20, 100^3 29.0 / 27.3.
   L.gather = h->nt <= (1 << 18);
-  L.nt = beyond_cache(h, kind, false);
+  set_loads(h, &L, kCgVectors);
   return L;
 }
 
@@ -539,6 +553,7 @@ int tune_all(tfg_matrix* h, const double* val) {
         continue;
       }
       L.sym = true;
+      set_loads(h, &L, kCgVectors);
     }
     const tfg::SpmvShape m = shape_of(h, k);
     for (int w = 0; w < 2; ++w) HIP_TRY(tfg::launch_spmv_plain(L, m, val, h->p, h->q));
@@ -1003,14 +1018,14 @@ int solve_ir(tfg_matrix* h, int prec, const double* val, const double* b, int mi
   if (sym) {
     L32.kind = tfg::K_SYM_DIA;
     L32.grid_spmv = h->grid32;
-    L32.nt = beyond_cache(h, L32.kind, true);
+    L32.nt = beyond_cache(h, L32.kind, kCg32Vectors, true);
   } else {
     if (L32.kind != tfg::K_STAGE2048 && L32.kind != tfg::K_PIPE2048_CODED &&
         L32.kind != tfg::K_PIPE_PATTERN)
       L32.kind = tfg::K_PIPE2048;
     L32.grid_spmv = h->grid[L32.kind];
     L32.vec_val = h->nnz >= 4;
-    L32.nt = beyond_cache(h, L32.kind, true);
+    L32.nt = beyond_cache(h, L32.kind, kCg32Vectors, true);
   }
   // one grid for every product-shaped kernel of this solve (their partials
   // are swept with it)
@@ -1207,7 +1222,7 @@ int solve_ir_ns(tfg_matrix* h, int method, int prec, const double* val, const do
     L32.kind = tfg::K_PIPE2048;
   L32.grid_spmv = h->grid[L32.kind];
   L32.vec_val = h->nnz >= 4;
-  L32.nt = beyond_cache(h, L32.kind, true);
+  L32.nt = beyond_cache(h, L32.kind, kNsMoreVectors, true);
   tfg::Launch L = launch_of(h, val, h->kind);
   L.grid_spmv = L32.grid_spmv;
   tfg::CgArgs a = args_of(h, h->kind);
@@ -2533,6 +2548,9 @@ int tfg_solve_native_ex(tfg_matrix* h, const char* solver, int solver_len, const
       if (rs != TFG_OK) return rs;
       a.sd = h->sym;
     }
+    set_loads(h, &L, method == tfg::NS_NONE   ? kCgVectors
+                     : method == tfg::NS_BICG ? kNsMoreVectors
+                                              : kNsVectors);
     HIP_TRY(tfg::launch_diag_sum(L, a));
     const bool icc = pr == tfg::PREC_ICC;
     tfg::IccArgs ic{};
@@ -2804,6 +2822,7 @@ int tfg_solve_native_noalloc(tfg_matrix* h, const char* solver, int solver_len, 
     HIP_TRY(hipMemcpyAsync(&asym, flag, sizeof(int), hipMemcpyDeviceToHost, S));
     HIP_TRY(hipStreamSynchronize(S));
     L.sym = asym == 0;
+    set_loads(h, &L, kCgVectors);
     h->sym_state = L.sym ? 1 : 0;
     a.sd = sd;
   }
@@ -2919,14 +2938,14 @@ int tfg_spmv_fp32(tfg_matrix* h, const double* d_val, double fn, const float* d_
   if (sym) {
     L32.kind = tfg::K_SYM_DIA;
     L32.grid_spmv = h->grid32;
-    L32.nt = beyond_cache(h, L32.kind, true);
+    L32.nt = beyond_cache(h, L32.kind, kCg32Vectors, true);
   } else {
     if (L32.kind != tfg::K_STAGE2048 && L32.kind != tfg::K_PIPE2048_CODED &&
         L32.kind != tfg::K_PIPE_PATTERN)
       L32.kind = tfg::K_PIPE2048;
     L32.grid_spmv = h->grid[L32.kind];
     L32.vec_val = h->nnz >= 4;
-    L32.nt = beyond_cache(h, L32.kind, true);
+    L32.nt = beyond_cache(h, L32.kind, kCg32Vectors, true);
   }
   tfg::Launch L = launch_of(h, d_val, h->kind);
   tfg::CgArgs a = args_of(h, h->kind);
@@ -2970,6 +2989,7 @@ int tfg_spmv(tfg_matrix* h, const double* d_val, const double* d_p, double* d_q)
   if (h->kind == tfg::K_SYM_DIA) {
     const int rs = sym_prepare(h, d_val, &L.sym);
     if (rs != TFG_OK) return rs;
+    set_loads(h, &L, kCgVectors);
   }
   HIP_TRY(tfg::launch_spmv_plain(L, shape_of(h, h->kind), d_val, d_p, d_q));
   return TFG_OK;
@@ -3008,6 +3028,7 @@ int tfg_spmv_bench(tfg_matrix* h, const double* d_val, const double* d_p, double
   if (h->kind == tfg::K_SYM_DIA) {
     const int rs = sym_prepare(h, d_val, &L.sym);
     if (rs != TFG_OK) return rs;
+    set_loads(h, &L, kCgVectors);
   }
   const tfg::SpmvShape m = shape_of(h, h->kind);
   HIP_TRY(hipEventRecord(h->ev_t0, h->stream));

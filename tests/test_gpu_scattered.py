@@ -1,7 +1,7 @@
 """Products of an unstructured matrix in random numbering (no windows of
 columns): entries dealt to the threads up to 262144 rows, a row per thread
-above, its matrix loads non-temporal beyond two thirds of the Infinity Cache
-(92^3 in FP64, 116^3 in the FP32 form).  Bit for bit against the oracle."""
+above, its matrix loads non-temporal where x passes 5.5 MB (92^3 in FP64, 116^3
+in the FP32 form).  Bit for bit against the oracle."""
 import numpy as np
 import pytest
 
